@@ -114,7 +114,7 @@ typedef struct void_dense_args {
   int32_t b_col_major;    /* 0: (k,n) at b[k*ldb+n]; 1: (k,n) at b[n*ldb+k] */
   int32_t N;
   float b_scale;          /* per-tensor scale of B, used when b_scale_vec is NULL */
-  const float* b_scale_vec; /* [N] per-column scale of B, or NULL */
+  const float* b_scale_vec; /* [N] per-column scale of B, or NULL; see b_scale_one */
   const float* bias;      /* [N] added before the activation, or NULL */
   void* c;                /* M x N row-major output */
   int64_t ldc;
@@ -122,7 +122,8 @@ typedef struct void_dense_args {
   int32_t activation;     /* void_activation */
   int32_t bias_per_row;   /* 0: bias[N] per column; 1: bias[M] per output row (the reference's
                              row-bias kernel, void/fusion.py:202-304; float SpMM only) */
-  int32_t reserved;       /* 0 */
+  int32_t b_scale_one;    /* 1: b_scale_vec holds a single scale for all columns (a per-tensor scale
+                             that stays in device memory); 0: [N] */
 } void_dense_args;
 
 /* ---------------------------------------------------------------------- */
@@ -260,6 +261,21 @@ int void_spmm_f16(const void_bsr_desc* a, const void_dense_args* d, const void_p
  * 16-byte aligned, q 4-byte aligned. */
 int void_quantize_b_i8(const float* b, int64_t n, int8_t* q, float* scale, uint32_t* partials,
                        hipStream_t stream);
+
+/* The same for a K x N matrix (n = K N), the codes of row k at q + k ldq:
+ * ldq >= N, a multiple of 4, with q 4-byte aligned; q[k ldq + N ..] is
+ * written as zero.  A pitch that is a multiple of 16 gives the SpMM the
+ * aligned rows of its LDS-DMA ring for any N.  K ldq / 4 < 2^31. */
+int void_quantize_b_i8_rows(const float* b, int32_t K, int32_t N, int8_t* q, int32_t ldq, float* scale,
+                            uint32_t* partials, hipStream_t stream);
+
+/* Row copy of a rows x cols byte matrix (an 8-bit B whose rows are not
+ * 16-byte aligned) to dst with rows ld_dst apart (a multiple of 16, at least
+ * cols; dst 16-byte aligned), for the SpMM's LDS-DMA ring.  Bytes cols ..
+ * ceil16(cols) - 1 of a row are written as zero, the rest of the pitch is
+ * left alone.  At most 2^31 - 1 chunks.  No counterpart in the reference. */
+int void_copy_rows_b8(const void* src, int64_t ld_src, int32_t rows, int32_t cols, void* dst, int64_t ld_dst,
+                      hipStream_t stream);
 
 /* dst[c * ld_dst + r] = src[r * ld_src + c] for a rows x cols byte matrix:
  * a column-major int8 or E4M3 B (src: its N columns of K bytes, ld_src

@@ -1,0 +1,105 @@
+"""An 8-bit B of any width on the column-group kernels: aligned copies of
+unaligned rows, padded quantisation of a float B, and rows whose last 16-byte
+chunk is cut off by N."""
+
+import numpy as np
+import pytest
+import torch
+
+import cases
+import oracle
+import void_amd
+from void_amd import _runtime, tuning
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [1, 15, 17, 63, 65, 127, 129, 250, 513]
+
+
+@pytest.fixture
+def gpu():
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (3, 16), (70, 17), (33, 65), (129, 250), (64, 513)])
+@pytest.mark.parametrize("shift", [0, 1, 7])
+def test_aligned_copy_bytes(gpu, shape, shift):
+    K, N = shape
+    flat = torch.randint(-128, 128, (K * (N + 3) + shift,), dtype=torch.int8, device=gpu)
+    b = flat[shift:].view(K, N + 3)[:, :N]
+    out = _runtime.aligned_copy_b8(b, b.stride(0))
+    assert out.stride(0) == tuning.aligned_pitch(N) and out.data_ptr() % 16 == 0
+    assert torch.equal(out, b)
+
+
+@pytest.mark.parametrize("N", WIDTHS)
+def test_padded_quantisation_matches_flat(gpu, N):
+    from void_amd.int_quant import IntFormat, IntQuantConfig, ScaleMode, _quantize_b_per_tensor, quantize_tensor
+    b = torch.randn(77, N, generator=torch.Generator().manual_seed(N))
+    cfg = IntQuantConfig(format=IntFormat.INT8, symmetric=True, scale_mode=ScaleMode.PER_TENSOR)
+    ref, params = quantize_tensor(b, cfg)
+    q, scale = _quantize_b_per_tensor(b.to(gpu))
+    assert q.stride(0) % 16 == 0 and torch.equal(q.cpu(), ref)
+    assert torch.equal(scale.cpu(), params.scale.reshape(1))
+
+
+@pytest.mark.parametrize("kernel", ["default", "cg", "cgd", "cgd3", "cgdk", "bsr"])
+@pytest.mark.parametrize("pad", ["0", "1", "pitch", "shift"])
+@pytest.mark.parametrize("N", WIDTHS)
+def test_int8_any_width(gpu, monkeypatch, kernel, pad, N):
+    """Accumulators bit-exact for every kernel; columns past N hold other data."""
+    if kernel != "default":
+        monkeypatch.setenv("VOID_AMD_KERNEL", kernel)
+    monkeypatch.setenv("VOID_AMD_PAD", "0" if pad == "0" else "1")
+    case = cases.uniform_blocks(170, 203, N, 25, seed=N)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu"))
+    rng = np.random.default_rng(N)
+    bq = rng.integers(-128, 128, (203, N), dtype=np.int8)
+    pitch, shift = (N + 31) // 16 * 16 if pad == "pitch" else N, 5 if pad == "shift" else 0
+    flat = torch.full((203 * pitch + shift,), 99, dtype=torch.int8)
+    b = flat[shift:].view(203, pitch)[:, :N]
+    b.copy_(torch.from_numpy(bq))
+    b = flat.to(gpu)[shift:].view(203, pitch)[:, :N]
+    A = oracle.Bsr(q.values.numpy(), q.scales.numpy(), case.block_rows, case.block_cols, (170, 203))
+    qd = q.to(gpu)
+    got = void_amd.void_spmm_int8(qd, b, epilogue="raw_i32").cpu().numpy()
+    assert np.array_equal(got, oracle.i8_acc(A, bq))
+    # A misaligned output view as well.
+    wide = torch.full((170, N + 3), -7, dtype=torch.int32, device=gpu)
+    void_amd.void_spmm_int8(qd, b, epilogue="raw_i32", out=wide[:, 1:N + 1])
+    assert np.array_equal(wide[:, 1:N + 1].cpu().numpy(), got)
+    assert bool((wide[:, 0] == -7).all()) and bool((wide[:, N + 1:] == -7).all())
+
+
+@pytest.mark.parametrize("N", WIDTHS)
+def test_float_b_scale_stays_single(gpu, N):
+    """Row-mean with the device scale of a float B, bit for bit the oracle's."""
+    case = cases.uniform_blocks(170, 203, N, 25, seed=N + 1)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu"))
+    bq, bs = oracle.quantize_i8_tensor(case.b)
+    A = oracle.Bsr(q.values.numpy(), q.scales.numpy(), case.block_rows, case.block_cols, (170, 203))
+    ref = oracle.row_mean(A, oracle.i8_acc(A, bq), bs)
+    got = void_amd.void_spmm_int8(q.to(gpu), torch.from_numpy(case.b).to(gpu)).cpu().numpy()
+    assert np.array_equal(got.view(np.int32), ref.view(np.int32))
+
+
+@pytest.mark.parametrize("N", [17, 250])
+def test_fp8_nan_codes_past_n(gpu, N):
+    """Chunks cut off by N may hold NaN codes in the next columns: never stored, never mixed in."""
+    case = cases.uniform_blocks(96, 200, N, 14, seed=N)
+    f8 = void_amd.void_tensor_to_fp8(cases.make_void_tensor(case, "cpu"))
+    pitch = (N + 31) // 16 * 16
+    raw = torch.full((200, pitch), 0x7f, dtype=torch.uint8)
+    codes = torch.from_numpy(case.b).clamp(-400, 400).to(torch.float8_e4m3fn)
+    raw[:, :N] = codes.view(torch.uint8)
+    b = raw.to(gpu).view(torch.float8_e4m3fn)[:, :N]
+    out = void_amd.void_spmm_fp8(f8.to(gpu), b, output_dtype=torch.float32).double().cpu()
+    dense = torch.zeros(96, 224, dtype=torch.float64)
+    mag = torch.zeros(96, 224, dtype=torch.float64)
+    t = f8.values_fp8.double() * f8.scaling_info.scale.double()[:, None, None]
+    for i, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+        dense[32 * r:32 * r + 32, 32 * c:32 * c + 32] = t[i]
+    mag = dense.abs()
+    bd = codes.double()
+    ref, bound = dense[:, :200] @ bd, mag[:, :200] @ bd.abs()
+    assert bool(((out - ref).abs() <= 2.0 ** -13 * bound + 1e-30).all())

@@ -90,7 +90,7 @@ class DenseArgs(ctypes.Structure):
         ("out_dtype", c_int32),
         ("activation", c_int32),
         ("bias_per_row", c_int32),
-        ("reserved", c_int32),
+        ("b_scale_one", c_int32),
     ]
 
 
@@ -121,6 +121,8 @@ SIGNATURES = {
     "void_spmm_f16": (c_int, [POINTER(BsrDesc), POINTER(DenseArgs), POINTER(Plan),
                               c_void_p, c_size_t, c_void_p]),
     "void_transpose_b8": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64, c_void_p]),
+    "void_quantize_b_i8_rows": (c_int, [c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
+    "void_copy_rows_b8": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64, c_void_p]),
     "void_quantize_b_i8": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "void_quantize_tiles_i8": (c_int, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
     "void_quantize_tiles_fp8": (c_int, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),

@@ -368,11 +368,23 @@ def row_major_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
     return out
 
 
+def aligned_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
+    """Copy of a row-major 8-bit B (rows ld apart) with 16-byte aligned rows."""
+    K, N = b.shape
+    pitch = tuning.aligned_pitch(N)
+    out = torch.empty(K, pitch, dtype=b.dtype, device=b.device)[:, :N]
+    st = _lib.lib().void_copy_rows_b8(b.data_ptr(), ld, K, N, out.data_ptr(), pitch,
+                                      torch.cuda.current_stream(b.device).cuda_stream)
+    _lib.check(st, "void_copy_rows_b8")
+    return out
+
+
 def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
-           b_scale_vec: Optional[torch.Tensor] = None, out: torch.Tensor, epilogue: int,
+           b_scale_vec: Optional[torch.Tensor] = None, b_scale_one: bool = False, out: torch.Tensor, epilogue: int,
            activation: int = _lib.ACT_NONE, bias: Optional[torch.Tensor] = None,
            chunk: int) -> torch.Tensor:
-    """Launch one SpMM on the current stream of out's device; returns out."""
+    """Launch one SpMM on the current stream of out's device; returns out.
+    With b_scale_one, b_scale_vec holds one scale for every column."""
     lib = _lib.lib()
     N = b.shape[1]
     b_t, ldb, col_major = dense_operand(b)
@@ -381,6 +393,12 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
     target = out
     if out.stride(1) != 1 or out.stride(0) < N:
         target = torch.empty(out.shape, dtype=out.dtype, device=out.device)
+    if (kind in ("int8", "fp8") and N and not col_major and (ldb % 16 or b_t.data_ptr() % 16)
+            and chunk <= tuning.FP32_B_MAX_CHUNK):
+        dword = ((N | ldb | b_t.data_ptr() | target.stride(0)) % 4 == 0) and target.data_ptr() % 16 == 0
+        if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword):
+            b_t = aligned_copy_b8(b_t, ldb)
+            ldb = b_t.stride(0)
     plan = dbsr.plan(chunk)
     stream = torch.cuda.current_stream(out.device).cuda_stream
     ws, ws_bytes = plan.workspace(N, out.device, stream)
@@ -391,6 +409,8 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
         bias=bias.data_ptr() if bias is not None else None,
         c=target.data_ptr(), ldc=target.stride(0), out_dtype=_OUT_CODES[target.dtype],
         activation=activation)
+    if b_scale_one:
+        dense.b_scale_one = 1
     desc = dbsr.desc()
     ws_ptr = ws.data_ptr() if ws is not None else None
     if kind == "int8":

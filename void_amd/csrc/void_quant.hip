@@ -14,6 +14,7 @@
 
 #include <algorithm>
 
+#include <climits>
 #include <cstdint>
 
 #include "void_amd.h"
@@ -214,6 +215,70 @@ __global__ __launch_bounds__(kQbThreads) void b_quant_kernel(const float* __rest
     q[i] = (int8_t)code(b[i]);
 }
 
+// b_quant_kernel with the codes in rows of pitch ldq: a thread takes four
+// columns of one row (one 16-byte load, any alignment of b's rows, and one
+// 4-byte store), a group past column N writes zeros.  Bound by b's bytes, as
+// the flat kernel is (3001 x 730: 5.2 us against 5.6 us flat); the padded
+// rows let the SpMM run its LDS-DMA ring on any N.
+__global__ __launch_bounds__(kQbThreads) void b_quant_rows_kernel(const float* __restrict__ b, int32_t K, int32_t N,
+                                                                const uint32_t* __restrict__ partials,
+                                                                int32_t n_partials, int8_t* __restrict__ q,
+                                                                int32_t ldq, float* __restrict__ scale_out) {
+  __shared__ uint32_t red[kQbThreads / 64];
+  uint32_t m = 0;
+  for (int i = threadIdx.x; i < n_partials; i += kQbThreads) m = max(m, partials[i]);
+  m = block_max_u32(m, red);
+  // torch.clamp(scale, min=1e-8) keeps a NaN scale (fmaxf would drop it).
+  const float amax = __uint_as_float(m) / 128.0f;
+  const float scale = amax != amax ? amax : fmaxf(amax, 1e-8f);
+  if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = scale;
+  auto code = [&](float x) -> uint32_t {
+    const float r = __builtin_rintf(__fdiv_rn(x, scale));
+    return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(r, -128.0f), 127.0f);
+  };
+  const uint32_t per_row = (uint32_t)ldq / 4, total = (uint32_t)K * per_row;
+  for (uint32_t i = blockIdx.x * kQbThreads + threadIdx.x; i < total; i += gridDim.x * kQbThreads) {
+    const uint32_t k = i / per_row, c = 4 * (i - k * per_row);
+    const float* src = b + (int64_t)k * N + c;
+    float x[4] = {0.f, 0.f, 0.f, 0.f};
+    if ((int32_t)c + 4 <= N) __builtin_memcpy(x, src, 16);
+    else
+      for (int e = 0; e < 4; ++e)
+        if ((int32_t)c + e < N) x[e] = src[e];
+    uint32_t w = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w |= ((int32_t)c + e < N ? code(x[e]) : 0u) << (8 * e);
+    reinterpret_cast<uint32_t*>(q)[i] = w;
+  }
+}
+
+// Rows of bytes at any alignment to rows of 16-byte chunks: a thread writes one
+// chunk from one 16-byte load of any alignment (the row's last chunk byte by
+// byte, zeros past cols).
+__global__ __launch_bounds__(256) void copy_rows_b8_kernel(const uint8_t* __restrict__ src, int64_t ld_src,
+                                                          int32_t rows, int32_t cols, uint8_t* __restrict__ dst,
+                                                          int64_t ld_dst) {
+  typedef int v4i __attribute__((ext_vector_type(4)));
+  const uint32_t per_row = ((uint32_t)cols + 15) / 16;
+  const uint32_t total = (uint32_t)rows * per_row;
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+    const uint32_t r = i / per_row;
+    const int32_t c = (int32_t)(i - r * per_row) * 16;
+    const uint8_t* s = src + (int64_t)r * ld_src + c;
+    v4i v;
+    if (c + 16 <= cols) {
+      __builtin_memcpy(&v, s, 16);
+    } else {
+      uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (c + e < cols) w[e >> 2] |= (uint32_t)s[e] << (8 * (e & 3));
+      v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    }
+    *reinterpret_cast<v4i*>(dst + (int64_t)r * ld_dst + c) = v;
+  }
+}
+
 // dst[c][r] = src[r][c] for a rows x cols byte matrix (int8 or E4M3 codes):
 // a column-major B made row-major for the SpMM's LDS-DMA ring.  A workgroup
 // moves a 64-row x 256-column tile through LDS: 16-byte loads along the
@@ -270,6 +335,46 @@ int void_quantize_b_i8(const float* b, int64_t n, int8_t* q, float* scale, uint3
   const int gq = (int)std::min<int64_t>(2048, std::max<int64_t>(1, (n + 4095) / 4096));
   hipLaunchKernelGGL(b_quant_kernel, dim3(gq), dim3(kQbThreads), 0, stream, b, n, partials, g, q, scale);
   e = hipGetLastError();
+  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
+  return VOID_OK;
+}
+
+int void_quantize_b_i8_rows(const float* b, int32_t K, int32_t N, int8_t* q, int32_t ldq, float* scale,
+                            uint32_t* partials, hipStream_t stream) {
+  void_internal_fail(VOID_OK, "");
+  if (K < 0 || N < 0) return void_internal_fail(VOID_ERR_ARG, "negative size");
+  if ((int64_t)K * N == 0) return VOID_OK;
+  if (!b || !q || !scale || !partials) return void_internal_fail(VOID_ERR_ARG, "null pointer");
+  if ((uintptr_t)b % 16 || (uintptr_t)q % 4) return void_internal_fail(VOID_ERR_ARG, "b must be 16-byte, q 4-byte aligned");
+  if (ldq < N || ldq % 4) return void_internal_fail(VOID_ERR_ARG, "ldq must be a multiple of 4 and at least N");
+  const int64_t n = (int64_t)K * N, groups = (int64_t)K * (ldq / 4);
+  if (groups > INT32_MAX) return void_internal_fail(VOID_ERR_UNSUPPORTED, "too many code groups");
+  const int g = (int)std::min<int64_t>(kQbMaxPartials, std::max<int64_t>(1, (n + 4095) / 4096));
+  hipLaunchKernelGGL(b_amax_kernel, dim3(g), dim3(kQbThreads), 0, stream, b, n, partials);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
+  const int gq = (int)std::min<int64_t>(2048, std::max<int64_t>(1, (groups + 1023) / 1024));
+  hipLaunchKernelGGL(b_quant_rows_kernel, dim3(gq), dim3(kQbThreads), 0, stream, b, K, N, partials, g, q, ldq, scale);
+  e = hipGetLastError();
+  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
+  return VOID_OK;
+}
+
+int void_copy_rows_b8(const void* src, int64_t ld_src, int32_t rows, int32_t cols, void* dst, int64_t ld_dst,
+                      hipStream_t stream) {
+  void_internal_fail(VOID_OK, "");
+  if (rows < 0 || cols < 0) return void_internal_fail(VOID_ERR_ARG, "negative size");
+  if ((int64_t)rows * cols == 0) return VOID_OK;
+  if (!src || !dst) return void_internal_fail(VOID_ERR_ARG, "null pointer");
+  if (ld_src < cols || ld_dst < cols) return void_internal_fail(VOID_ERR_ARG, "leading dimension smaller than cols");
+  if (ld_dst % 16 || (uintptr_t)dst % 16)
+    return void_internal_fail(VOID_ERR_UNSUPPORTED, "void_copy_rows_b8 writes 16-byte aligned rows");
+  const int64_t chunks = (int64_t)rows * ((cols + 15) / 16);
+  if (chunks > INT32_MAX) return void_internal_fail(VOID_ERR_UNSUPPORTED, "too many chunks");
+  const int g = (int)std::min<int64_t>(8192, (chunks + 255) / 256);
+  hipLaunchKernelGGL(copy_rows_b8_kernel, dim3(g), dim3(256), 0, stream, static_cast<const uint8_t*>(src), ld_src, rows,
+                     cols, static_cast<uint8_t*>(dst), ld_dst);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
   return VOID_OK;
 }

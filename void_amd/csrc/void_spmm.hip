@@ -89,6 +89,7 @@ struct Params {
   int64_t ldb;
   int64_t ldc;
   float b_scale;
+  int32_t b_scale_stride;  // 1: b_scale_vec[N]; 0: b_scale_vec holds one scale for every column
   int32_t per_tensor_a;
   int32_t M, N, K;
   int32_t n_panels;
@@ -723,7 +724,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const int cc = min(col0 + c, cmax);
-      vs[c] = sbp[p.b_scale_vec ? cc : 0];
+      vs[c] = sbp[p.b_scale_vec ? cc * p.b_scale_stride : 0];
       vb[c] = bip[p.bias ? cc : 0];
     }
 #pragma unroll
@@ -946,8 +947,8 @@ int launch(const Params& p, int grid, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// Column-group kernel: row-major B with 16-byte aligned rows, or
-// column-major B with K % 32 == 0.
+// Column-group kernel: row-major B with 16-byte aligned rows (any N), or
+// column-major B with 16-byte aligned columns and K % 32 == 0.
 //
 // One workgroup = 4 wave64s = one work item x one 128-column panel, as for
 // spmm_bsr_kernel, but every wave runs all of the item's tiles for its own 32
@@ -1242,7 +1243,7 @@ __global__ __launch_bounds__(kThreads * KS) __attribute__((amdgpu_waves_per_eu(
     const float* sbp = p.b_scale_vec ? p.b_scale_vec : reinterpret_cast<const float*>(p.row_ptr);
     const float* bip = p.bias ? p.bias : reinterpret_cast<const float*>(p.row_ptr);
     const int cc = min(col, p.N - 1);
-    const float vs = sbp[p.b_scale_vec ? cc : 0];
+    const float vs = sbp[p.b_scale_vec ? cc * p.b_scale_stride : 0];
     const float vb = bip[p.bias && !p.bias_per_row ? cc : 0];  // a per-row bias has M entries
     sb = p.b_scale_vec ? vs : p.b_scale;
     bias = p.bias ? vb : 0.f;
@@ -2259,6 +2260,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   p.ldb = d->ldb;
   p.b_scale = d->b_scale;
   p.b_scale_vec = d->b_scale_vec;
+  p.b_scale_stride = d->b_scale_one ? 0 : 1;
   p.bias = d->bias;
   p.c = d->c;
   p.ldc = d->ldc;
@@ -2320,6 +2322,15 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     layout = kRowLds;
   else
     layout = (c_ok && (bu % 4 == 0) && (d->ldb % 4 == 0)) ? kRowVec : kRowByte;
+  // What the column-group kernel asks of an 8-bit B: 16-byte aligned rows (or
+  // columns, with whole 32-row slabs).  Its 16-byte reads start at columns
+  // below N that are multiples of 16, so with a row pitch that is a multiple
+  // of 16 they stay inside the row for any N; what lies past N only feeds
+  // output columns that are never stored.  C may have any width and
+  // alignment: blocks that are cut off or unaligned leave element by element.
+  // (5003 x 3001, 2950 tiles, N = 730, float B: the general kernel's bytewise
+  // loads 132 us, this kernel on padded rows 21 us.)
+  const bool b16 = (bu % 16 == 0) && (d->ldb % 16 == 0) && (!d->b_col_major || a->K % kTile == 0);
   if (grid_exact > 0x7fffffff) return fail(VOID_ERR_ARG, "grid too large");
   const int grid = p.xcd_exact ? (int)grid_exact : (int)grid64;
 
@@ -2436,10 +2447,9 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   const bool offsets_ok = (int64_t)a->n_blocks * kTile * kTile < kLim && b_span < kLim &&
                           (int64_t)a->M * d->ldc * esz < kLim;
 
-  const bool cg_ok = (layout == kRowLds || layout == kColVec) && plan->chunk_tiles <= kCgMaxTiles && offsets_ok &&
-                     !force_bsr;
+  const bool cg_ok = b16 && plan->chunk_tiles <= kCgMaxTiles && offsets_ok && !force_bsr;
   if (cg_ok) {
-    const bool bcol = layout == kColVec;
+    const bool bcol = d->b_col_major;
     // Row-major B takes the LDS-DMA ring unless VOID_AMD_KERNEL=cg asks for
     // the register-staged loop.
     const bool dma = !bcol && !force_cg;

@@ -331,8 +331,21 @@ def _b_scale_args(b_scale, N: int, device) -> Tuple[float, Optional[torch.Tensor
 def _quantize_b_per_tensor(b: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """A float B quantised per tensor as the reference does (symmetric int8,
     min-max scale), the scale left on the device: for a contiguous fp32 B
-    on the gfx950 kernels (void_quantize_b_i8), otherwise with quantize_tensor."""
+    on the gfx950 kernels (void_quantize_b_i8, or void_quantize_b_i8_rows
+    into rows of an aligned pitch when b is 2-D with rows that are not whole
+    16-byte chunks of codes), otherwise with quantize_tensor."""
     if b.dtype == torch.float32 and b.is_contiguous() and b.data_ptr() % 16 == 0:
+        if b.dim() == 2 and b.shape[1] % 16 and b.shape[0] * tuning.aligned_pitch(b.shape[1]) < 1 << 31:
+            K, N = b.shape
+            pitch = tuning.aligned_pitch(N)
+            q = torch.empty(K, pitch, dtype=torch.int8, device=b.device)[:, :N]
+            scale = torch.empty(1, dtype=torch.float32, device=b.device)
+            partials = torch.empty(1024, dtype=torch.int32, device=b.device)
+            st = _lib.lib().void_quantize_b_i8_rows(b.data_ptr(), K, N, q.data_ptr(), pitch, scale.data_ptr(),
+                                                    partials.data_ptr(),
+                                                    torch.cuda.current_stream(b.device).cuda_stream)
+            _lib.check(st, "void_quantize_b_i8_rows")
+            return q, scale
         q = torch.empty(b.shape, dtype=torch.int8, device=b.device)
         scale = torch.empty(1, dtype=torch.float32, device=b.device)
         partials = torch.empty(1024, dtype=torch.int32, device=b.device)
@@ -379,10 +392,13 @@ def void_spmm_int8(
     if bias is not None and tuple(bias.shape) != (N,):
         raise ValueError(f"bias must be [{N}], got {tuple(bias.shape)}")
     _runtime.require_gpu(b, "B")
-    if b.dtype != torch.int8:
-        b, b_scale = _quantize_b_per_tensor(b)
-    scalar_scale, scale_vec, per_column = _b_scale_args(b_scale, N, b.device)
-    per_column = per_column and b_scale.numel() != 1 if isinstance(b_scale, torch.Tensor) else per_column
+    one = b.dtype != torch.int8
+    if one:  # the scale goes to the kernel where the quantiser left it
+        b, scale_vec = _quantize_b_per_tensor(b)
+        scalar_scale, per_column = 1.0, False
+    else:
+        scalar_scale, scale_vec, per_column = _b_scale_args(b_scale, N, b.device)
+        per_column = per_column and b_scale.numel() != 1 if isinstance(b_scale, torch.Tensor) else per_column
     if epilogue is None:
         epilogue = "per_block" if per_column else "row_mean"
     if epilogue not in _lib.EPILOGUES:
@@ -409,7 +425,7 @@ def void_spmm_int8(
     chunk = chunk_tiles or tuning.select_chunk("int8", a.n_blocks, N, dbsr.max_row)
     if bias is not None:
         bias = bias.to(device=b.device, dtype=torch.float32).contiguous()
-    return _runtime.launch("int8", dbsr, b, b_scale=scalar_scale, b_scale_vec=scale_vec, out=out,
+    return _runtime.launch("int8", dbsr, b, b_scale=scalar_scale, b_scale_vec=scale_vec, b_scale_one=one, out=out,
                            epilogue=_lib.EPILOGUES[epilogue], activation=get_activation_code(activation),
                            bias=bias, chunk=chunk)
 

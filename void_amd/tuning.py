@@ -86,3 +86,31 @@ def copy_col_major_b(n_blocks: int, K: int) -> bool:
     if env in ("0", "1"):
         return env == "1"
     return 32 * n_blocks >= COL_MAJOR_COPY_RATIO * max(K, 1)
+
+
+# An 8-bit row-major B whose rows are not 16-byte aligned (N or the row pitch
+# not a multiple of 16, or a shifted view) cannot feed the LDS-DMA ring; the
+# general kernel gathers it by 4-byte loads where rows and C allow that
+# (``dword``), byte by byte otherwise.  A copy to aligned rows costs a launch
+# and one pass over B (2-4 us).  Against the bytewise loads it always pays
+# (46 tiles, N = 155: 24.1 -> 8.2 us; 2950 tiles, N = 730: 131 -> 19.6 us with
+# the copy).  Against the 4-byte loads it pays where the slabs gathered exceed
+# 32 times B over more than one panel (14336 x 4096, 14336 tiles, N = 500:
+# 51 -> 43 us, N = 2004: 161 -> 121 us; 4096 x 4096, 1638 tiles (13 x B), N = 500:
+# 10.2 against 14.1 us with the copy; 14336 tiles, N = 100: 15.8 against 16.4).
+# VOID_AMD_PAD=0 / 1 forces it off / on.
+def aligned_pitch(N: int) -> int:
+    """Row pitch of an aligned copy of an 8-bit B: whole 128-byte lines, so
+    that a panel's slab rows start on a line (N up to 64: whole 16-byte
+    chunks, one line holding several rows)."""
+    return (N + 127) // 128 * 128 if N > 64 else (N + 15) // 16 * 16
+
+
+def copy_unaligned_b(n_blocks: int, K: int, N: int, dword: bool) -> bool:
+    import os
+    env = os.environ.get("VOID_AMD_PAD")
+    if env in ("0", "1"):
+        return env == "1"
+    if K * aligned_pitch(N) >= 1 << 31:  # past the ring's 31-bit offsets
+        return False
+    return not dword or (N > PANEL_COLUMNS and 32 * n_blocks >= COL_MAJOR_COPY_RATIO * max(K, 1))
