@@ -69,7 +69,7 @@ class VOIDSpMMFunction(Function):
         if ctx.needs_input_grad[6]:
             at = _vt(a_values.detach().permute(0, 2, 1).contiguous(), cols, rows, (K, M),
                      ctx.a_tile_size[::-1], ctx.a_n_blocks)
-            grad_b = float_spmm(at, grad_output.contiguous()).to(b.dtype)
+            grad_b = float_spmm(at, _runtime.contiguous_2d(grad_output)).to(b.dtype)
         if ctx.needs_input_grad[0]:
             grad_a = _runtime.sddmm_tiles(grad_output, b, rows, cols, (M, K), a_values.dtype,
                                           layout=_layout(rows, cols, (M, K)) if rows.is_cuda else None)

@@ -286,7 +286,7 @@ def void_spmm_fp8(a: FP8VOIDTensor, b: torch.Tensor, output_dtype: torch.dtype =
         # A 16-bit B is taken as it is, on the 16-bit MFMA (A decoded exactly
         # to its type), when its rows and the output's are 16-byte aligned
         # and N % 8 == 0; otherwise it is widened to fp32 below.
-        b16 = b if b.stride(1) == 1 else b.contiguous()
+        b16 = b if b.stride(1) == 1 else _runtime.contiguous_2d(b)
         if (N % 8 == 0 and b16.stride(0) % 8 == 0 and b16.data_ptr() % 16 == 0 and a.n_blocks * 1024 < (1 << 31)
                 and (K + 31) // 32 * 32 * b16.stride(0) * 2 < (1 << 31) and M * N * out.element_size() < (1 << 31)):
             kind = "fp8_bf16b" if b.dtype == torch.bfloat16 else "fp8_f16b"
@@ -328,7 +328,7 @@ def _launch_f32b(dbsr, b: torch.Tensor, out: Optional[torch.Tensor], output_dtyp
     M = dst.shape[0]
     N4 = (N + 3) // 4 * 4
     if N4 == N:
-        b32 = b.to(torch.float32).contiguous()
+        b32 = _runtime.contiguous_2d(b.to(torch.float32))
         if b32.data_ptr() % 16:
             b32 = b32.clone()
         tgt = out if out is not None else torch.empty(M, N, dtype=output_dtype, device=b.device)

@@ -202,9 +202,9 @@ class FusedSparseLinear(torch.nn.Module):
         return vt
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from .ops import float_spmm
+        from . import _runtime
         x_flat = x.reshape(-1, self.in_features)
-        b = x_flat.t().contiguous()  # [in, batch], row-major, as the reference passes it
+        b = _runtime.contiguous_2d(x_flat.t())  # [in, batch], row-major, as the reference passes it
         bias = self.bias.detach() if self.bias is not None else None
         vt = self.get_void_tensor()
         if vt.n_blocks == 0:

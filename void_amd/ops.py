@@ -70,14 +70,14 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
     entry = "void_spmm_f32"
     bk = None
     if a.values.dtype == b.dtype and b.dtype in _K16:
-        bk = b if b.stride(1) == 1 else b.contiguous()
+        bk = b if b.stride(1) == 1 else _runtime.contiguous_2d(b)
         if not _fits16(a, bk, target):
             bk = None
     if bk is not None:
         entry = _K16[b.dtype]
         dbsr = a.device_bsr(b.dtype)
     else:
-        bk = b.to(torch.float32).contiguous()
+        bk = _runtime.contiguous_2d(b.to(torch.float32))
         dbsr = a.device_bsr()
     if plan is None:
         plan = dbsr.plan(F32_CHUNK)
