@@ -228,3 +228,39 @@ def test_inference_mode(gpu):
         q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu")).to(gpu)
         z = void_amd.void_spmm_int8(q, torch.from_numpy(bq).to(gpu), b_scale=torch.from_numpy(bs).to(gpu))
         assert torch.equal(z, z_ref)
+
+
+def test_layout_plans_shared_and_streams(gpu):
+    """One structure's plans serve every step, also from a second stream, with
+    bit-identical results; capture is refused as before."""
+    from void_amd import autograd
+    case = cases.uniform_blocks(256, 4096, 96, 700, seed=5)  # rows beyond 64 tiles: split plans
+    vt = cases.make_void_tensor(case, "cpu").to(gpu)
+    mod = void_amd.VOIDSpMM(vt)
+    b = torch.from_numpy(case.b).to(gpu)
+
+    def step():
+        x = b.clone().requires_grad_()
+        mod.zero_grad(set_to_none=True)
+        y = mod(x)
+        y.backward(torch.ones_like(y))
+        return [y.detach().clone(), x.grad.clone(), mod.values.grad.clone()]
+
+    ref = step()
+    lay = autograd._layout(mod.block_rows, mod.block_cols, mod.shape)
+    plan = lay.plans[64]
+    assert plan.n_split_tiles > 0
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = step()
+    torch.cuda.current_stream().wait_stream(side)
+    for other in (got, step()):
+        assert all(torch.equal(p, q) for p, q in zip(ref, other))
+    assert lay.plans[64] is plan and len(plan.workspaces) == 2
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError, match="captured"):
+        with torch.cuda.graph(g):
+            mod(b)
+    assert torch.equal(mod(b).detach(), ref[0])

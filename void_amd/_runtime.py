@@ -37,6 +37,31 @@ MAX_STREAM_WORKSPACES = 8
 MAX_SPARE_WORKSPACE = 64 << 20
 
 
+def raw_stream(device: torch.device) -> int:
+    """Handle of torch's current stream on a GPU device
+    (torch.cuda.current_stream(device).cuda_stream without the Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None
+                                              else torch.cuda.current_device())
+
+
+_DEVICE_KEYS: Dict[torch.device, str] = {}
+
+
+def device_key(device: torch.device) -> str:
+    """str(device), kept per device."""
+    k = _DEVICE_KEYS.get(device)
+    if k is None:
+        k = _DEVICE_KEYS[device] = str(device)
+    return k
+
+
+def vector_f32(t: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """t as a contiguous fp32 vector on the device; t itself when it is one."""
+    if t.dtype is torch.float32 and t.device == device and t.dim() == 1 and t.is_contiguous():
+        return t
+    return t.reshape(-1).to(device=device, dtype=torch.float32).contiguous()
+
+
 @dataclass
 class DevicePlan:
     items: torch.Tensor          # int32 [n_items, 32] on device (void_work_item)
@@ -51,13 +76,21 @@ class DevicePlan:
     capture_by_id: Dict[Tuple[int, int, int], torch.Tensor] = field(default_factory=dict)  # (capture, stream, nbytes)
     ws_sizes: Dict[int, int] = field(default_factory=dict)  # N -> void_workspace_bytes
     _cplan: Optional["_lib.Plan"] = None
+    _cplan_ref: object = None
 
     def cplan(self) -> "_lib.Plan":
         """The C descriptor of this plan (its arrays never change: built once)."""
         if self._cplan is None:
             self._cplan = _lib.Plan(items=self.items.data_ptr(), n_items=self.n_items,
                                     n_split_tiles=self.n_split_tiles, n_slots=self.n_slots, chunk_tiles=self.chunk)
+            self._cplan_ref = ctypes.byref(self._cplan)
         return self._cplan
+
+    def cplan_ref(self):
+        """The same by reference, as the C calls take it."""
+        if self._cplan_ref is None:
+            self.cplan()
+        return self._cplan_ref
 
     def counter_bytes(self, N: int) -> int:
         """Bytes of split-row arrival counters at the start of the workspace
@@ -249,6 +282,7 @@ class DeviceBsr:
     plans: Dict[int, DevicePlan] = field(default_factory=dict)
     _max_row: Optional[int] = None
     _desc: Optional[_lib.BsrDesc] = None
+    _desc_ref: object = None
     order: Optional[torch.Tensor] = None  # BSR position -> index of the source tile
     src_key: tuple = ()                   # source_key of the tensors the arrays were gathered from
 
@@ -291,7 +325,14 @@ class DeviceBsr:
         """The C descriptor of this matrix (its arrays never change: built once)."""
         if self._desc is None:
             self._desc = self._make_desc()
+            self._desc_ref = ctypes.byref(self._desc)
         return self._desc
+
+    def desc_ref(self):
+        """The same by reference, as the C calls take it."""
+        if self._desc_ref is None:
+            self.desc()
+        return self._desc_ref
 
     def _make_desc(self) -> _lib.BsrDesc:
         return _lib.BsrDesc(
@@ -324,9 +365,10 @@ def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torc
     else:
         s = s.index_select(0, lay.order).contiguous() if s.numel() else s.contiguous()
     return DeviceBsr(tiles=tiles, scales=s, row_ptr=lay.row_ptr, col_idx=lay.col_idx,
-                     row_ptr_host=lay.row_ptr_host, col_idx_host=lay.col_idx.cpu().numpy(),
+                     row_ptr_host=lay.row_ptr_host,
+                     col_idx_host=lay.col_idx_host if lay.col_idx_host is not None else lay.col_idx.cpu().numpy(),
                      per_tensor=per_tensor, M=M, K=K,
-                     n_blocks=int(values.shape[0]), n_block_rows=n_br, order=lay.order)
+                     n_blocks=int(values.shape[0]), n_block_rows=n_br, order=lay.order, plans=lay.plans)
 
 
 def source_key(*tensors: torch.Tensor) -> tuple:
@@ -345,10 +387,11 @@ def require_gpu(t: torch.Tensor, what: str) -> None:
 
 def dense_operand(b: torch.Tensor) -> Tuple[torch.Tensor, int, bool]:
     """(tensor, ld, col_major) for B without copying when B is row- or column-major."""
-    if b.stride(1) == 1 and (b.stride(0) >= b.shape[1] or b.shape[0] <= 1):
-        return b, max(b.stride(0), b.shape[1]), False
-    if b.stride(0) == 1 and (b.stride(1) >= b.shape[0] or b.shape[1] <= 1):
-        return b, max(b.stride(1), b.shape[0]), True
+    (s0, s1), (K, N) = b.stride(), b.shape
+    if s1 == 1 and (s0 >= N or K <= 1):
+        return b, max(s0, N), False
+    if s0 == 1 and (s1 >= K or N <= 1):
+        return b, max(s1, K), True
     b = b.contiguous()
     return b, b.shape[1], False
 
@@ -361,7 +404,7 @@ def row_major_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
     out = torch.empty(K, N, dtype=b.dtype, device=b.device)
     if K % 16 == 0 and N % 16 == 0 and ld % 16 == 0 and b.data_ptr() % 16 == 0:
         st = _lib.lib().void_transpose_b8(b.data_ptr(), ld, N, K, out.data_ptr(), N,
-                                          torch.cuda.current_stream(b.device).cuda_stream)
+                                          raw_stream(b.device))
         _lib.check(st, "void_transpose_b8")
         return out
     out.copy_(b)
@@ -386,7 +429,7 @@ def contiguous_2d(t: torch.Tensor) -> torch.Tensor:
         return t.contiguous()
     out = torch.empty(R, C, dtype=t.dtype, device=t.device)
     st = _lib.lib().void_transpose(t.data_ptr(), t.stride(1), C, R, out.data_ptr(), C, t.element_size(),
-                                   torch.cuda.current_stream(t.device).cuda_stream)
+                                   raw_stream(t.device))
     _lib.check(st, "void_transpose")
     return out
 
@@ -397,7 +440,7 @@ def aligned_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
     pitch = tuning.aligned_pitch(N)
     out = torch.empty(K, pitch, dtype=b.dtype, device=b.device)[:, :N]
     st = _lib.lib().void_copy_rows_b8(b.data_ptr(), ld, K, N, out.data_ptr(), pitch,
-                                      torch.cuda.current_stream(b.device).cuda_stream)
+                                      raw_stream(b.device))
     _lib.check(st, "void_copy_rows_b8")
     return out
 
@@ -414,7 +457,8 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
     if col_major and kind in ("int8", "fp8") and tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K):
         b_t, ldb, col_major = row_major_copy_b8(b_t, ldb), N, False  # for the LDS-DMA ring
     target = out
-    if out.stride(1) != 1 or out.stride(0) < N:
+    so0, so1 = out.stride()
+    if so1 != 1 or so0 < N:
         target = torch.empty(out.shape, dtype=out.dtype, device=out.device)
     if (kind in ("int8", "fp8") and N and not col_major and (ldb % 16 or b_t.data_ptr() % 16)
             and chunk <= tuning.FP32_B_MAX_CHUNK):
@@ -423,35 +467,27 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
             b_t = aligned_copy_b8(b_t, ldb)
             ldb = b_t.stride(0)
     plan = dbsr.plan(chunk)
-    stream = torch.cuda.current_stream(out.device).cuda_stream
+    stream = raw_stream(out.device)
     ws, ws_bytes = plan.workspace(N, out.device, stream)
-    cplan = plan.cplan()
-    dense = _lib.DenseArgs(
-        b=b_t.data_ptr(), ldb=ldb, b_col_major=int(col_major), N=N, b_scale=float(b_scale),
-        b_scale_vec=b_scale_vec.data_ptr() if b_scale_vec is not None else None,
-        bias=bias.data_ptr() if bias is not None else None,
-        c=target.data_ptr(), ldc=target.stride(0), out_dtype=_OUT_CODES[target.dtype],
-        activation=activation)
-    if b_scale_one:
-        dense.b_scale_one = 1
-    desc = dbsr.desc()
-    ws_ptr = ws.data_ptr() if ws is not None else None
+    # Fields in the struct's order.
+    dense = _lib.DenseArgs(b_t.data_ptr(), ldb, col_major, N, b_scale,
+                           b_scale_vec.data_ptr() if b_scale_vec is not None else None,
+                           bias.data_ptr() if bias is not None else None, target.data_ptr(), target.stride(0),
+                           _OUT_CODES[target.dtype], activation, 0, b_scale_one)
+    args = (plan.cplan_ref(), ws.data_ptr() if ws is not None else None, ws_bytes, stream)
     if kind == "int8":
-        st = lib.void_spmm_int8(ctypes.byref(desc), ctypes.byref(dense), epilogue, ctypes.byref(cplan),
-                                ws_ptr, ws_bytes, stream)
+        st = lib.void_spmm_int8(dbsr.desc_ref(), ctypes.byref(dense), epilogue, *args)
     elif kind == "fp8":
-        st = lib.void_spmm_fp8(ctypes.byref(desc), ctypes.byref(dense), ctypes.byref(cplan),
-                               ws_ptr, ws_bytes, stream)
+        st = lib.void_spmm_fp8(dbsr.desc_ref(), ctypes.byref(dense), *args)
     elif kind == "fp8_f32b":
-        st = lib.void_spmm_fp8_f32b(ctypes.byref(desc), ctypes.byref(dense), ctypes.byref(cplan),
-                                    ws_ptr, ws_bytes, stream)
+        st = lib.void_spmm_fp8_f32b(dbsr.desc_ref(), ctypes.byref(dense), *args)
     elif kind in ("fp8_bf16b", "fp8_f16b"):
         bdt = _lib.DT_BF16 if kind == "fp8_bf16b" else _lib.DT_F16
-        st = lib.void_spmm_fp8_b16(ctypes.byref(desc), ctypes.byref(dense), bdt, ctypes.byref(cplan),
-                                   ws_ptr, ws_bytes, stream)
+        st = lib.void_spmm_fp8_b16(dbsr.desc_ref(), ctypes.byref(dense), bdt, *args)
     else:
         raise ValueError(f"unknown SpMM kind {kind!r}")
-    _lib.check(st, f"void_spmm_{kind}")
+    if st:
+        _lib.check(st, f"void_spmm_{kind}")
     if target is not out:
         out.copy_(target)
     return out
@@ -475,7 +511,7 @@ def quantize_tiles_i8(values: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]
     q = torch.empty(values.shape, dtype=torch.int8, device=values.device)
     scales = torch.empty(n, dtype=torch.float32, device=values.device)
     st = _lib.lib().void_quantize_tiles_i8(values.data_ptr(), n, q.data_ptr(), scales.data_ptr(),
-                                           torch.cuda.current_stream(values.device).cuda_stream)
+                                           raw_stream(values.device))
     _lib.check(st, "void_quantize_tiles_i8")
     return q, scales
 
@@ -487,7 +523,7 @@ def quantize_tiles_fp8(values: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor
     scales = torch.empty(n, dtype=torch.float32, device=values.device)
     amax = torch.empty(n, dtype=torch.float32, device=values.device)
     st = _lib.lib().void_quantize_tiles_fp8(values.data_ptr(), n, q.data_ptr(), scales.data_ptr(),
-                                            amax.data_ptr(), torch.cuda.current_stream(values.device).cuda_stream)
+                                            amax.data_ptr(), raw_stream(values.device))
     _lib.check(st, "void_quantize_tiles_fp8")
     return q, scales, amax
 
@@ -504,7 +540,7 @@ def csr_to_tiles(indptr: np.ndarray, indices: np.ndarray, data: np.ndarray, shap
     ws_bytes = lib.void_csr_workspace_bytes(M, N)
     if ws_bytes == 0:
         return None
-    stream = torch.cuda.current_stream(device).cuda_stream
+    stream = raw_stream(device)
     d_indptr = torch.from_numpy(np.ascontiguousarray(indptr, dtype=np.int32)).to(device)
     d_indices = torch.from_numpy(np.ascontiguousarray(indices, dtype=np.int32)).to(device)
     d_data = torch.from_numpy(np.ascontiguousarray(data, dtype=np.float32)).to(device)
@@ -541,7 +577,7 @@ def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor,
         return out
     if N == 0:
         return out.zero_()
-    stream = torch.cuda.current_stream(grad_c.device).cuda_stream
+    stream = raw_stream(grad_c.device)
     entry16 = {torch.bfloat16: "void_sddmm_rows_bf16", torch.float16: "void_sddmm_rows_f16"}.get(grad_c.dtype)
     if layout is not None and entry16 is not None and b.dtype == grad_c.dtype:
         # 16-bit operands of one dtype on the 16-bit MFMA (16-byte rows).

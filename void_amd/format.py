@@ -64,6 +64,10 @@ class BsrLayout:
     row_ptr: torch.Tensor   # int32 [n_block_rows + 1] on device
     col_idx: torch.Tensor   # int32 [n_blocks] on device
     row_ptr_host: np.ndarray  # int32 copy on the host, for the planner
+    col_idx_host: Optional[np.ndarray] = None
+    # Stream-K plans by chunk: they depend on the structure only, so every
+    # device copy of tiles with this layout shares them.
+    plans: dict = field(default_factory=dict)
     sddmm_groups: Optional[torch.Tensor] = None  # int32 [n_groups, 3], built on first use
 
     def row_groups(self) -> torch.Tensor:
@@ -101,6 +105,7 @@ def build_bsr_layout(block_rows: torch.Tensor, block_cols: torch.Tensor, n_block
         row_ptr=torch.from_numpy(row_ptr).to(device),
         col_idx=torch.from_numpy(col_idx).to(device),
         row_ptr_host=row_ptr,
+        col_idx_host=col_idx,
     )
 
 
@@ -132,12 +137,14 @@ class VOIDTensor:
         and dtype and gathered again when the values change in place, since
         the reference reads them on every call."""
         from . import _runtime
-        key = str(self.values.device) if dtype == torch.float32 else f"{self.values.device}/{dtype}"
+        key = _runtime.device_key(self.values.device)
+        if dtype != torch.float32:
+            key = f"{key}/{dtype}"
         src = _runtime.source_key(self.values)
         d = self._device_bsr.get(key)
         if d is None:
-            ones = torch.ones(1, dtype=torch.float32, device=self.values.device)
-            d = _runtime.make_device_bsr(self.values.detach().to(dtype).contiguous(), ones, self.block_rows,
+            none = torch.empty(0, dtype=torch.float32, device=self.values.device)  # float tiles have no scales
+            d = _runtime.make_device_bsr(self.values.detach().to(dtype).contiguous(), none, self.block_rows,
                                          self.block_cols, self.shape, self.tile_size, self.values.device, True,
                                          layout=self._bsr_layout)
             d.src_key = src

@@ -17,6 +17,8 @@ from typing import Dict, Literal, Optional, Tuple, Union
 import torch
 
 from . import _lib, _runtime, tuning
+from .fusion import apply_activation_torch, get_activation_code
+from .int_quant import _b_scale_args
 
 
 class FP8Format(Enum):
@@ -197,7 +199,7 @@ class FP8VOIDTensor:
     def device_bsr(self) -> "_runtime.DeviceBsr":
         """Block-row-major device copy of the tiles (built once per device,
         gathered again when the codes or scales change in place)."""
-        key = str(self.values_fp8.device)
+        key = _runtime.device_key(self.values_fp8.device)
         scales = self.scaling_info.scale.reshape(-1)
         src = _runtime.source_key(self.values_fp8, self.scaling_info.scale)
         d = self._device_bsr.get(key)
@@ -255,7 +257,6 @@ def void_spmm_fp8(a: FP8VOIDTensor, b: torch.Tensor, output_dtype: torch.dtype =
     float_b = b.dtype != torch.float8_e4m3fn
     if float_b and not b.is_floating_point():
         raise TypeError(f"B must be float8_e4m3fn or a float tensor, got {b.dtype}")
-    from .int_quant import _b_scale_args
     scalar_scale, scale_vec, _ = _b_scale_args(b_scale, N, b.device)
     if out is None:
         out = torch.empty(M, N, dtype=output_dtype, device=b.device)
@@ -264,15 +265,13 @@ def void_spmm_fp8(a: FP8VOIDTensor, b: torch.Tensor, output_dtype: torch.dtype =
     if a.n_blocks == 0:
         out.zero_()
         if bias is not None or activation != "none":
-            from .fusion import apply_activation_torch
             out.copy_(apply_activation_torch(out.float() + (bias if bias is not None else 0), activation))
         return out
     _runtime.require_gpu(a.values_fp8, "A")
     if a.values_fp8.device != b.device:
         raise ValueError(f"A on {a.values_fp8.device}, B on {b.device}")
-    from .fusion import get_activation_code
     if bias is not None:
-        bias = bias.to(device=b.device, dtype=torch.float32).contiguous()
+        bias = _runtime.vector_f32(bias, b.device)
     dbsr = a.device_bsr()
     chunk = chunk_tiles or tuning.select_chunk("fp8", a.n_blocks, N, dbsr.max_row)
     act = get_activation_code(activation)

@@ -16,6 +16,7 @@ from typing import Dict, Literal, Optional, Tuple, Union
 import torch
 
 from . import _lib, _runtime, tuning
+from .fusion import apply_activation_torch, get_activation_code
 
 
 class IntFormat(Enum):
@@ -131,7 +132,7 @@ class Int8VOIDTensor:
         """Block-row-major device copy of the tiles (built once per device,
         gathered again when the values or scales change in place, since the
         reference reads them on every call)."""
-        key = str(self.values.device)
+        key = _runtime.device_key(self.values.device)
         src = _runtime.source_key(self.values, self.scales)
         d = self._device_bsr.get(key)
         if d is not None and d.src_key != src:
@@ -324,7 +325,7 @@ def _b_scale_args(b_scale, N: int, device) -> Tuple[float, Optional[torch.Tensor
             return 1.0, b_scale.reshape(1).to(device=device, dtype=torch.float32).expand(N).contiguous(), False
         if b_scale.numel() != N:
             raise ValueError(f"b_scale has {b_scale.numel()} entries, expected 1 or N={N}")
-        return 1.0, b_scale.reshape(-1).to(device=device, dtype=torch.float32).contiguous(), True
+        return 1.0, _runtime.vector_f32(b_scale, device), True
     return float(b_scale), None, False
 
 
@@ -343,14 +344,14 @@ def _quantize_b_per_tensor(b: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]
             partials = torch.empty(1024, dtype=torch.int32, device=b.device)
             st = _lib.lib().void_quantize_b_i8_rows(b.data_ptr(), K, N, q.data_ptr(), pitch, scale.data_ptr(),
                                                     partials.data_ptr(),
-                                                    torch.cuda.current_stream(b.device).cuda_stream)
+                                                    _runtime.raw_stream(b.device))
             _lib.check(st, "void_quantize_b_i8_rows")
             return q, scale
         q = torch.empty(b.shape, dtype=torch.int8, device=b.device)
         scale = torch.empty(1, dtype=torch.float32, device=b.device)
         partials = torch.empty(1024, dtype=torch.int32, device=b.device)
         st = _lib.lib().void_quantize_b_i8(b.data_ptr(), b.numel(), q.data_ptr(), scale.data_ptr(),
-                                           partials.data_ptr(), torch.cuda.current_stream(b.device).cuda_stream)
+                                           partials.data_ptr(), _runtime.raw_stream(b.device))
         _lib.check(st, "void_quantize_b_i8")
         return q, scale
     cfg = IntQuantConfig(format=IntFormat.INT8, symmetric=True, scale_mode=ScaleMode.PER_TENSOR)
@@ -414,17 +415,15 @@ def void_spmm_int8(
     if a.n_blocks == 0:
         out.zero_()
         if bias is not None or activation != "none":
-            from .fusion import apply_activation_torch
             out.copy_(apply_activation_torch(out.float() + (bias if bias is not None else 0), activation))
         return out
     _runtime.require_gpu(a.values, "A")
     if a.values.device != b.device:
         raise ValueError(f"A on {a.values.device}, B on {b.device}")
-    from .fusion import get_activation_code
     dbsr = a.device_bsr()
     chunk = chunk_tiles or tuning.select_chunk("int8", a.n_blocks, N, dbsr.max_row)
     if bias is not None:
-        bias = bias.to(device=b.device, dtype=torch.float32).contiguous()
+        bias = _runtime.vector_f32(bias, b.device)
     return _runtime.launch("int8", dbsr, b, b_scale=scalar_scale, b_scale_vec=scale_vec, b_scale_one=one, out=out,
                            epilogue=_lib.EPILOGUES[epilogue], activation=get_activation_code(activation),
                            bias=bias, chunk=chunk)

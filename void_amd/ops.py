@@ -61,7 +61,7 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
     if bias is not None:
         if bias.shape != ((M,) if bias_per_row else (N,)):
             raise ValueError(f"bias must be [{M if bias_per_row else N}]")
-        bias = bias.to(device=b.device, dtype=torch.float32).contiguous()
+        bias = _runtime.vector_f32(bias, b.device)
     lib = _lib.lib()
     target = out if (out.stride(1) == 1 and out.stride(0) >= N) else torch.empty_like(out)
     # 16-bit tiles times a B of the same dtype run on the 16-bit MFMA (the
@@ -83,17 +83,14 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
         plan = dbsr.plan(F32_CHUNK)
     elif plan.chunk > F32_CHUNK:
         raise ValueError(f"the float kernel takes work items of at most {F32_CHUNK} tiles, got {plan.chunk}")
-    ws, ws_bytes = plan.workspace(N, out.device)
-    cplan = _lib.Plan(items=plan.items.data_ptr(), n_items=plan.n_items, n_split_tiles=plan.n_split_tiles,
-                      n_slots=plan.n_slots, chunk_tiles=plan.chunk)
-    dense = _lib.DenseArgs(b=bk.data_ptr(), ldb=bk.stride(0), b_col_major=0, N=N, b_scale=1.0, b_scale_vec=None,
-                           bias=bias.data_ptr() if bias is not None else None, c=target.data_ptr(),
-                           ldc=target.stride(0), out_dtype=_runtime.out_code(target.dtype), activation=activation,
-                           bias_per_row=int(bias_per_row))
-    desc = dbsr.desc()
-    st = getattr(lib, entry)(ctypes.byref(desc), ctypes.byref(dense), ctypes.byref(cplan),
-                             ws.data_ptr() if ws is not None else None, ws_bytes,
-                             torch.cuda.current_stream(out.device).cuda_stream)
+    stream = _runtime.raw_stream(out.device)
+    ws, ws_bytes = plan.workspace(N, out.device, stream)
+    # Fields in the struct's order.
+    dense = _lib.DenseArgs(bk.data_ptr(), bk.stride(0), 0, N, 1.0, None, bias.data_ptr() if bias is not None else None,
+                           target.data_ptr(), target.stride(0), _runtime.out_code(target.dtype), activation,
+                           bias_per_row, 0)
+    st = getattr(lib, entry)(dbsr.desc_ref(), ctypes.byref(dense), plan.cplan_ref(),
+                             ws.data_ptr() if ws is not None else None, ws_bytes, stream)
     _lib.check(st, entry)
     if target is not out:
         out.copy_(target)

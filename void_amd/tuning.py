@@ -26,6 +26,7 @@ is fixed by the hardware instead:
 from __future__ import annotations
 
 import math
+import os
 
 GFX950_CUS = 256
 GFX950_XCDS = 8
@@ -81,7 +82,6 @@ COL_MAJOR_COPY_RATIO = 32
 
 
 def copy_col_major_b(n_blocks: int, K: int) -> bool:
-    import os
     env = os.environ.get("VOID_AMD_BT")
     if env in ("0", "1"):
         return env == "1"
@@ -107,7 +107,6 @@ def aligned_pitch(N: int) -> int:
 
 
 def copy_unaligned_b(n_blocks: int, K: int, N: int, dword: bool) -> bool:
-    import os
     env = os.environ.get("VOID_AMD_PAD")
     if env in ("0", "1"):
         return env == "1"
