@@ -331,6 +331,13 @@ int void_csr_to_tiles(const int32_t* indptr, const int32_t* indices, const float
                       void* workspace, size_t workspace_bytes, int64_t n_blocks, float* values,
                       int32_t* block_rows, int32_t* block_cols, int64_t* morton, hipStream_t stream);
 
+/* dst[p] = transpose(src[order[p]]) for n 32x32 tiles of 2- or 4-byte elements
+ * (elem_bytes), 16-byte aligned: the tiles of A^T in their block-row order,
+ * the operand of the gradient of B (the reference permutes and makes
+ * contiguous, void/autograd.py:175-189). */
+int void_gather_tiles_t(const void* src, const int64_t* order, int32_t n, int32_t elem_bytes, void* dst,
+                        hipStream_t stream);
+
 /* ---- Backward: gradient on the nonzero tiles (SDDMM) ------------------ */
 
 /* grad_tiles[t] = grad_c[32 br .. +32, :] @ b[32 bc .. +32, :]^T for every

@@ -264,3 +264,79 @@ def test_layout_plans_shared_and_streams(gpu):
         with torch.cuda.graph(g):
             mod(b)
     assert torch.equal(mod(b).detach(), ref[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [1, 3, 33, 1000])
+def test_gather_tiles_transposed(gpu, dtype, n):
+    v = torch.randn(n, 32, 32, device=gpu).to(dtype)
+    order = torch.randperm(n, device=gpu)
+    got = _runtime.gather_tiles_t(v, order).view(dtype).view(n, 32, 32)
+    assert torch.equal(got, v[order].transpose(1, 2))
+    shifted = torch.cat([v.reshape(-1)[:1], v.reshape(-1)])[1:].view(n, 32, 32)  # not 16-byte aligned
+    assert torch.equal(_runtime.gather_tiles_t(shifted, order).view(dtype).view(n, 32, 32), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [1, 7, 33, 260])
+@pytest.mark.parametrize("token_major_grad", [True, False])
+def test_linear_bias_fused_step(gpu, monkeypatch, dtype, tokens, token_major_grad):
+    """SparseLinear on token-major input: output, gradients of input, tiles and
+    bias against float64, with either layout of the incoming gradient; a
+    forward hook on the weight module takes the unfused path to the same
+    values within one more rounding."""
+    monkeypatch.setattr(_runtime, "TRANSPOSE_MIN_NUMEL", 1)
+    case = cases.uniform_blocks(130, 200, tokens, 20, seed=tokens)
+    vt = cases.make_void_tensor(case, "cpu").to(gpu).to_dtype(dtype)
+    lin = void_amd.SparseLinear(200, 130, vt).to(gpu)
+    g = torch.Generator(device=gpu).manual_seed(tokens)
+    with torch.no_grad():
+        lin.bias.copy_(torch.randn(130, generator=g, device=gpu))
+    x = torch.randn(tokens, 200, generator=g, device=gpu).to(dtype).requires_grad_()
+    gy = torch.randn(tokens, 130, generator=g, device=gpu).to(dtype)
+    if not token_major_grad:
+        gy = gy.t().contiguous().t()
+
+    def step():
+        lin.zero_grad(set_to_none=True)
+        x.grad = None
+        y = lin(x)
+        y.backward(gy)
+        return [y.detach(), x.grad, lin.sparse_weight.values.grad, lin.bias.grad]
+
+    fused = step()
+    assert fused[1].is_contiguous()
+    handle = lin.sparse_weight.register_forward_hook(lambda m, i, o: None)
+    plain = step()
+    handle.remove()
+    W = torch.zeros(160, 224, dtype=torch.float64, device=gpu)
+    for t, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+        W[32 * r:32 * r + 32, 32 * c:32 * c + 32] = vt.values[t].double()
+    gp = torch.zeros(tokens, 160, dtype=torch.float64, device=gpu)
+    xp = torch.zeros(tokens, 224, dtype=torch.float64, device=gpu)
+    gp[:, :130], xp[:, :200] = gy.double(), x.detach().double()
+    gw = gp.t() @ xp
+    gwa = gp.abs().t() @ xp.abs()
+    pick = lambda m: torch.stack([m[32 * r:32 * r + 32, 32 * c:32 * c + 32]
+                                  for r, c in zip(case.block_rows, case.block_cols)])
+    b64 = lin.bias.detach().double()
+    refs = [(xp @ W.t())[:, :130] + b64, (gp @ W)[:, :200], pick(gw), gp[:, :130].sum(0)]
+    mags = [(xp.abs() @ W.abs().t())[:, :130] + b64.abs(), (gp.abs() @ W.abs())[:, :200], pick(gwa),
+            gp[:, :130].abs().sum(0)]
+    rnd = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dtype]
+    for k, (out, alt, ref, mag) in enumerate(zip(fused, plain, refs, mags)):
+        tol = 300 * U * mag + rnd * ref.abs() + 1e-30
+        assert bool(((out.double() - ref).abs() <= tol).all()), k
+        # The unfused sum rounds twice.
+        assert bool(((alt.double() - ref).abs() <= tol + rnd * mag).all()), k
+
+
+def test_linear_create_graph_bias(gpu):
+    """With create_graph the bias gradient stays differentiable in the output gradient."""
+    case = cases.uniform_blocks(64, 64, 5, 3, seed=2)
+    lin = void_amd.SparseLinear(64, 64, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu)
+    x = torch.randn(5, 64, device=gpu)
+    gy = torch.randn(5, 64, device=gpu, requires_grad=True)
+    (gb,) = torch.autograd.grad(lin(x), lin.bias, gy, create_graph=True)
+    (gg,) = torch.autograd.grad(gb.sum(), gy)
+    assert torch.equal(gg, torch.ones_like(gy))

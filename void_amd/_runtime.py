@@ -344,11 +344,25 @@ class DeviceBsr:
             per_tensor_a=int(self.per_tensor), reserved=0)
 
 
+def gather_tiles_t(values: torch.Tensor, order: torch.Tensor) -> torch.Tensor:
+    """uint8 [n, 32, 32 esz]: values[order] with every 32x32 tile transposed
+    (void_gather_tiles_t)."""
+    values = values.contiguous()
+    if values.data_ptr() % 16:
+        values = values.clone()
+    out = torch.empty_like(values)
+    st = _lib.lib().void_gather_tiles_t(values.data_ptr(), order.data_ptr(), values.shape[0], values.element_size(),
+                                        out.data_ptr(), raw_stream(values.device))
+    _lib.check(st, "void_gather_tiles_t")
+    return out.view(torch.uint8)
+
+
 def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torch.Tensor,
                     block_cols: torch.Tensor, shape: Tuple[int, int], tile_size: Tuple[int, int],
-                    device: torch.device, per_tensor: bool, layout=None) -> DeviceBsr:
+                    device: torch.device, per_tensor: bool, layout=None, transpose: bool = False) -> DeviceBsr:
     """Gather the tiles into block-row-major order.  ``layout`` (a BsrLayout
-    of the same block structure) skips the host-side ordering."""
+    of the same block structure) skips the host-side ordering; ``transpose``
+    takes every (float) tile transposed, the indices being the result's."""
     if tuple(tile_size) != (32, 32):
         raise NotImplementedError(f"the gfx950 kernels take 32x32 tiles, got {tile_size}")
     M, K = shape
@@ -356,9 +370,12 @@ def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torc
     n_bc = (K + 31) // 32
     lay = layout if layout is not None else build_bsr_layout(block_rows, block_cols, n_br, n_bc, device)
     v = values.to(device)
-    if v.dtype != torch.uint8:
-        v = v.view(torch.uint8)
-    tiles = v.index_select(0, lay.order).contiguous() if v.shape[0] else v.contiguous()
+    if transpose and v.shape[0]:
+        tiles = gather_tiles_t(v, lay.order)
+    else:
+        if v.dtype != torch.uint8:
+            v = v.view(torch.uint8)
+        tiles = v.index_select(0, lay.order).contiguous() if v.shape[0] else v.contiguous()
     s = scales.to(device=device, dtype=torch.float32)
     if per_tensor:
         s = s.reshape(-1)[:1].contiguous()

@@ -54,8 +54,8 @@ def _layout(block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int
     return hit[0]
 
 
-def _vt(values, block_rows, block_cols, shape, tile_size, n_blocks) -> VOIDTensor:
-    vt = VOIDTensor(values=values, block_rows=block_rows, block_cols=block_cols,
+def _vt(values, block_rows, block_cols, shape, tile_size, n_blocks, cls=VOIDTensor) -> VOIDTensor:
+    vt = cls(values=values, block_rows=block_rows, block_cols=block_cols,
                     morton_codes=torch.empty(0, dtype=torch.int64, device=values.device), shape=tuple(shape),
                     tile_size=tuple(tile_size), nnz_original=0, n_blocks=n_blocks, density=0.0, dtype=values.dtype)
     if n_blocks and values.is_cuda:
@@ -68,29 +68,76 @@ def _vt(values, block_rows, block_cols, shape, tile_size, n_blocks) -> VOIDTenso
     return vt
 
 
+class _TransposedTiles(VOIDTensor):
+    """A^T over A's own tiles: the device copy gathers them transposed."""
+
+    def device_bsr(self, dtype: torch.dtype = torch.float32):
+        values = self.values.detach().to(dtype)
+        none = torch.empty(0, dtype=torch.float32, device=values.device)
+        return _runtime.make_device_bsr(values, none, self.block_rows, self.block_cols, self.shape, self.tile_size,
+                                        values.device, True, layout=self._bsr_layout, transpose=True)
+
+
+def _forward(ctx: Any, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b, bias=None):
+    c = float_spmm(_vt(a_values.detach(), a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks), b,
+                   bias=None if bias is None else bias.detach(), bias_per_row=bias is not None)
+    ctx.save_for_backward(a_values, a_block_rows, a_block_cols, b)
+    ctx.a_shape, ctx.a_tile_size, ctx.a_n_blocks = tuple(a_shape), tuple(a_tile_size), a_n_blocks
+    return c
+
+
+def _backward(ctx: Any, grad_output: torch.Tensor):
+    """(gradient of the tiles, gradient of B) where asked for, and grad_output row-major."""
+    a_values, rows, cols, b = ctx.saved_tensors
+    M, K = ctx.a_shape
+    grad_a = grad_b = None
+    if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[6]):
+        return None, None, grad_output
+    # One row-major copy of a token-major gradient serves every use of it.
+    grad = _runtime.contiguous_2d(grad_output)
+    if ctx.needs_input_grad[6]:
+        at = _vt(a_values.detach(), cols, rows, (K, M), ctx.a_tile_size[::-1], ctx.a_n_blocks, cls=_TransposedTiles)
+        grad_b = float_spmm(at, grad).to(b.dtype)
+        if b.stride(0) == 1 and b.stride(1) >= K > 1:
+            # A column-major B (X.t() of token-major activations) gets a
+            # gradient of its own layout, which autograd then takes as it is.
+            grad_b = _runtime.contiguous_2d(grad_b.t()).t()
+    if ctx.needs_input_grad[0]:
+        grad_a = _runtime.sddmm_tiles(grad, b, rows, cols, (M, K), a_values.dtype,
+                                      layout=_layout(rows, cols, (M, K)) if rows.is_cuda else None)
+    return grad_a, grad_b, grad
+
+
 class VOIDSpMMFunction(Function):
     """C = A @ B with gradients for the tile values and for B (autograd.py:99-216)."""
 
     @staticmethod
     def forward(ctx: Any, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b):
-        c = float_spmm(_vt(a_values.detach(), a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks), b)
-        ctx.save_for_backward(a_values, a_block_rows, a_block_cols, b)
-        ctx.a_shape, ctx.a_tile_size, ctx.a_n_blocks = tuple(a_shape), tuple(a_tile_size), a_n_blocks
-        return c
+        return _forward(ctx, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b)
 
     @staticmethod
     def backward(ctx: Any, grad_output: torch.Tensor):
-        a_values, rows, cols, b = ctx.saved_tensors
-        M, K = ctx.a_shape
-        grad_a = grad_b = None
-        if ctx.needs_input_grad[6]:
-            at = _vt(a_values.detach().permute(0, 2, 1).contiguous(), cols, rows, (K, M),
-                     ctx.a_tile_size[::-1], ctx.a_n_blocks)
-            grad_b = float_spmm(at, _runtime.contiguous_2d(grad_output)).to(b.dtype)
-        if ctx.needs_input_grad[0]:
-            grad_a = _runtime.sddmm_tiles(grad_output, b, rows, cols, (M, K), a_values.dtype,
-                                          layout=_layout(rows, cols, (M, K)) if rows.is_cuda else None)
+        grad_a, grad_b, _ = _backward(ctx, grad_output)
         return grad_a, None, None, None, None, None, grad_b
+
+
+class _BiasSpMMFunction(Function):
+    """C = A @ B + bias[:, None], the bias in the SpMM's epilogue (C is rounded
+    once, after the addition) and its gradient summed along the rows of the
+    row-major gradient that the other two read."""
+
+    @staticmethod
+    def forward(ctx: Any, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b, bias):
+        return _forward(ctx, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b, bias)
+
+    @staticmethod
+    def backward(ctx: Any, grad_output: torch.Tensor):
+        grad_a, grad_b, grad = _backward(ctx, grad_output)
+        grad_bias = None
+        if ctx.needs_input_grad[7]:
+            # Under create_graph the sum stays a function of grad_output.
+            grad_bias = (grad_output if torch.is_grad_enabled() else grad).sum(1)
+        return grad_a, None, None, None, None, None, grad_b, grad_bias
 
 
 class VOIDSpMM(torch.nn.Module):
@@ -122,6 +169,12 @@ class VOIDSpMM(torch.nn.Module):
                           tile_size=self.tile_size, nnz_original=0, n_blocks=self.n_blocks, density=0.0)
 
 
+def _observed(m: torch.nn.Module) -> bool:
+    """Whether calling m runs more than its class's forward (hooks, a replaced forward)."""
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__ or torch.nn.modules.module._has_any_global_hook())
+
+
 class SparseLinear(torch.nn.Module):
     """nn.Linear with a VOID weight: y = x W^T + b (autograd.py:288-352)."""
 
@@ -141,9 +194,16 @@ class SparseLinear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x_flat = x.reshape(-1, self.in_features)
-        y = self.sparse_weight(x_flat.T).T
-        if self.bias is not None:
-            y = y + self.bias
+        w, bias = self.sparse_weight, self.bias
+        if (bias is not None and x.is_cuda and x.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                and bias.dtype == x.dtype and bias.device == x.device and bias.shape == (self.out_features,)
+                and type(w) is VOIDSpMM and w.n_blocks and not _observed(w)):
+            y = _BiasSpMMFunction.apply(w.values, w.block_rows, w.block_cols, w.shape, w.tile_size, w.n_blocks,
+                                        x_flat.T, bias).T
+        else:
+            y = w(x_flat.T).T
+            if bias is not None:
+                y = y + bias
         return y.reshape(x.shape[:-1] + (self.out_features,))
 
     def extra_repr(self) -> str:
