@@ -103,3 +103,92 @@ def test_fp8_nan_codes_past_n(gpu, N):
     bd = codes.double()
     ref, bound = dense[:, :200] @ bd, mag[:, :200] @ bd.abs()
     assert bool(((out - ref).abs() <= 2.0 ** -13 * bound + 1e-30).all())
+
+
+def _layouts(bq, gpu):
+    """B as row- and column-major views: aligned, padded, and shifted by a byte."""
+    K, N = bq.shape
+    src = torch.from_numpy(bq)
+    for col in (False, True):
+        rows, cols = (N, K) if col else (K, N)
+        for pitch, shift in ((cols, 0), ((cols + 31) // 16 * 16, 0), (cols + 1, 1)):
+            flat = torch.full((rows * pitch + shift,), 0x7f, dtype=torch.int8)  # NaN as E4M3
+            v = flat[shift:].view(rows, pitch)[:, :cols]
+            v.copy_(src.t() if col else src)
+            v = flat.to(gpu)[shift:].view(rows, pitch)[:, :cols]
+            yield v.t() if col else v
+
+
+@pytest.mark.parametrize("N", [1, 2, 15, 16, 17, 31, 32, 33, 48, 63, 64])
+@pytest.mark.parametrize("K", [200, 256, 1])
+@pytest.mark.parametrize("chunk", [None, 3])
+def test_narrow_int8(gpu, N, K, chunk):
+    """The narrow kernel: int32 and row-mean bit-exact and per-block within
+    1e-5 on every layout, unsplit rows (one longer than 24 tiles where K
+    allows) and split ones, empty rows and a misaligned output included."""
+    n_bc = -(-K // 32)
+    case = cases.uniform_blocks(300, K, N, min(6 * n_bc, 10 * n_bc - 1), seed=N)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu"))
+    A = oracle.Bsr(q.values.numpy(), q.scales.numpy(), case.block_rows, case.block_cols, (300, K))
+    bq, bs = oracle.quantize_i8_tensor(case.b)
+    acc = oracle.i8_acc(A, bq)
+    mean = oracle.row_mean(A, acc, bs)
+    qd = q.to(gpu)
+    wide = torch.full((300, N + 3), -7.0, device=gpu)
+    for b in _layouts(bq, gpu):
+        kw = dict(chunk_tiles=chunk)
+        got = void_amd.void_spmm_int8(qd, b, epilogue="raw_i32", **kw)
+        assert np.array_equal(got.cpu().numpy(), acc)
+        got = void_amd.void_spmm_int8(qd, b, b_scale=float(bs), out=wide[:, 1:N + 1], **kw).cpu().numpy()
+        assert np.array_equal(np.ascontiguousarray(got).view(np.int32), mean.view(np.int32))
+        assert bool((wide[:, 0] == -7).all()) and bool((wide[:, N + 1:] == -7).all())
+        first = void_amd.void_spmm_int8(qd, b, b_scale=float(bs), epilogue="per_block", **kw)
+        again = void_amd.void_spmm_int8(qd, b, b_scale=float(bs), epilogue="per_block", **kw)
+        assert torch.equal(first, again)
+        t = q.values.double() * q.scales.double()[:, None, None]
+        dense = torch.zeros(320, 32 * n_bc, dtype=torch.float64)
+        for i, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+            dense[32 * r:32 * r + 32, 32 * c:32 * c + 32] = t[i]
+        dense = dense[:300, :K]
+        bd = torch.from_numpy(bq).double() * float(bs)
+        assert bool(((first.double().cpu() - dense @ bd).abs() <= 1e-5 * (dense.abs() @ bd.abs()) + 1e-30).all())
+
+
+@pytest.mark.parametrize("N", [1, 17, 32, 64])
+@pytest.mark.parametrize("chunk", [None, 5])
+def test_narrow_long_rows_and_activation(gpu, N, chunk):
+    """Rows of up to 64 tiles, per-column scales, bias and GELU into bf16 and fp16."""
+    case = cases.uniform_blocks(160, 4096, N, 300, seed=N)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu"))
+    bq, bs = oracle.quantize_i8_columns(case.b)
+    bias = torch.linspace(-1, 1, N)
+    dense = torch.zeros(160, 4096, dtype=torch.float64)
+    t = q.values.double() * q.scales.double()[:, None, None]
+    for i, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+        dense[32 * r:32 * r + 32, 32 * c:32 * c + 32] = t[i]
+    x = (dense @ (torch.from_numpy(bq).double() * torch.from_numpy(bs).double()) + bias.double()) * 0.02
+    small = torch.from_numpy(bs * np.float32(0.02))
+    ref = x * torch.sigmoid(2 * 0.7978845608 * (x + 0.044715 * x ** 3))
+    for dtype, rnd in ((torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)):
+        for b in _layouts(bq, gpu):
+            out = void_amd.void_spmm_int8(q.to(gpu), b, b_scale=small.to(gpu), bias=0.02 * bias.to(gpu),
+                                          epilogue="per_block", out_dtype=dtype, activation="gelu", chunk_tiles=chunk)
+            assert bool(((out.double().cpu() - ref).abs() <= rnd * ref.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("N", [1, 16, 33, 64])
+def test_narrow_fp8(gpu, N):
+    """E4M3 on every layout with NaN codes in the bytes around B."""
+    case = cases.uniform_blocks(96, 200, N, 14, seed=N)
+    f8 = void_amd.void_tensor_to_fp8(cases.make_void_tensor(case, "cpu"))
+    codes = torch.from_numpy(case.b).clamp(-400, 400).to(torch.float8_e4m3fn)
+    dense = torch.zeros(96, 224, dtype=torch.float64)
+    t = f8.values_fp8.double() * f8.scaling_info.scale.double()[:, None, None]
+    for i, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+        dense[32 * r:32 * r + 32, 32 * c:32 * c + 32] = t[i]
+    dense = dense[:, :200]
+    ref, bound = dense @ codes.double(), dense.abs() @ codes.double().abs()
+    for b in _layouts(codes.view(torch.int8).numpy(), gpu):
+        raw = b.view(torch.float8_e4m3fn) if b.stride(1) == 1 else b.t().view(torch.float8_e4m3fn).t()
+        out = void_amd.void_spmm_fp8(f8.to(gpu), raw, output_dtype=torch.float32).double().cpu()
+        assert bool(((out - ref).abs() <= 2.0 ** -13 * bound + 1e-30).all())

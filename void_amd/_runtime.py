@@ -416,9 +416,12 @@ def dense_operand(b: torch.Tensor) -> Tuple[torch.Tensor, int, bool]:
 def row_major_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
     """Row-major K x N copy of a column-major 8-bit B (N columns of K bytes,
     ld apart): void_transpose_b8 where the shape allows, torch's copy
-    otherwise."""
+    otherwise (into rows of an aligned pitch, which the ring reads for any N)."""
     K, N = b.shape
-    out = torch.empty(K, N, dtype=b.dtype, device=b.device)
+    if N % 16:
+        out = torch.empty(K, tuning.aligned_pitch(N), dtype=b.dtype, device=b.device)[:, :N]
+    else:
+        out = torch.empty(K, N, dtype=b.dtype, device=b.device)
     if K % 16 == 0 and N % 16 == 0 and ld % 16 == 0 and b.data_ptr() % 16 == 0:
         st = _lib.lib().void_transpose_b8(b.data_ptr(), ld, N, K, out.data_ptr(), N,
                                           raw_stream(b.device))
@@ -471,19 +474,21 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
     lib = _lib.lib()
     N = b.shape[1]
     b_t, ldb, col_major = dense_operand(b)
-    if col_major and kind in ("int8", "fp8") and tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K):
-        b_t, ldb, col_major = row_major_copy_b8(b_t, ldb), N, False  # for the LDS-DMA ring
+    plan = dbsr.plan(chunk)
+    short = chunk <= tuning.FP32_B_MAX_CHUNK  # items the narrow and column-group kernels take
+    panels8 = kind in ("int8", "fp8") and not (short and tuning.narrow(N, plan.n_split_tiles))
+    if col_major and panels8 and tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K):
+        b_t, col_major = row_major_copy_b8(b_t, ldb), False  # for the LDS-DMA ring
+        ldb = max(b_t.stride(0), N)
     target = out
     so0, so1 = out.stride()
     if so1 != 1 or so0 < N:
         target = torch.empty(out.shape, dtype=out.dtype, device=out.device)
-    if (kind in ("int8", "fp8") and N and not col_major and (ldb % 16 or b_t.data_ptr() % 16)
-            and chunk <= tuning.FP32_B_MAX_CHUNK):
+    if panels8 and short and N and not col_major and (ldb % 16 or b_t.data_ptr() % 16):
         dword = ((N | ldb | b_t.data_ptr() | target.stride(0)) % 4 == 0) and target.data_ptr() % 16 == 0
         if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword):
             b_t = aligned_copy_b8(b_t, ldb)
             ldb = b_t.stride(0)
-    plan = dbsr.plan(chunk)
     stream = raw_stream(out.device)
     ws, ws_bytes = plan.workspace(N, out.device, stream)
     # Fields in the struct's order.

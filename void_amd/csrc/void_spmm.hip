@@ -99,6 +99,7 @@ struct Params {
   int32_t item_piles;   // XCDs among which one panel group's items are dealt (see wg_map)
   int32_t xcd_exact;    // grid laid out per XCD (see wg_map)
   int32_t bias_per_row;  // float kernel: bias indexed by output row
+  int32_t out_dtype;     // narrow kernel (the others take it as a template argument)
   int32_t pair_snake;    // exact layout: second half of an XCD's share reversed (see wg_map)
 };
 
@@ -1974,6 +1975,303 @@ int launch_cg(const Params& p, int grid, hipStream_t stream) {
 }
 
 
+// ---------------------------------------------------------------------------
+// Narrow kernel: an 8-bit B of at most 64 columns (decode, small batches), any
+// layout and alignment.
+//
+// With so few columns the tiles are the traffic (14336 tiles, N = 16: 14.7 MB
+// of A against 64 KB of B and 0.5 MB of C), and a 128-column panel leaves three
+// of the column-group kernel's four waves without a column while one wave
+// runs all of a row's tiles.  Here up to 8 waves of a workgroup take an item's
+// tiles round-robin, each tile one 16-byte A load per lane (1 KB, whole
+// lines), with kNarrowBatch tiles' loads of a wave in flight, so that a row of
+// 32 tiles is requested at once; the partial blocks meet in LDS, in a fixed
+// order.  B goes from memory to the MFMA operand directly (column-major: 16
+// bytes of a column per lane) or through 1 KB of the wave's LDS and a
+// transposed read (row-major); rows or columns at any byte alignment take
+// unaligned 16-byte loads, byte loads where those would pass B's end.
+// The block columns of the first 24 tiles come with the item's record, so
+// most B addresses wait for one round trip only.
+// Measured (us, graph replays; panel kernels before, here): 14336 x 4096, 14336
+// tiles, N = 16 column-major 14.2 -> 4.7 (3.1 TB/s of tiles), N = 64 11.3 -> 7.4;
+// 4096 x 4096, 1638 tiles, N = 16 6.8 -> 3.1, N = 17 25.1 -> 3.6; Zipf rows of up to
+// 256 tiles, N = 32 12.4 -> 10.4.  On split rows two column groups lose (N = 64:
+// 12.6 -> 16.4), so those keep the panel kernels above 32 columns.
+constexpr int kNarrowWaves = 8;
+constexpr int kNarrowBatch = 4;
+constexpr int kNarrowN = 64;
+enum NarrowB { kNbRow16 = 0, kNbCol16 = 1, kNbRowAny = 2, kNbColAny = 3 };
+
+// 16 bytes at s, zeros for the bytes at or past `limit` bytes.
+__device__ __forceinline__ v4i load_bytes16(const uint8_t* s, int limit) {
+  v4i v;
+  if (limit >= 16) {
+    __builtin_memcpy(&v, s, 16);
+  } else {
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (e < limit) w[e >> 2] |= (uint32_t)s[e] << (8 * (e & 3));
+    v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+  }
+  return v;
+}
+
+template <int ELT, int EPI, int BMODE, int NG>
+__global__ __launch_bounds__(64 * kNarrowWaves) void spmm_narrow_kernel(const void_work_item* __restrict__ items,
+                                                                        Params p) {
+  using A = Accum1<ELT, EPI>;
+  constexpr bool kInt = A::kInt;
+  constexpr bool kScales = EPI == VOID_EPI_PER_BLOCK;
+  constexpr bool kCol = BMODE == kNbCol16 || BMODE == kNbColAny;
+  constexpr int kBlock = kTile * kTile;
+  // Per wave: its B slabs (row-major B) during the tile loop, then its partial
+  // block(s), register r of lane l at r * 64 + l.
+  __shared__ __attribute__((aligned(16))) int lds[kNarrowWaves][NG * kBlock];
+  static_assert(kNarrowBatch * 1024 <= kBlock * 4, "B slabs fit the wave's area");
+  __shared__ int s_last;
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int j = lane & 31, g = lane >> 5;
+  const void_work_item* itp = items + blockIdx.x;
+  const int rec_col = itp->cols[min(lane, kInline - 1)];
+  const int row = itp->row, begin = itp->begin, end = itp->end, split_tile = itp->tile;
+  const int nt = end - begin;
+
+  // Lane i: block column and scale of tile min(i, nt - 1).
+  const int ti = begin + min(lane, max(nt - 1, 0));
+  int colw = rec_col;
+  if (nt > kInline) {
+    const int c = p.col_idx[ti];
+    colw = lane < kInline ? rec_col : c;
+  }
+  float scw = 0.f;
+  if constexpr (kScales) {
+    if (nt > 0) scw = p.a_scale[p.per_tensor_a ? 0 : ti];
+  }
+
+  const Rsrc ra = make_rsrc(p.tiles), rbm = make_rsrc(p.b);
+  const int voff_a = j * kTile + 16 * g;
+  const int brow = lane >> 1, bhalf = 16 * (lane & 1);  // row-major: this lane's 16 bytes of a slab
+  auto load_a = [&](int idx) -> v4i {
+    const bool live = idx < nt;
+    return __builtin_amdgcn_raw_buffer_load_b128(ra, live ? voff_a : kOutOfRange,
+                                                 (begin + (live ? idx : 0)) * (kTile * kTile), 0);
+  };
+  auto load_b = [&](int idx, int kb, int q) -> v4i {
+    const bool live = idx < nt;
+    if constexpr (BMODE == kNbRow16) {
+      // The last 16-byte chunk below N stays inside the row's pitch.
+      const bool in = live && bhalf + 32 * q < p.N && brow < p.K - kb * kTile;
+      return __builtin_amdgcn_raw_buffer_load_b128(rbm, in ? brow * (int)p.ldb + bhalf + 32 * q : kOutOfRange,
+                                                   kb * kTile * (int)p.ldb, 0);
+    } else if constexpr (BMODE == kNbCol16) {
+      const int c = 32 * q + j;
+      const bool in = live && c < p.N;
+      return __builtin_amdgcn_raw_buffer_load_b128(rbm, in ? c * (int)p.ldb + 16 * g : kOutOfRange, kb * kTile, 0);
+    } else if constexpr (BMODE == kNbRowAny) {
+      const int k = kb * kTile + brow, c = bhalf + 32 * q;
+      if (!live || c >= p.N || k >= p.K) return v4i{0, 0, 0, 0};
+      // Bytes past N belong to the next row; the last row ends at N.
+      const int64_t left = (int64_t)(p.K - 1 - k) * p.ldb + (p.N - c);
+      return load_bytes16(p.b + (int64_t)k * p.ldb + c, (int)min(left, (int64_t)16));
+    } else {
+      const int k = kb * kTile + 16 * g, c = 32 * q + j;
+      if (!live || c >= p.N || k >= p.K) return v4i{0, 0, 0, 0};
+      return load_bytes16(p.b + (int64_t)c * p.ldb + k, min(p.K - k, 16));
+    }
+  };
+
+  typename A::Reg acc[NG];
+#pragma unroll
+  for (int q = 0; q < NG; ++q) acc[q] = typename A::Reg{};
+  uint8_t* slots = reinterpret_cast<uint8_t*>(&lds[wave][0]);
+  // Short rows use fewer waves, a full batch each: longer chains of fused
+  // multiply-adds, so fewer roundings, and the same loads in flight.
+  const int nw = min(kNarrowWaves, (nt + kNarrowBatch - 1) / kNarrowBatch);
+  for (int base = wave < nw ? wave : nt; base < nt; base += nw * kNarrowBatch) {
+    v4i a[kNarrowBatch], b[kNarrowBatch][NG];
+#pragma unroll
+    for (int u = 0; u < kNarrowBatch; ++u) a[u] = load_a(base + u * nw);
+#pragma unroll
+    for (int u = 0; u < kNarrowBatch; ++u) {
+      const int idx = base + u * nw;
+      const int kb = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_readlane(colw, min(idx, nt - 1)));
+#pragma unroll
+      for (int q = 0; q < NG; ++q) b[u][q] = load_b(idx, kb, q);
+    }
+#pragma unroll
+    for (int u = 0; u < kNarrowBatch; ++u) {
+      const int idx = base + u * nw;
+      if (idx >= nt) break;
+      const float sc = kScales ? bcast(scw, idx) : 0.f;
+#pragma unroll
+      for (int q = 0; q < NG; ++q) {
+        Frag1 f;
+        f.a = a[u];
+        if constexpr (kCol) {
+          f.b = b[u][q];
+        } else {
+          // 32 rows of 32 bytes; the transposed read of read_tr on that pitch.
+          uint8_t* slot = slots + (u & 3) * 1024;
+          *reinterpret_cast<v4i*>(slot + lane * 16) = b[u][q];
+          const int i = j & 15;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint8_t* src = slot + (16 * g + 8 * h + (i >> 1)) * 32 + 16 * (j >> 4) + 8 * (i & 1);
+            const v2i v = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (__attribute__((address_space(3))) v2i*)(const_cast<uint8_t*>(src)));
+            f.b[2 * h] = v[0];
+            f.b[2 * h + 1] = v[1];
+          }
+        }
+        A::step(acc[q], f, sc);
+      }
+    }
+  }
+
+  // Epilogue inputs of this lane's columns.
+  float sb[NG], bias[NG];
+#pragma unroll
+  for (int q = 0; q < NG; ++q) {
+    const int cc = min(32 * q + j, p.N - 1);
+    sb[q] = p.b_scale_vec ? p.b_scale_vec[cc * p.b_scale_stride] : p.b_scale;
+    bias[q] = p.bias ? p.bias[cc] : 0.f;
+  }
+  int rb = 0, re = 0;
+  float row_scale = 0.f;
+  if constexpr (EPI == VOID_EPI_ROW_MEAN) {
+    rb = split_tile < 0 ? begin : p.row_ptr[row];
+    re = split_tile < 0 ? end : p.row_ptr[row + 1];
+    if (re > rb) row_scale = p.a_scale[p.per_tensor_a ? 0 : rb + min(lane, re - rb - 1)];
+  }
+
+  // Wave w finishes registers 2 w and 2 w + 1 of every block: row
+  // 8 (r / 4) + 4 g + r % 4, column j of group q.
+#pragma unroll
+  for (int q = 0; q < NG; ++q)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      lds[wave][q * kBlock + r * 64 + lane] = kInt ? (int)acc[q][r] : __float_as_int((float)acc[q][r]);
+  __syncthreads();
+  using Sum = typename std::conditional<kInt, int, float>::type;
+  Sum sum[NG][2];
+  auto value = [](int w) -> Sum {
+    if constexpr (kInt) return w;
+    else return __int_as_float(w);
+  };
+#pragma unroll
+  for (int q = 0; q < NG; ++q)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      // Pairwise: three roundings deep, as exact as the panel kernels' sums.
+      Sum x[kNarrowWaves];
+#pragma unroll
+      for (int w = 0; w < kNarrowWaves; ++w) x[w] = value(lds[w][q * kBlock + (2 * wave + e) * 64 + lane]);
+#pragma unroll
+      for (int n = kNarrowWaves / 2; n > 0; n >>= 1)
+#pragma unroll
+        for (int w = 0; w < n; ++w) x[w] += x[w + n];
+      sum[q][e] = x[0];
+    }
+
+  if (split_tile >= 0) {
+    // Split row: the publish / count / reduce-in-chunk-order protocol of the
+    // other kernels (see publish_wait); group q takes the place of wave q's
+    // block of panel 0.
+    const int nchunks = itp->nchunks, slot = itp->slot, chunk = itp->chunk;
+    int* part = static_cast<int*>(p.partials);
+    auto word = [&](int c, int q, int e) -> int* {
+      return part + ((size_t)(slot + c) * kWaves + q) * kBlock + (2 * wave + e) * 64 + lane;
+    };
+#pragma unroll
+    for (int q = 0; q < NG; ++q)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        __hip_atomic_store(word(chunk, q, e), kInt ? (int)sum[q][e] : __float_as_int((float)sum[q][e]),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    publish_wait();
+    __syncthreads();
+    unsigned* ctr = p.counters + split_tile;
+    if (tid == 0) {
+      const unsigned old = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      s_last = (old == (unsigned)(nchunks - 1));
+    }
+    __syncthreads();
+    if (!s_last) return;
+    if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    compiler_order();
+#pragma unroll
+    for (int q = 0; q < NG; ++q)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        Sum x = 0;
+        for (int c = 0; c < nchunks; ++c)
+          x += value(__hip_atomic_load(word(c, q, e), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        sum[q][e] = x;
+      }
+  }
+
+#pragma unroll
+  for (int q = 0; q < NG; ++q) {
+    float mul = 1.f;
+    if constexpr (EPI == VOID_EPI_ROW_MEAN) {
+      // int_quant.py:519-526, in the order of the other kernels' epilogues.
+      float S = 0.f;
+      for (int t0 = rb; t0 < re; t0 += 64) {
+        const int n = min(64, re - t0);
+        const float mine =
+            t0 == rb ? row_scale : (p.per_tensor_a ? p.a_scale[0] : p.a_scale[t0 + min(lane, n - 1)]);
+        for (int k = 0; k < n; ++k) S = __fadd_rn(S, __fmul_rn(bcast(mine, k), sb[q]));
+      }
+      mul = (re > rb) ? __fdiv_rn(S, (float)(re - rb)) : 0.f;
+    } else if constexpr (EPI == VOID_EPI_PER_BLOCK) {
+      mul = sb[q];
+    }
+    const int col = 32 * q + j;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int r = 2 * wave + e;
+      const int grow = row * kTile + 8 * (r >> 2) + 4 * g + (r & 3);
+      if (grow >= p.M || col >= p.N) continue;
+      const int64_t off = (int64_t)grow * p.ldc + col;
+      if constexpr (EPI == VOID_EPI_RAW_I32) {
+        static_cast<int*>(p.c)[off] = sum[q][e];
+      } else {
+        float x = __fmul_rn((float)sum[q][e], mul);
+        if (p.bias) x = __fadd_rn(x, bias[q]);
+        x = activate(x, p.activation);
+        if (p.out_dtype == VOID_DT_F32) static_cast<float*>(p.c)[off] = x;
+        else if (p.out_dtype == VOID_DT_BF16) static_cast<uint16_t*>(p.c)[off] = (uint16_t)f32_to_bf16_bits(x);
+        else static_cast<uint16_t*>(p.c)[off] = (uint16_t)f32_to_f16_bits(x);
+      }
+    }
+  }
+}
+
+template <int ELT, int EPI>
+int launch_narrow(const Params& p, hipStream_t stream, int bmode) {
+  auto go = [&](auto mode_c, auto ng_c) -> int {
+    hipLaunchKernelGGL((spmm_narrow_kernel<ELT, EPI, decltype(mode_c)::value, decltype(ng_c)::value>),
+                       dim3(p.n_items), dim3(64 * kNarrowWaves), 0, stream, p.items, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(VOID_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
+    return VOID_OK;
+  };
+  auto pick = [&](auto mode_c) -> int {
+    if (p.N <= kTile) return go(mode_c, std::integral_constant<int, 1>{});
+    return go(mode_c, std::integral_constant<int, 2>{});
+  };
+  switch (bmode) {
+    case kNbRow16: return pick(std::integral_constant<int, kNbRow16>{});
+    case kNbCol16: return pick(std::integral_constant<int, kNbCol16>{});
+    case kNbRowAny: return pick(std::integral_constant<int, kNbRowAny>{});
+    default: return pick(std::integral_constant<int, kNbColAny>{});
+  }
+}
+
 // B layouts: column-major (direct 16-byte loads), row-major through LDS
 // (16-byte aligned rows), row-major with in-register transposes (4-byte
 // aligned rows), or bytewise (anything else).
@@ -2299,6 +2597,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     }
   }
   p.bias_per_row = d->bias_per_row;
+  p.out_dtype = d->out_dtype;
   p.items = items;
   p.trace = g_trace;
   if (n_split_tiles > 0 && fixed) {
@@ -2454,6 +2753,19 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   const bool offsets_ok = (int64_t)a->n_blocks * kTile * kTile < kLim && b_span < kLim &&
                           (int64_t)a->M * d->ldc * esz < kLim;
 
+  // Few columns: the narrow kernel, for every B layout (VOID_AMD_KERNEL=narrow
+  // names it, any other value keeps the panel kernels).
+  if (d->N <= (n_split_tiles > 0 ? kTile : kNarrowN) && plan->chunk_tiles <= kCgMaxTiles && offsets_ok && (!force || strcmp(force, "narrow") == 0)) {
+    if (d->out_dtype < VOID_DT_F32 || d->out_dtype > VOID_DT_I32)
+      return fail(VOID_ERR_UNSUPPORTED, "out_dtype %d not supported with this epilogue", d->out_dtype);
+    const int bmode = d->b_col_major ? (b16 ? kNbCol16 : kNbColAny) : (b16 ? kNbRow16 : kNbRowAny);
+    if (elt == kEltFp8) return launch_narrow<kEltFp8, VOID_EPI_PER_BLOCK>(p, stream, bmode);
+    switch (epilogue) {
+      case VOID_EPI_RAW_I32: return launch_narrow<kEltI8, VOID_EPI_RAW_I32>(p, stream, bmode);
+      case VOID_EPI_ROW_MEAN: return launch_narrow<kEltI8, VOID_EPI_ROW_MEAN>(p, stream, bmode);
+      default: return launch_narrow<kEltI8, VOID_EPI_PER_BLOCK>(p, stream, bmode);
+    }
+  }
   const bool cg_ok = b16 && plan->chunk_tiles <= kCgMaxTiles && offsets_ok && !force_bsr;
   if (cg_ok) {
     const bool bcol = d->b_col_major;
