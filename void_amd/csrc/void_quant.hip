@@ -148,7 +148,8 @@ int check_args(const float* tiles, int32_t n_tiles, const void* q, const float* 
 
 // Per-tensor symmetric INT8 quantisation of a float B (int_quant.py:178-214,
 // 308-325 with qmin = -128, qmax = 127): scale = max(max |b| / 128, 1e-8),
-// q = clamp(rint(b / scale), -128, 127) with IEEE division.  Two launches:
+// q = clamp(rint(b / scale), -128, 127) with IEEE division.  Two launches (one
+// for a small B):
 // the first writes one partial max |b| per workgroup (as bits: for the
 // non-negative floats the integer order is the float order, and a NaN's
 // bits exceed infinity's), the second reduces the partials in every
@@ -162,94 +163,178 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return v;
 }
 
+constexpr int kQbBatch = 4;       // 16-byte loads a thread keeps in flight
+constexpr int kQbSmallThreads = 1024;
+constexpr int64_t kQbSmall = 1 << 16;  // largest n of the one-launch kernel
+
+__device__ __forceinline__ uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+// max |b| (as bits) over the float4s i0, i0 + stride, ... below n4, BATCH loads
+// at a time.
+template <int BATCH>
+__device__ __forceinline__ uint32_t amax_strided(const v4f* b, int64_t i0, int64_t stride, int64_t n4) {
+  uint32_t m = 0;
+  for (int64_t i = i0; i < n4; i += BATCH * stride) {
+    v4f x[BATCH];
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) x[u] = b[i + u * stride < n4 ? i + u * stride : i];
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) m = max(m, abs_bits(x[u][k]));
+  }
+  return m;
+}
+
+template <int THREADS>
 __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* red) {
   v = wave_max_u32(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   uint32_t m = red[0];
 #pragma unroll
-  for (int w = 1; w < kQbThreads / 64; ++w) m = max(m, red[w]);
+  for (int w = 1; w < THREADS / 64; ++w) m = max(m, red[w]);
   return m;
+}
+
+// torch.clamp(scale, min=1e-8) keeps a NaN scale (fmaxf would drop it).
+__device__ __forceinline__ float b_scale_of(uint32_t amax_bits) {
+  const float s = __uint_as_float(amax_bits) / 128.0f;
+  return s != s ? s : fmaxf(s, 1e-8f);
+}
+
+__device__ __forceinline__ uint32_t b_code(float x, float scale) {
+  const float r = __builtin_rintf(__fdiv_rn(x, scale));
+  return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(r, -128.0f), 127.0f);
+}
+
+// Code words of b: FLAT, word i holds the codes of b[4 i .. 4 i + 3] (n4 whole
+// words; the last n % 4 codes go out byte by byte in `tail`).  Rows, word i
+// holds columns 4 c .. + 3 of row k, i = k (ldq / 4) + c, zeros past column N.
+struct BWords {
+  const float* b;
+  int8_t* q;
+  int64_t n;
+  int32_t N;
+  uint32_t per_row;
+  uint64_t total;  // below 2^32 for rows
+};
+
+template <bool FLAT>
+__device__ __forceinline__ v4f load_word(const BWords& w, uint64_t i, int32_t& valid) {
+  v4f x = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (FLAT) {
+    valid = 4;
+    x = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(w.b) + i);
+  } else {
+    const uint32_t k = (uint32_t)i / w.per_row, c = 4 * ((uint32_t)i - k * w.per_row);
+    const float* src = w.b + (int64_t)k * w.N + c;
+    valid = w.N - (int32_t)c;
+    if (valid >= 4) {
+      __builtin_memcpy(&x, src, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (e < valid) x[e] = src[e];
+    }
+  }
+  return x;
+}
+
+__device__ __forceinline__ void store_word(const BWords& w, uint64_t i, v4f x, int32_t valid, float scale) {
+  uint32_t c = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c |= (e < valid ? b_code(x[e], scale) : 0u) << (8 * e);
+  reinterpret_cast<uint32_t*>(w.q)[i] = c;
+}
+
+template <bool FLAT>
+__device__ __forceinline__ void tail(const BWords& w, float scale, int64_t i0, int64_t stride) {
+  if constexpr (FLAT)
+    for (int64_t i = 4 * (w.n / 4) + i0; i < w.n; i += stride) w.q[i] = (int8_t)b_code(w.b[i], scale);
 }
 
 __global__ __launch_bounds__(kQbThreads) void b_amax_kernel(const float* __restrict__ b, int64_t n,
                                                           uint32_t* __restrict__ partials) {
   __shared__ uint32_t red[kQbThreads / 64];
-  typedef float v4f __attribute__((ext_vector_type(4)));
-  uint32_t m = 0;
-  const int64_t n4 = n / 4;
-  for (int64_t i = (int64_t)blockIdx.x * kQbThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kQbThreads) {
-    const v4f x = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(b) + i);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) m = max(m, __float_as_uint(x[k]) & 0x7fffffffu);
-  }
-  for (int64_t i = 4 * n4 + (int64_t)blockIdx.x * kQbThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kQbThreads)
-    m = max(m, __float_as_uint(b[i]) & 0x7fffffffu);
-  m = block_max_u32(m, red);
+  const int64_t i0 = (int64_t)blockIdx.x * kQbThreads + threadIdx.x, stride = (int64_t)gridDim.x * kQbThreads;
+  uint32_t m = amax_strided<kQbBatch>(reinterpret_cast<const v4f*>(b), i0, stride, n / 4);
+  for (int64_t i = n / 4 * 4 + i0; i < n; i += stride) m = max(m, abs_bits(b[i]));
+  m = block_max_u32<kQbThreads>(m, red);
   if (threadIdx.x == 0) partials[blockIdx.x] = m;
 }
 
-__global__ __launch_bounds__(kQbThreads) void b_quant_kernel(const float* __restrict__ b, int64_t n,
-                                                           const uint32_t* __restrict__ partials, int32_t n_partials,
-                                                           int8_t* __restrict__ q, float* __restrict__ scale_out) {
+// The second launch: each workgroup reduces the partials and quantises its
+// words; the first kQbBatch loads of a thread are issued before the reduction,
+// whose round trip they then hide under.
+template <bool FLAT>
+__global__ __launch_bounds__(kQbThreads) void b_quant_kernel(BWords w, const uint32_t* __restrict__ partials,
+                                                           int32_t n_partials, float* __restrict__ scale_out) {
   __shared__ uint32_t red[kQbThreads / 64];
-  typedef float v4f __attribute__((ext_vector_type(4)));
+  const uint64_t i0 = blockIdx.x * kQbThreads + threadIdx.x, stride = gridDim.x * kQbThreads;
+  v4f x[kQbBatch];
+  int32_t valid[kQbBatch];
+#pragma unroll
+  for (int u = 0; u < kQbBatch; ++u) {
+    const uint64_t i = i0 + u * stride;
+    if (i < w.total) x[u] = load_word<FLAT>(w, i, valid[u]);
+  }
   uint32_t m = 0;
   for (int i = threadIdx.x; i < n_partials; i += kQbThreads) m = max(m, partials[i]);
-  m = block_max_u32(m, red);
-  // torch.clamp(scale, min=1e-8) keeps a NaN scale (fmaxf would drop it).
-  const float amax = __uint_as_float(m) / 128.0f;
-  const float scale = amax != amax ? amax : fmaxf(amax, 1e-8f);
+  const float scale = b_scale_of(block_max_u32<kQbThreads>(m, red));
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = scale;
-  auto code = [&](float x) -> uint32_t {
-    const float r = __builtin_rintf(__fdiv_rn(x, scale));
-    return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(r, -128.0f), 127.0f);
-  };
-  const int64_t n4 = n / 4;
-  for (int64_t i = (int64_t)blockIdx.x * kQbThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kQbThreads) {
-    const v4f x = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(b) + i);
-    const uint32_t w = code(x[0]) | (code(x[1]) << 8) | (code(x[2]) << 16) | (code(x[3]) << 24);
-    reinterpret_cast<uint32_t*>(q)[i] = w;
+#pragma unroll
+  for (int u = 0; u < kQbBatch; ++u) {
+    const uint64_t i = i0 + u * stride;
+    if (i < w.total) store_word(w, i, x[u], valid[u], scale);
   }
-  for (int64_t i = 4 * n4 + (int64_t)blockIdx.x * kQbThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kQbThreads)
-    q[i] = (int8_t)code(b[i]);
+  for (uint64_t i = i0 + kQbBatch * stride; i < w.total; i += stride) {
+    int32_t v;
+    const v4f y = load_word<FLAT>(w, i, v);
+    store_word(w, i, y, v, scale);
+  }
+  tail<FLAT>(w, scale, i0, stride);
 }
 
-// b_quant_kernel with the codes in rows of pitch ldq: a thread takes four
-// columns of one row (one 16-byte load, any alignment of b's rows, and one
-// 4-byte store), a group past column N writes zeros.  Bound by b's bytes, as
-// the flat kernel is (3001 x 730: 5.2 us against 5.6 us flat); the padded
-// rows let the SpMM run its LDS-DMA ring on any N.
-__global__ __launch_bounds__(kQbThreads) void b_quant_rows_kernel(const float* __restrict__ b, int32_t K, int32_t N,
-                                                                const uint32_t* __restrict__ partials,
-                                                                int32_t n_partials, int8_t* __restrict__ q,
-                                                                int32_t ldq, float* __restrict__ scale_out) {
-  __shared__ uint32_t red[kQbThreads / 64];
-  uint32_t m = 0;
-  for (int i = threadIdx.x; i < n_partials; i += kQbThreads) m = max(m, partials[i]);
-  m = block_max_u32(m, red);
-  // torch.clamp(scale, min=1e-8) keeps a NaN scale (fmaxf would drop it).
-  const float amax = __uint_as_float(m) / 128.0f;
-  const float scale = amax != amax ? amax : fmaxf(amax, 1e-8f);
+// Small B (n up to kQbSmall floats, 256 KB): one launch, in which every
+// workgroup takes the maximum of the whole of B (from L2, 16 loads per thread
+// at most) and quantises its share.
+template <bool FLAT>
+__global__ __launch_bounds__(kQbSmallThreads) void b_small_kernel(BWords w, float* __restrict__ scale_out) {
+  __shared__ uint32_t red[kQbSmallThreads / 64];
+  uint32_t m = amax_strided<8>(reinterpret_cast<const v4f*>(w.b), threadIdx.x, kQbSmallThreads, w.n / 4);
+  for (int64_t i = w.n / 4 * 4 + threadIdx.x; i < w.n; i += kQbSmallThreads) m = max(m, abs_bits(w.b[i]));
+  const float scale = b_scale_of(block_max_u32<kQbSmallThreads>(m, red));
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = scale;
-  auto code = [&](float x) -> uint32_t {
-    const float r = __builtin_rintf(__fdiv_rn(x, scale));
-    return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(r, -128.0f), 127.0f);
-  };
-  const uint32_t per_row = (uint32_t)ldq / 4, total = (uint32_t)K * per_row;
-  for (uint32_t i = blockIdx.x * kQbThreads + threadIdx.x; i < total; i += gridDim.x * kQbThreads) {
-    const uint32_t k = i / per_row, c = 4 * (i - k * per_row);
-    const float* src = b + (int64_t)k * N + c;
-    float x[4] = {0.f, 0.f, 0.f, 0.f};
-    if ((int32_t)c + 4 <= N) __builtin_memcpy(x, src, 16);
-    else
-      for (int e = 0; e < 4; ++e)
-        if ((int32_t)c + e < N) x[e] = src[e];
-    uint32_t w = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) w |= ((int32_t)c + e < N ? code(x[e]) : 0u) << (8 * e);
-    reinterpret_cast<uint32_t*>(q)[i] = w;
+  const uint64_t i0 = blockIdx.x * kQbSmallThreads + threadIdx.x, stride = gridDim.x * kQbSmallThreads;
+  for (uint64_t i = i0; i < w.total; i += stride) {
+    int32_t v;
+    const v4f x = load_word<FLAT>(w, i, v);
+    store_word(w, i, x, v, scale);
   }
+  tail<FLAT>(w, scale, i0, stride);
+}
+
+// Up to kQbSmall floats one launch is faster on the device (512 x 128: 4.2 us
+// against 5.2 for two) and saves the host a launch; at twice that it is not
+// (1024 x 128: 6.7 against 5.4).  Above, both passes keep four loads per thread
+// in flight (4096 x 512: 9.0 -> 7.8 us, 4096 x 2048: 17.6 -> 16.4).
+template <bool FLAT>
+int quantize_b(const BWords& w, float* scale, uint32_t* partials, hipStream_t stream) {
+  if (w.n <= kQbSmall) {
+    const int g = (int)std::max<int64_t>(1, std::min<int64_t>(32, ((int64_t)w.total + kQbSmallThreads - 1) / kQbSmallThreads));
+    hipLaunchKernelGGL(b_small_kernel<FLAT>, dim3(g), dim3(kQbSmallThreads), 0, stream, w, scale);
+  } else {
+    const int g = (int)std::min<int64_t>(kQbMaxPartials, (w.n + 4095) / 4096);
+    hipLaunchKernelGGL(b_amax_kernel, dim3(g), dim3(kQbThreads), 0, stream, w.b, w.n, partials);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
+    const int gq = (int)std::min<int64_t>(2048, ((int64_t)w.total + 1023) / 1024);
+    hipLaunchKernelGGL(b_quant_kernel<FLAT>, dim3(gq), dim3(kQbThreads), 0, stream, w, partials, g, scale);
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
+  return VOID_OK;
 }
 
 // Rows of bytes at any alignment to rows of 16-byte chunks: a thread writes one
@@ -416,15 +501,7 @@ int void_quantize_b_i8(const float* b, int64_t n, int8_t* q, float* scale, uint3
   if (n == 0) return VOID_OK;
   if (!b || !q || !scale || !partials) return void_internal_fail(VOID_ERR_ARG, "null pointer");
   if ((uintptr_t)b % 16 || (uintptr_t)q % 4) return void_internal_fail(VOID_ERR_ARG, "b must be 16-byte, q 4-byte aligned");
-  const int g = (int)std::min<int64_t>(kQbMaxPartials, std::max<int64_t>(1, (n + 4095) / 4096));
-  hipLaunchKernelGGL(b_amax_kernel, dim3(g), dim3(kQbThreads), 0, stream, b, n, partials);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
-  const int gq = (int)std::min<int64_t>(2048, std::max<int64_t>(1, (n + 4095) / 4096));
-  hipLaunchKernelGGL(b_quant_kernel, dim3(gq), dim3(kQbThreads), 0, stream, b, n, partials, g, q, scale);
-  e = hipGetLastError();
-  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
-  return VOID_OK;
+  return quantize_b<true>(BWords{b, q, n, 0, 0, (uint64_t)(n / 4)}, scale, partials, stream);
 }
 
 int void_quantize_b_i8_rows(const float* b, int32_t K, int32_t N, int8_t* q, int32_t ldq, float* scale,
@@ -437,15 +514,7 @@ int void_quantize_b_i8_rows(const float* b, int32_t K, int32_t N, int8_t* q, int
   if (ldq < N || ldq % 4) return void_internal_fail(VOID_ERR_ARG, "ldq must be a multiple of 4 and at least N");
   const int64_t n = (int64_t)K * N, groups = (int64_t)K * (ldq / 4);
   if (groups > INT32_MAX) return void_internal_fail(VOID_ERR_UNSUPPORTED, "too many code groups");
-  const int g = (int)std::min<int64_t>(kQbMaxPartials, std::max<int64_t>(1, (n + 4095) / 4096));
-  hipLaunchKernelGGL(b_amax_kernel, dim3(g), dim3(kQbThreads), 0, stream, b, n, partials);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
-  const int gq = (int)std::min<int64_t>(2048, std::max<int64_t>(1, (groups + 1023) / 1024));
-  hipLaunchKernelGGL(b_quant_rows_kernel, dim3(gq), dim3(kQbThreads), 0, stream, b, K, N, partials, g, q, ldq, scale);
-  e = hipGetLastError();
-  if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
-  return VOID_OK;
+  return quantize_b<false>(BWords{b, q, n, N, (uint32_t)ldq / 4, (uint64_t)groups}, scale, partials, stream);
 }
 
 int void_copy_rows_b8(const void* src, int64_t ld_src, int32_t rows, int32_t cols, void* dst, int64_t ld_dst,
