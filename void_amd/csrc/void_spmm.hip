@@ -2575,7 +2575,16 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   p.n_panels = n_panels;
   p.activation = d->activation;
   p.n_items = n_items;
-  p.panel_group = n_panels >= 16 ? n_panels / 8 : 1;
+  // Panels per XCD share, as long as the B columns of a group fit the XCD's
+  // 4 MB L2: past it, each panel's columns come from the Infinity Cache again
+  // (4096 x 14336, 14336 bf16 tiles, N = 2048, 3.7 MB a panel: 180 us in groups of
+  // two, 135 us one by one; at 2 MB a panel both take the same time).
+  {
+    const int b_esz = (elt == kEltF32 || elt == kEltFp8F32) ? 4 : (elt == kEltI8 || elt == kEltFp8) ? 1 : 2;
+    const int64_t panel_bytes = (int64_t)a->K * kPanel * b_esz;
+    const int fit = (int)std::max<int64_t>(1, ((int64_t)4 << 20) / std::max<int64_t>(panel_bytes, 1));
+    p.panel_group = n_panels >= 16 ? std::min(n_panels / 8, fit) : 1;
+  }
   // With split rows (a long-tailed distribution) every XCD that shares a
   // panel group gets a dealt share of the longest-first list; otherwise the
   // first of them would take all the longest rows.  Without splits the
