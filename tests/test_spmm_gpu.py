@@ -521,3 +521,22 @@ def test_transpose_b8(gpu, rows, cols, pad):
     _lib.check(st, "void_transpose_b8")
     assert torch.equal(dst[:, :rows], src[:, :cols].t())
     assert torch.all(dst[:, rows:] == 7)
+
+
+@pytest.mark.parametrize("rows,N", [(129, 1024), (128, 1024), (256, 512), (200, 512), (65, 2048), (100, 1152)])
+def test_snaked_grid_covers_every_block(gpu, monkeypatch, rows, N):
+    """Grids of 513 to 1024 workgroups (one past it, shares that are no multiple
+    of 32, groups of two panels, panels that no layout divides): every block
+    once, on the default kernel, unequal rows and empty ones included."""
+    monkeypatch.delenv("VOID_AMD_KERNEL", raising=False)
+    M = 32 * rows - 5
+    rng = np.random.default_rng(rows)
+    case = cases.uniform_blocks(M, 320, N, 3 * rows, seed=rows)
+    keep = (case.block_rows % 7 != 3) | (rng.random(len(case.block_rows)) < 0.3)
+    keep[case.block_rows == rows - 1] = True
+    for f in ("tiles", "block_rows", "block_cols"):
+        setattr(case, f, np.ascontiguousarray(getattr(case, f)[keep]))
+    qd, A, bq, bs = _int8_setup(case, gpu)
+    raw = void_amd.void_spmm_int8(qd, torch.from_numpy(bq).to(gpu), epilogue="raw_i32",
+                                  out=torch.full((M, N), -1, dtype=torch.int32, device=gpu))
+    assert np.array_equal(raw.cpu().numpy(), oracle.i8_acc(A, bq))

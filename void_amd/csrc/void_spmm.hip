@@ -206,6 +206,19 @@ __device__ __forceinline__ void wg_tile(int L, int n_items, int n_panels, int pg
   item = undeal(pos, n_items, item_piles);
 }
 
+// Position k of an XCD's longest-first share such that the workgroups of one
+// CU get long and short rows: in shares of up to 64 (two workgroups per CU)
+// the second half reversed, in longer ones every other run of 32 (one run
+// gives each of the 32 CUs one workgroup).
+__device__ __forceinline__ int snake(int k, int share) {
+  if (share <= 64) {
+    const int half = (share + 1) >> 1;
+    return k < half ? k : share - 1 - (k - half);
+  }
+  const int lo = k & ~31, hi = min(lo + 32, share);
+  return (k & 32) ? lo + hi - 1 - k : k;
+}
+
 // Hardware workgroup id -> (work item, panel); false for the padding
 // workgroups of the exact layout below, which do nothing.
 //
@@ -215,13 +228,15 @@ __device__ __forceinline__ void wg_tile(int L, int n_items, int n_panels, int pg
 // x % item_piles, one whole item (its panel_group panels back to back) after
 // another.  The grid is 8 x (that share's workgroups, rounded up), so every
 // XCD's share is a longest-first slice of equal length.  Unsplit grids of
-// one resident round (pair_snake) take the same layout with the second half
-// of each XCD's share reversed: the dispatcher gives each CU of an XCD one
-// workgroup of the first half and then one of the second (read from
+// one resident round (pair_snake) take the same layout with the share snaked
+// (see snake): the dispatcher gives each CU of an XCD one workgroup of the
+// first half and then one of the second (read from
 // HW_REG_HW_ID in an instrumented build: workgroups s and s + 32 of an XCD's
 // 64 share a CU), so a CU's pair is a long and a short row.  Against
 // contiguous ranges, where one XCD of a panel took all its longest rows, c2
-// went 8.6-8.8 -> 7.9-8.1 us and c3 10.9-11.1 -> 10.2-10.7 us cold.
+// went 8.6-8.8 -> 7.9-8.1 us and c3 10.9-11.1 -> 10.2-10.7 us cold; with four
+// one-ring workgroups per CU (1024), 256 rows x 4 panels of bf16 17.9 -> 15.8 us,
+// of int8 13.2 -> 12.0, 128 rows x 8 panels of fp32 62.2 -> 58.8.
 // Otherwise each XCD runs a contiguous range of logical ids (xcd_remap),
 // mapped by wg_tile.
 __device__ __forceinline__ bool wg_map(const Params& p, int& item, int& panel) {
@@ -231,10 +246,7 @@ __device__ __forceinline__ bool wg_map(const Params& p, int& item, int& panel) {
     const int piles = p.item_piles, pg = p.panel_group;
     int k = s / pg;
     panel = (x / piles) * pg + (s - k * pg);
-    if (p.pair_snake) {
-      const int share = (p.n_items + piles - 1) / piles, half = (share + 1) >> 1;
-      k = k < half ? k : share - 1 - (k - half);
-    }
+    if (p.pair_snake) k = snake(k, (p.n_items + piles - 1) / piles);
     item = k * piles + x % piles;
     return item < p.n_items;
   }
@@ -254,10 +266,7 @@ __device__ __forceinline__ bool wg_map_args(int map_word, int n_items, int n_pan
     const int x = h & 7, s = h >> 3;
     int k = s / pg;
     panel = (x / piles) * pg + (s - k * pg);
-    if (map_word & 2) {
-      const int share = (n_items + piles - 1) / piles, half = (share + 1) >> 1;
-      k = k < half ? k : share - 1 - (k - half);
-    }
+    if (map_word & 2) k = snake(k, (n_items + piles - 1) / piles);
     item = k * piles + x % piles;
     return item < n_items;
   }
@@ -2594,13 +2603,16 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     const int n_groups = (n_panels + p.panel_group - 1) / p.panel_group;
     p.item_piles = n_split_tiles > 0 ? std::max(1, 8 / n_groups) : 1;
     // One-round unsplit grids (every workgroup resident from the start) take
-    // the same dealt layout, with the second half of each XCD's share in
-    // reverse: a CU's two workgroups are then one long and one short row.
-    if (n_split_tiles == 0 && grid64 <= kPairGridMax) {
+    // the same dealt layout, snaked: a CU's workgroups are then long and short
+    // rows.  Up to two 8-wave workgroups per CU always; up to four 4-wave ones
+    // where the layout is exact (with 6 panels, dealing into the piles that fit
+    // ranges across panels measured 8 % slower than the plain order).
+    const bool exact = n_panels % p.panel_group == 0 && 8 % n_groups == 0;
+    if (n_split_tiles == 0 && grid64 <= (exact ? 2 * kPairGridMax : kPairGridMax)) {
       p.item_piles = std::max(1, 8 / n_groups);
       p.pair_snake = 1;
     }
-    if ((n_split_tiles > 0 || p.pair_snake) && n_panels % p.panel_group == 0 && 8 % n_groups == 0) {
+    if ((n_split_tiles > 0 || p.pair_snake) && exact) {
       p.xcd_exact = 1;
       grid_exact = 8 * (((int64_t)n_items + p.item_piles - 1) / p.item_piles) * p.panel_group;
     }
