@@ -340,3 +340,29 @@ def test_linear_create_graph_bias(gpu):
     (gb,) = torch.autograd.grad(lin(x), lin.bias, gy, create_graph=True)
     (gg,) = torch.autograd.grad(gb.sum(), gy)
     assert torch.equal(gg, torch.ones_like(gy))
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 1e38])
+@pytest.mark.parametrize("grouped", ["tiles", "grouped"])
+def test_sddmm_non_finite_follow_fp32(gpu, monkeypatch, bad, grouped):
+    """A tile whose sums are not finite equals the fp32 MFMA's (the
+    register-staged kernel's); the others stay within the fp32 bound."""
+    from void_amd.format import build_bsr_layout
+    case = cases.uniform_blocks(130, 200, 100, 20, seed=4)
+    g = torch.randn(130, 100, device=gpu)
+    b = torch.from_numpy(case.b).to(gpu)
+    g[40, 7] = bad
+    if bad == 1e38:
+        g[40, 8] = -bad
+        b *= 100
+    rows, cols = torch.from_numpy(case.block_rows).to(gpu), torch.from_numpy(case.block_cols).to(gpu)
+    lay = build_bsr_layout(rows, cols, 5, 7, gpu)
+    out = {}
+    for mode in (grouped, "rows"):
+        monkeypatch.setenv("VOID_AMD_SDDMM", mode)
+        out[mode] = _runtime.sddmm_tiles(g, b, rows, cols, (130, 200), torch.float32, layout=lay)
+    a, r = out[grouped], out["rows"]
+    assert not bool(torch.isfinite(r).all())
+    assert torch.equal(torch.isnan(a), torch.isnan(r)) and torch.equal(torch.isinf(a), torch.isinf(r))
+    ok = torch.isfinite(r).all(dim=2).all(dim=1)
+    assert bool(ok.any()) and bool(((a - r)[ok].abs() <= 1e-5 * r[ok].abs().max()).all())
