@@ -107,6 +107,17 @@ typedef struct void_plan {
   int32_t chunk_tiles;
 } void_plan;
 
+/* void_dense_args.flags */
+/* b_scale_vec holds a single scale for all columns (a per-tensor scale that
+ * stays in device memory) instead of [N]. */
+#define VOID_DENSE_ONE_B_SCALE 1
+/* Float B (fp32, bf16, fp16) of any width: the kernels may read a row of B up
+ * to the next multiple of 16 bytes past column N (inside its pitch ldb; what
+ * lies there does not matter).  Lifts the N % 4 and N % 8 conditions and those
+ * on C of the float SpMMs below; b stays 16-byte aligned with ldb a multiple
+ * of 16 bytes. */
+#define VOID_DENSE_PADDED_B 2
+
 /* The dense operand and the output of one SpMM call. */
 typedef struct void_dense_args {
   const void* b;          /* K x N: int8 (void_spmm_int8), e4m3fn (void_spmm_fp8), fp32 (void_spmm_f32) */
@@ -114,7 +125,7 @@ typedef struct void_dense_args {
   int32_t b_col_major;    /* 0: (k,n) at b[k*ldb+n]; 1: (k,n) at b[n*ldb+k] */
   int32_t N;
   float b_scale;          /* per-tensor scale of B, used when b_scale_vec is NULL */
-  const float* b_scale_vec; /* [N] per-column scale of B, or NULL; see b_scale_one */
+  const float* b_scale_vec; /* [N] per-column scale of B, or NULL; see VOID_DENSE_ONE_B_SCALE */
   const float* bias;      /* [N] added before the activation, or NULL */
   void* c;                /* M x N row-major output */
   int64_t ldc;
@@ -122,8 +133,7 @@ typedef struct void_dense_args {
   int32_t activation;     /* void_activation */
   int32_t bias_per_row;   /* 0: bias[N] per column; 1: bias[M] per output row (the reference's
                              row-bias kernel, void/fusion.py:202-304; float SpMM only) */
-  int32_t b_scale_one;    /* 1: b_scale_vec holds a single scale for all columns (a per-tensor scale
-                             that stays in device memory); 0: [N] */
+  int32_t flags;          /* VOID_DENSE_* bits, or 0 */
 } void_dense_args;
 
 /* ---------------------------------------------------------------------- */

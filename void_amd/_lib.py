@@ -18,6 +18,9 @@ ABI_VERSION = 5
 NOALLOC_COUNTER_BYTES = 1 << 20
 NOALLOC_PARTIAL_BYTES = 31 << 20
 
+# void_dense_args.flags
+DENSE_ONE_B_SCALE, DENSE_PADDED_B = 1, 2
+
 # enum void_epilogue
 EPI_RAW_I32 = 0
 EPI_ROW_MEAN = 1
@@ -90,7 +93,7 @@ class DenseArgs(ctypes.Structure):
         ("out_dtype", c_int32),
         ("activation", c_int32),
         ("bias_per_row", c_int32),
-        ("b_scale_one", c_int32),
+        ("flags", c_int32),
     ]
 
 

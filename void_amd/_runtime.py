@@ -454,6 +454,65 @@ def contiguous_2d(t: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def aligned_rows(t: torch.Tensor) -> bool:
+    """Unit column stride and 16-byte aligned rows (2-D)."""
+    s0, s1 = t.stride()
+    return s1 == 1 and s0 >= t.shape[1] and s0 * t.element_size() % 16 == 0 and t.data_ptr() % 16 == 0
+
+
+def padded_rows(t: torch.Tensor, zero_tail: bool = False) -> torch.Tensor:
+    """A 2-D 16- or 32-bit GPU tensor as aligned_rows: t itself where it is,
+    else a copy whose pitch is a multiple of 16 bytes (of a 128-byte line from
+    there on) and whose rows are zero from their end to the next multiple of
+    16 bytes.  With zero_tail, t itself only if its rows end on one."""
+    R, C = t.shape
+    per = 16 // t.element_size()
+    s0, s1 = t.stride()
+    if not t.numel() or (aligned_rows(t) and not (zero_tail and C % per)):
+        return t
+    line = 8 * per
+    pitch = -(-C // line) * line if C > line else -(-C // per) * per
+    if s1 == 1 and s0 >= C and R * -(-C // per) < 1 << 31:
+        out = torch.empty(R, pitch, dtype=t.dtype, device=t.device)[:, :C]
+        esz = t.element_size()
+        st = _lib.lib().void_copy_rows_b8(t.data_ptr(), s0 * esz, R, C * esz, out.data_ptr(), pitch * esz,
+                                          raw_stream(t.device))
+        _lib.check(st, "void_copy_rows_b8")
+        return out
+    buf = torch.empty(R, pitch, dtype=t.dtype, device=t.device)
+    if C % per:
+        buf[:, C:-(-C // per) * per].zero_()
+    out = buf[:, :C]
+    if s0 == 1 and s1 >= R and t.numel() >= TRANSPOSE_MIN_NUMEL and max(R, C) <= 64 * 65535:
+        st = _lib.lib().void_transpose(t.data_ptr(), s1, C, R, out.data_ptr(), pitch, t.element_size(),
+                                       raw_stream(t.device))
+        _lib.check(st, "void_transpose")
+    else:
+        out.copy_(t)
+    return out
+
+
+# A float B (or gradient) whose rows are not 16-byte aligned is copied to
+# padded rows for the LDS-DMA rings from this many elements on (eager calls:
+# 1000 x 257 bf16, 200 tiles 29.7 -> 19.8 us; 4096 x 730, 1638 tiles, bf16
+# 87 -> 19 us, fp32 80 -> 39; bf16 training step of 4096 x 4096, 1001 tokens
+# 802 -> 334).  Smaller ones keep the element-wise fp32 kernels, whose single
+# launch takes no longer (512 x 130, 60 tiles: bf16 18.3 against 20.0 us with the
+# copy, fp32 15.1 against 18.5).
+PAD_FLOAT_MIN_NUMEL = 1 << 17
+
+
+def row_major(t: torch.Tensor) -> torch.Tensor:
+    """t (2-D) row-major for the float kernels: in place with aligned rows, a
+    padded copy from PAD_FLOAT_MIN_NUMEL elements on, contiguous otherwise."""
+    if t.is_cuda and t.element_size() in (2, 4) and t.numel():
+        if aligned_rows(t):
+            return t
+        if t.numel() >= PAD_FLOAT_MIN_NUMEL and (t.shape[1] * t.element_size()) % 16:
+            return padded_rows(t)
+    return contiguous_2d(t)
+
+
 def aligned_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
     """Copy of a row-major 8-bit B (rows ld apart) with 16-byte aligned rows."""
     K, N = b.shape
@@ -466,11 +525,11 @@ def aligned_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
 
 
 def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
-           b_scale_vec: Optional[torch.Tensor] = None, b_scale_one: bool = False, out: torch.Tensor, epilogue: int,
+           b_scale_vec: Optional[torch.Tensor] = None, flags: int = 0, out: torch.Tensor, epilogue: int,
            activation: int = _lib.ACT_NONE, bias: Optional[torch.Tensor] = None,
            chunk: int) -> torch.Tensor:
     """Launch one SpMM on the current stream of out's device; returns out.
-    With b_scale_one, b_scale_vec holds one scale for every column."""
+    flags: DENSE_* bits of _lib."""
     lib = _lib.lib()
     N = b.shape[1]
     b_t, ldb, col_major = dense_operand(b)
@@ -495,7 +554,7 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
     dense = _lib.DenseArgs(b_t.data_ptr(), ldb, col_major, N, b_scale,
                            b_scale_vec.data_ptr() if b_scale_vec is not None else None,
                            bias.data_ptr() if bias is not None else None, target.data_ptr(), target.stride(0),
-                           _OUT_CODES[target.dtype], activation, 0, b_scale_one)
+                           _OUT_CODES[target.dtype], activation, 0, flags)
     args = (plan.cplan_ref(), ws.data_ptr() if ws is not None else None, ws_bytes, stream)
     if kind == "int8":
         st = lib.void_spmm_int8(dbsr.desc_ref(), ctypes.byref(dense), epilogue, *args)
@@ -584,13 +643,16 @@ def csr_to_tiles(indptr: np.ndarray, indices: np.ndarray, data: np.ndarray, shap
 
 
 def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor, block_cols: torch.Tensor,
-                shape: Tuple[int, int], out_dtype: torch.dtype, layout=None) -> torch.Tensor:
+                shape: Tuple[int, int], out_dtype: torch.dtype, layout=None, grad_padded: bool = False) -> torch.Tensor:
     """[n, 32, 32] gradient of the nonzero tiles: grad_c[rows of t] @ b[cols of t]^T.
 
     With the tiles' BsrLayout (block-row order and the Morton index of each
     position), void_sddmm_rows_f32 shares each block-row's grad_c rows among
     its tiles (void_sddmm_rows_bf16 / _f16 when grad_c and b share a 16-bit
-    dtype); without it, void_sddmm_f32 takes the tiles one by one."""
+    dtype); without it, void_sddmm_f32 takes the tiles one by one.  The ring
+    kernels take whole 16-byte chunks of a row: other widths run on copies
+    with zeros up to the next chunk (grad_padded: grad_c comes from
+    padded_rows with zero_tail)."""
     M, K = shape
     n = int(block_rows.numel())
     N = grad_c.shape[1]
@@ -600,22 +662,32 @@ def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor,
     if N == 0:
         return out.zero_()
     stream = raw_stream(grad_c.device)
+    pad = max(M, K) * N >= PAD_FLOAT_MIN_NUMEL
     entry16 = {torch.bfloat16: "void_sddmm_rows_bf16", torch.float16: "void_sddmm_rows_f16"}.get(grad_c.dtype)
-    if layout is not None and entry16 is not None and b.dtype == grad_c.dtype:
+    if layout is not None and entry16 is not None and b.dtype == grad_c.dtype and (N % 8 == 0 or pad):
         # 16-bit operands of one dtype on the 16-bit MFMA (16-byte rows).
-        g16 = grad_c if grad_c.stride(1) == 1 else contiguous_2d(grad_c)
-        b16 = b if b.stride(1) == 1 else contiguous_2d(b)
-        if (N % 8 == 0 and g16.stride(0) % 8 == 0 and b16.stride(0) % 8 == 0 and g16.data_ptr() % 16 == 0
+        if N % 8 == 0:
+            g16 = grad_c if grad_c.stride(1) == 1 else contiguous_2d(grad_c)
+            b16 = b if b.stride(1) == 1 else contiguous_2d(b)
+        else:
+            g16 = grad_c if grad_padded else padded_rows(grad_c, zero_tail=True)
+            b16 = padded_rows(b, zero_tail=True)
+        if (g16.stride(0) % 8 == 0 and b16.stride(0) % 8 == 0 and g16.data_ptr() % 16 == 0
                 and b16.data_ptr() % 16 == 0 and 32 * max(g16.stride(0), b16.stride(0)) * 2 < (1 << 31)):
             groups = layout.row_groups()
             st = getattr(_lib.lib(), entry16)(g16.data_ptr(), g16.stride(0), b16.data_ptr(), b16.stride(0),
                                               groups.data_ptr(), int(groups.shape[0]), layout.col_idx.data_ptr(),
-                                              layout.order.data_ptr(), M, N, K, out.data_ptr(), out_code(out_dtype),
-                                              stream)
+                                              layout.order.data_ptr(), M, -(-N // 8) * 8, K, out.data_ptr(),
+                                              out_code(out_dtype), stream)
             _lib.check(st, entry16)
             return out
-    g = contiguous_2d(grad_c.to(torch.float32))
-    bb = contiguous_2d(b.to(torch.float32))
+    g, bb = grad_c.to(torch.float32), b.to(torch.float32)
+    if N % 4 and pad:
+        g = g if grad_padded and g is grad_c else padded_rows(g, zero_tail=True)
+        bb = padded_rows(bb, zero_tail=True)
+        N = -(-N // 4) * 4
+    else:
+        g, bb = contiguous_2d(g), contiguous_2d(bb)
     groups = layout.row_groups() if layout is not None else None
     # Up to 1.5 row groups per CU: the per-tile kernel, whose workgroups
     # always hold 8 tiles, outweighs the shared grad_c rows (c2, 262 groups of

@@ -94,7 +94,11 @@ def _backward(ctx: Any, grad_output: torch.Tensor):
     if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[6]):
         return None, None, grad_output
     # One row-major copy of a token-major gradient serves every use of it.
-    grad = _runtime.contiguous_2d(grad_output)
+    # (rows of whole 16-byte chunks where the kernels would copy it to such).
+    N, per = grad_output.shape[1], 16 // max(grad_output.element_size(), 1)
+    padded = (N % per != 0 and max(M, K) * N >= _runtime.PAD_FLOAT_MIN_NUMEL and grad_output.is_cuda
+              and grad_output.element_size() in (2, 4))
+    grad = _runtime.padded_rows(grad_output, zero_tail=True) if padded else _runtime.contiguous_2d(grad_output)
     if ctx.needs_input_grad[6]:
         at = _vt(a_values.detach(), cols, rows, (K, M), ctx.a_tile_size[::-1], ctx.a_n_blocks, cls=_TransposedTiles)
         grad_b = float_spmm(at, grad).to(b.dtype)
@@ -104,7 +108,8 @@ def _backward(ctx: Any, grad_output: torch.Tensor):
             grad_b = _runtime.contiguous_2d(grad_b.t()).t()
     if ctx.needs_input_grad[0]:
         grad_a = _runtime.sddmm_tiles(grad, b, rows, cols, (M, K), a_values.dtype,
-                                      layout=_layout(rows, cols, (M, K)) if rows.is_cuda else None)
+                                      layout=_layout(rows, cols, (M, K)) if rows.is_cuda else None,
+                                      grad_padded=padded)
     return grad_a, grad_b, grad
 
 

@@ -2552,6 +2552,9 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   if (elt == kEltFp8 && epilogue != VOID_EPI_PER_BLOCK)
     return fail(VOID_ERR_UNSUPPORTED, "fp8 SpMM supports only the per-block epilogue");
   const bool b_f32 = elt == kEltF32 || elt == kEltFp8F32;
+  // A float B of any width in rows of 16-byte chunks (the rings read whole
+  // chunks, C leaves element by element where it is cut off or unaligned).
+  const bool padded = (d->flags & VOID_DENSE_PADDED_B) != 0;
   if (b_f32 && d->b_col_major) return fail(VOID_ERR_UNSUPPORTED, "an fp32 B must be row-major");
   if (d->bias_per_row && !unscaled)
     return fail(VOID_ERR_UNSUPPORTED, "a per-row bias is supported by the float SpMM only");
@@ -2574,7 +2577,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   p.ldb = d->ldb;
   p.b_scale = d->b_scale;
   p.b_scale_vec = d->b_scale_vec;
-  p.b_scale_stride = d->b_scale_one ? 0 : 1;
+  p.b_scale_stride = (d->flags & VOID_DENSE_ONE_B_SCALE) ? 0 : 1;
   p.bias = d->bias;
   p.c = d->c;
   p.ldc = d->ldc;
@@ -2666,7 +2669,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     // N % 4 == 0, 31-bit byte offsets); the Python wrapper pads other shapes.
     const int64_t lim = (int64_t)1 << 31;
     const int esz = (d->out_dtype == VOID_DT_BF16 || d->out_dtype == VOID_DT_F16) ? 2 : 4;
-    if (!(c_ok && (bu % 16 == 0) && (d->ldb % 4 == 0)))
+    if (!((c_ok || padded) && (bu % 16 == 0) && (d->ldb % 4 == 0)))
       return fail(VOID_ERR_UNSUPPORTED, "E4M3 x fp32 SpMM needs 16-byte aligned B and C rows and N %% 4 == 0");
     if (!((int64_t)a->n_blocks * kTile * kTile < lim && (int64_t)((a->K + kTile - 1) / kTile) * kTile * d->ldb * 4 < lim &&
           (int64_t)a->M * d->ldc * esz < lim))
@@ -2693,7 +2696,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     const int64_t lim = (int64_t)1 << 31;
     const int64_t a_tile_bytes = (elt == kEltBf16 || elt == kEltF16) ? 2048 : 1024;
     const int esz = (d->out_dtype == VOID_DT_BF16 || d->out_dtype == VOID_DT_F16) ? 2 : 4;
-    if (d->b_col_major || !(c_ok && (bu % 16 == 0) && (d->ldb % 8 == 0) && (d->N % 8 == 0)))
+    if (d->b_col_major || !((bu % 16 == 0) && (d->ldb % 8 == 0) && (padded || (c_ok && d->N % 8 == 0))))
       return fail(VOID_ERR_UNSUPPORTED, "16-bit SpMM needs a row-major B, 16-byte aligned B and C rows and N %% 8 == 0");
     if (plan->chunk_tiles > kCgMaxTiles)
       return fail(VOID_ERR_ARG, "16-bit SpMM takes work items of at most %d tiles (chunk_tiles %d)", kCgMaxTiles,
@@ -2730,7 +2733,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     // keeps the fp32 kernel of its own (the fallback for everything else).
     const char* fk = getenv("VOID_AMD_KERNEL");
     const int64_t lim = (int64_t)1 << 31;
-    const bool ring_ok = vec && !d->b_col_major && plan->chunk_tiles <= kCgMaxTiles &&
+    const bool ring_ok = (vec || (padded && (bu % 16 == 0) && (d->ldb % 4 == 0))) && !d->b_col_major && plan->chunk_tiles <= kCgMaxTiles &&
                          (int64_t)a->n_blocks * kTile * kTile * 4 < lim &&
                          (int64_t)((a->K + kTile - 1) / kTile) * kTile * d->ldb * 4 < lim &&
                          (int64_t)a->M * d->ldc * 4 < lim && !(fk && strcmp(fk, "f32") == 0);

@@ -130,12 +130,13 @@ def _void_spmm_activation_row_bias(a, b: torch.Tensor, bias: Optional[torch.Tens
                                    activation: str) -> torch.Tensor:
     """activation(A @ B + bias[:, None]) with a per-row bias [M] for float A
     (fusion.py:307-377): the fp32 kernel with bias_per_row, output in B's dtype;
-    B is made contiguous as the reference does."""
+    B is made row-major as the reference does."""
+    from . import _runtime
     from .format import VOIDTensor
     from .ops import float_spmm
     if not isinstance(a, VOIDTensor):
         raise TypeError("the row-bias activation SpMM takes a float VOIDTensor")
-    b = b.contiguous()
+    b = _runtime.row_major(b)
     if a.n_blocks == 0:
         res = torch.zeros(a.shape[0], b.shape[1], dtype=b.dtype, device=b.device) if out is None else out.zero_()
         if bias is not None:
@@ -204,7 +205,7 @@ class FusedSparseLinear(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         from . import _runtime
         x_flat = x.reshape(-1, self.in_features)
-        b = _runtime.contiguous_2d(x_flat.t())  # [in, batch], row-major, as the reference passes it
+        b = _runtime.row_major(x_flat.t())  # [in, batch], as the reference passes it
         bias = self.bias.detach() if self.bias is not None else None
         vt = self.get_void_tensor()
         if vt.n_blocks == 0:

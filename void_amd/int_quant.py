@@ -424,7 +424,8 @@ def void_spmm_int8(
     chunk = chunk_tiles or tuning.select_chunk("int8", a.n_blocks, N, dbsr.max_row)
     if bias is not None:
         bias = _runtime.vector_f32(bias, b.device)
-    return _runtime.launch("int8", dbsr, b, b_scale=scalar_scale, b_scale_vec=scale_vec, b_scale_one=one, out=out,
+    return _runtime.launch("int8", dbsr, b, b_scale=scalar_scale, b_scale_vec=scale_vec,
+                           flags=_lib.DENSE_ONE_B_SCALE if one else 0, out=out,
                            epilogue=_lib.EPILOGUES[epilogue], activation=get_activation_code(activation),
                            bias=bias, chunk=chunk)
 

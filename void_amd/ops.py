@@ -20,14 +20,11 @@ _K16 = {torch.bfloat16: "void_spmm_bf16", torch.float16: "void_spmm_f16"}
 
 
 def _fits16(a, b: torch.Tensor, c: torch.Tensor) -> bool:
-    """What void_spmm_bf16 / void_spmm_f16 take: row-major B and C with
-    16-byte aligned rows, N % 8 == 0, and operands within 31-bit offsets."""
+    """What void_spmm_bf16 / void_spmm_f16 take: row-major B with 16-byte
+    aligned rows, and operands within 31-bit offsets."""
     M, K = a.shape
-    N = b.shape[1]
     lim = 1 << 31
-    return (N % 8 == 0 and b.stride(0) % 8 == 0 and b.data_ptr() % 16 == 0 and
-            c.data_ptr() % 16 == 0 and c.stride(0) % 4 == 0 and
-            a.n_blocks * 2048 < lim and ((K + 31) // 32) * 32 * b.stride(0) * 2 < lim and
+    return (_runtime.aligned_rows(b) and a.n_blocks * 2048 < lim and ((K + 31) // 32) * 32 * b.stride(0) * 2 < lim and
             M * c.stride(0) * c.element_size() < lim)
 
 
@@ -70,15 +67,16 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
     entry = "void_spmm_f32"
     bk = None
     if a.values.dtype == b.dtype and b.dtype in _K16:
-        bk = b if b.stride(1) == 1 else _runtime.contiguous_2d(b)
+        bk = _runtime.row_major(b)
         if not _fits16(a, bk, target):
             bk = None
     if bk is not None:
         entry = _K16[b.dtype]
         dbsr = a.device_bsr(b.dtype)
     else:
-        bk = _runtime.contiguous_2d(b.to(torch.float32))
+        bk = _runtime.row_major(b.to(torch.float32))
         dbsr = a.device_bsr()
+    flags = _lib.DENSE_PADDED_B if _runtime.aligned_rows(bk) else 0
     if plan is None:
         plan = dbsr.plan(F32_CHUNK)
     elif plan.chunk > F32_CHUNK:
@@ -88,7 +86,7 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
     # Fields in the struct's order.
     dense = _lib.DenseArgs(bk.data_ptr(), bk.stride(0), 0, N, 1.0, None, bias.data_ptr() if bias is not None else None,
                            target.data_ptr(), target.stride(0), _runtime.out_code(target.dtype), activation,
-                           bias_per_row, 0)
+                           bias_per_row, flags)
     st = getattr(lib, entry)(dbsr.desc_ref(), ctypes.byref(dense), plan.cplan_ref(),
                              ws.data_ptr() if ws is not None else None, ws_bytes, stream)
     _lib.check(st, entry)
