@@ -192,3 +192,19 @@ def test_narrow_fp8(gpu, N):
         raw = b.view(torch.float8_e4m3fn) if b.stride(1) == 1 else b.t().view(torch.float8_e4m3fn).t()
         out = void_amd.void_spmm_fp8(f8.to(gpu), raw, output_dtype=torch.float32).double().cpu()
         assert bool(((out - ref).abs() <= 2.0 ** -13 * bound + 1e-30).all())
+
+
+@pytest.mark.parametrize("K,N", [(203, 65), (256, 130), (200, 250), (96, 512), (1, 70), (33, 129)])
+def test_column_major_any_alignment(gpu, K, N):
+    """Column-major 8-bit B wider than the narrow kernel takes, at every
+    alignment: copied to aligned rows where only single-byte loads are left."""
+    case = cases.uniform_blocks(170, K, N, max(1, 5 * -(-K // 32) // 2), seed=N)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu")).to(gpu)
+    A = oracle.Bsr(q.values.cpu().numpy(), q.scales.cpu().numpy(), case.block_rows, case.block_cols, (170, K))
+    bq, _ = oracle.quantize_i8_tensor(case.b)
+    acc = oracle.i8_acc(A, bq)
+    for b in _layouts(bq, gpu):
+        assert np.array_equal(void_amd.void_spmm_int8(q, b, epilogue="raw_i32").cpu().numpy(), acc)
+        if b.stride(0) == 1 and K > 1:
+            copy = _runtime.row_major_copy_b8(b, b.stride(1))
+            assert copy.stride(0) % 16 == 0 and torch.equal(copy, b)

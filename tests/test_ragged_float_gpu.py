@@ -19,7 +19,7 @@ ABS = {torch.float32: 0.0, torch.bfloat16: 0.0, torch.float16: 2.0 ** -25}
 
 @pytest.fixture(autouse=True)
 def always_pad(monkeypatch):
-    monkeypatch.setattr(_runtime, "PAD_FLOAT_MIN_NUMEL", 1)
+    monkeypatch.setattr(_runtime, "PAD_FLOAT_MIN_WORK", 1)
 
 
 def _views(b):
@@ -126,6 +126,6 @@ def test_training_step_any_width(gpu, dtype, tokens):
 def test_small_widths_keep_one_launch(gpu, monkeypatch):
     monkeypatch.undo()
     b = torch.randn(100, 37, device=gpu)
-    assert _runtime.row_major(b) is b
-    big = torch.randn(4000, 37, device=gpu)
-    assert _runtime.aligned_rows(_runtime.row_major(big)) and torch.equal(_runtime.row_major(big), big)
+    assert _runtime.row_major(b, 60) is b
+    out = _runtime.row_major(b, 600)
+    assert _runtime.aligned_rows(out) and torch.equal(out, b)

@@ -415,26 +415,28 @@ def dense_operand(b: torch.Tensor) -> Tuple[torch.Tensor, int, bool]:
 
 def row_major_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
     """Row-major K x N copy of a column-major 8-bit B (N columns of K bytes,
-    ld apart): void_transpose_b8 where the shape allows, torch's copy
-    otherwise (into rows of an aligned pitch, which the ring reads for any N)."""
+    ld apart): void_transpose_b8 where the shape allows, else void_transpose
+    into rows of an aligned pitch, which the ring reads for any N."""
     K, N = b.shape
-    if N % 16:
-        out = torch.empty(K, tuning.aligned_pitch(N), dtype=b.dtype, device=b.device)[:, :N]
-    else:
-        out = torch.empty(K, N, dtype=b.dtype, device=b.device)
     if K % 16 == 0 and N % 16 == 0 and ld % 16 == 0 and b.data_ptr() % 16 == 0:
-        st = _lib.lib().void_transpose_b8(b.data_ptr(), ld, N, K, out.data_ptr(), N,
-                                          raw_stream(b.device))
+        out = torch.empty(K, N, dtype=b.dtype, device=b.device)
+        st = _lib.lib().void_transpose_b8(b.data_ptr(), ld, N, K, out.data_ptr(), N, raw_stream(b.device))
         _lib.check(st, "void_transpose_b8")
         return out
-    out.copy_(b)
+    pitch = tuning.aligned_pitch(N)
+    out = torch.empty(K, pitch, dtype=b.dtype, device=b.device)[:, :N]
+    if N > 64 * 65535:
+        out.copy_(b)
+        return out
+    st = _lib.lib().void_transpose(b.data_ptr(), ld, N, K, out.data_ptr(), pitch, 1, raw_stream(b.device))
+    _lib.check(st, "void_transpose")
     return out
 
 
-# From this many elements on void_transpose beats torch's strided copy, whose
-# single dispatch costs the host less (eager calls, 512 x 512: torch 5.9 us,
-# void_transpose 8.1; 1024 x 4096 bf16: 22.4 against 9.1).
-TRANSPOSE_MIN_NUMEL = 1 << 20
+# From this many elements on void_transpose beats torch's strided copy (eager
+# calls, 512 x 512: torch 6.9 us, void_transpose 6.7; 1024 x 4096 bf16: 22.4
+# against 6.2).
+TRANSPOSE_MIN_NUMEL = 1 << 18
 
 
 def contiguous_2d(t: torch.Tensor) -> torch.Tensor:
@@ -493,22 +495,28 @@ def padded_rows(t: torch.Tensor, zero_tail: bool = False) -> torch.Tensor:
 
 
 # A float B (or gradient) whose rows are not 16-byte aligned is copied to
-# padded rows for the LDS-DMA rings from this many elements on (eager calls:
-# 1000 x 257 bf16, 200 tiles 29.7 -> 19.8 us; 4096 x 730, 1638 tiles, bf16
-# 87 -> 19 us, fp32 80 -> 39; bf16 training step of 4096 x 4096, 1001 tokens
-# 802 -> 334).  Smaller ones keep the element-wise fp32 kernels, whose single
-# launch takes no longer (512 x 130, 60 tiles: bf16 18.3 against 20.0 us with the
-# copy, fp32 15.1 against 18.5).
-PAD_FLOAT_MIN_NUMEL = 1 << 17
+# padded rows for the LDS-DMA rings where the tiles times the width reach this
+# (eager calls: 1638 tiles, N = 15 bf16 23.0 -> 19.2 us; 200 tiles, N = 257 bf16
+# 29.7 -> 19.8; 1638 tiles, N = 730 bf16 87 -> 19, fp32 80 -> 39; bf16 training
+# step of 4096 x 4096, 1001 tokens 802 -> 334).  Below, the element-wise fp32
+# kernels' single launch takes no longer (60 tiles, N = 130: bf16 18.3 against
+# 20.0 us with the copy, fp32 15.1 against 18.5).
+PAD_FLOAT_MIN_WORK = 1 << 14
 
 
-def row_major(t: torch.Tensor) -> torch.Tensor:
-    """t (2-D) row-major for the float kernels: in place with aligned rows, a
-    padded copy from PAD_FLOAT_MIN_NUMEL elements on, contiguous otherwise."""
-    if t.is_cuda and t.element_size() in (2, 4) and t.numel():
+def pad_float(n_blocks: int, N: int) -> bool:
+    return n_blocks * N >= PAD_FLOAT_MIN_WORK
+
+
+def row_major(t: torch.Tensor, n_blocks: int) -> torch.Tensor:
+    """t (2-D) row-major for the float kernels on n_blocks tiles: in place with
+    aligned rows, a padded copy where pad_float says so, else contiguous."""
+    esz = t.element_size()
+    if t.is_cuda and esz in (2, 4):
         if aligned_rows(t):
             return t
-        if t.numel() >= PAD_FLOAT_MIN_NUMEL and (t.shape[1] * t.element_size()) % 16:
+        N = t.shape[1]
+        if N * esz % 16 and pad_float(n_blocks, N):
             return padded_rows(t)
     return contiguous_2d(t)
 
@@ -536,7 +544,8 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
     plan = dbsr.plan(chunk)
     short = chunk <= tuning.FP32_B_MAX_CHUNK  # items the narrow and column-group kernels take
     panels8 = kind in ("int8", "fp8") and not (short and tuning.narrow(N, plan.n_split_tiles))
-    if col_major and panels8 and tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K):
+    if col_major and panels8 and N and tuning.copy_col_major_b(
+            dbsr.n_blocks, dbsr.K, bytewise=short and bool(ldb % 16 or dbsr.K % 32 or b_t.data_ptr() % 16)):
         b_t, col_major = row_major_copy_b8(b_t, ldb), False  # for the LDS-DMA ring
         ldb = max(b_t.stride(0), N)
     target = out
@@ -662,7 +671,7 @@ def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor,
     if N == 0:
         return out.zero_()
     stream = raw_stream(grad_c.device)
-    pad = max(M, K) * N >= PAD_FLOAT_MIN_NUMEL
+    pad = pad_float(n, N)
     entry16 = {torch.bfloat16: "void_sddmm_rows_bf16", torch.float16: "void_sddmm_rows_f16"}.get(grad_c.dtype)
     if layout is not None and entry16 is not None and b.dtype == grad_c.dtype and (N % 8 == 0 or pad):
         # 16-bit operands of one dtype on the 16-bit MFMA (16-byte rows).

@@ -96,7 +96,7 @@ def _backward(ctx: Any, grad_output: torch.Tensor):
     # One row-major copy of a token-major gradient serves every use of it.
     # (rows of whole 16-byte chunks where the kernels would copy it to such).
     N, per = grad_output.shape[1], 16 // max(grad_output.element_size(), 1)
-    padded = (N % per != 0 and max(M, K) * N >= _runtime.PAD_FLOAT_MIN_NUMEL and grad_output.is_cuda
+    padded = (N % per != 0 and _runtime.pad_float(ctx.a_n_blocks, N) and grad_output.is_cuda
               and grad_output.element_size() in (2, 4))
     grad = _runtime.padded_rows(grad_output, zero_tail=True) if padded else _runtime.contiguous_2d(grad_output)
     if ctx.needs_input_grad[6]:

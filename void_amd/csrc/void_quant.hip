@@ -28,6 +28,7 @@ constexpr int kWavesPerBlock = 4;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef v4i v4i_any __attribute__((aligned(1)));  // 16 bytes at any address
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -402,21 +403,20 @@ __global__ __launch_bounds__(256) void transpose_b8_kernel(const uint8_t* __rest
   }
 }
 
-// dst[c][r] = src[r][c] for 2- or 4-byte elements: token-major activations or
-// gradients made row-major for the float kernels' rings, whose slab rows are
-// read as whole lines.  A workgroup moves a 64 x 64 tile through LDS: 16-byte
-// loads along source rows, and 16-byte stores along destination rows, each
-// gathered from one LDS column; rows of 64 elements plus 4 bytes put the 8 (or
-// 16) chunks of a column on different banks.  Chunks that are cut off or
-// unaligned go element by element.  HBM-bound: both sides in whole lines
-// (2048 x 4096 bf16, 34 MB moved: 8.4 us, torch's strided copy 36.6 us;
+// dst[c][r] = src[r][c] for 1-, 2- or 4-byte elements: token-major activations
+// or gradients made row-major for the rings, whose slab rows are read as
+// whole lines.  A workgroup moves a 64 x 64 tile through LDS: 16-byte loads
+// along source rows, and 16-byte stores along destination rows, each gathered
+// from one LDS column; rows of 64 elements plus 4 bytes put the chunks of a
+// column on different banks.  Whole chunks move in one access at any
+// alignment, cut-off ones element by element.  HBM-bound: both sides in whole
+// lines (2048 x 4096 bf16, 34 MB moved: 8.4 us, torch's strided copy 36.6 us;
 // 2048 x 14336: 23.3 against 123 us in bf16, 40.8 against 127 us in fp32).
 constexpr int kT2 = 64;
 
 template <typename E>
 __global__ __launch_bounds__(256) void transpose_kernel(const E* __restrict__ src, int64_t ld_src, int32_t rows,
-                                                        int32_t cols, E* __restrict__ dst, int64_t ld_dst,
-                                                        int32_t vec_src, int32_t vec_dst) {
+                                                        int32_t cols, E* __restrict__ dst, int64_t ld_dst) {
   constexpr int kPer = 16 / (int)sizeof(E);   // elements per 16-byte chunk
   constexpr int kChunks = kT2 / kPer;         // chunks per tile row
   constexpr int kStride = kT2 + 4 / (int)sizeof(E);
@@ -426,18 +426,19 @@ __global__ __launch_bounds__(256) void transpose_kernel(const E* __restrict__ sr
 #pragma unroll
   for (int i = 0; i < kT2 * kChunks / 256; ++i) {
     const int q = tid + 256 * i, r = q / kChunks, c = (q % kChunks) * kPer;
-    E v[kPer];
     if (r0 + r < rows) {
       const E* s = src + (int64_t)(r0 + r) * ld_src + c0 + c;
-      if (vec_src && c0 + c + kPer <= cols) {
-        const v4i w = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(s));
-        __builtin_memcpy(v, &w, 16);
+      uint32_t w[4];
+      if (c0 + c + kPer <= cols) {
+        // Read once, so streamed.
+        const v4i v = __builtin_nontemporal_load(reinterpret_cast<const v4i_any*>(s));
+        __builtin_memcpy(w, &v, 16);
       } else {
+        E v[kPer];
 #pragma unroll
         for (int e = 0; e < kPer; ++e) v[e] = c0 + c + e < cols ? s[e] : E(0);
+        __builtin_memcpy(w, v, 16);
       }
-      uint32_t w[4];
-      __builtin_memcpy(w, v, 16);
       uint32_t* d = reinterpret_cast<uint32_t*>(t + r * kStride + c);
 #pragma unroll
       for (int e = 0; e < 4; ++e) d[e] = w[e];
@@ -452,10 +453,10 @@ __global__ __launch_bounds__(256) void transpose_kernel(const E* __restrict__ sr
 #pragma unroll
     for (int e = 0; e < kPer; ++e) v[e] = t[(r + e) * kStride + c];
     E* d = dst + (int64_t)(c0 + c) * ld_dst + r0 + r;
-    if (vec_dst && r0 + r + kPer <= rows) {
+    if (r0 + r + kPer <= rows) {
       v4i w;
       __builtin_memcpy(&w, v, 16);
-      *reinterpret_cast<v4i*>(d) = w;
+      *reinterpret_cast<v4i_any*>(d) = w;
     } else {
 #pragma unroll
       for (int e = 0; e < kPer; ++e)
@@ -472,7 +473,8 @@ int void_transpose(const void* src, int64_t ld_src, int32_t rows, int32_t cols, 
                    int32_t elem_bytes, hipStream_t stream) {
   void_internal_fail(VOID_OK, "");
   if (rows < 0 || cols < 0) return void_internal_fail(VOID_ERR_ARG, "negative size");
-  if (elem_bytes != 2 && elem_bytes != 4) return void_internal_fail(VOID_ERR_UNSUPPORTED, "elements of 2 or 4 bytes");
+  if (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4)
+    return void_internal_fail(VOID_ERR_UNSUPPORTED, "elements of 1, 2 or 4 bytes");
   if ((int64_t)rows * cols == 0) return VOID_OK;
   if (!src || !dst) return void_internal_fail(VOID_ERR_ARG, "null pointer");
   if (ld_src < cols || ld_dst < rows) return void_internal_fail(VOID_ERR_ARG, "leading dimension too small");
@@ -480,15 +482,14 @@ int void_transpose(const void* src, int64_t ld_src, int32_t rows, int32_t cols, 
     return void_internal_fail(VOID_ERR_ARG, "arrays must be aligned to their elements");
   const int64_t gx = ((int64_t)cols + kT2 - 1) / kT2, gy = ((int64_t)rows + kT2 - 1) / kT2;
   if (gy > 65535) return void_internal_fail(VOID_ERR_UNSUPPORTED, "too many rows");
-  const int vs = (uintptr_t)src % 16 == 0 && ld_src * elem_bytes % 16 == 0;
-  const int vd = (uintptr_t)dst % 16 == 0 && ld_dst * elem_bytes % 16 == 0;
-  const dim3 grid((unsigned)gx, (unsigned)gy);
-  if (elem_bytes == 2)
-    hipLaunchKernelGGL(transpose_kernel<uint16_t>, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(src),
-                       ld_src, rows, cols, static_cast<uint16_t*>(dst), ld_dst, vs, vd);
-  else
-    hipLaunchKernelGGL(transpose_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<const uint32_t*>(src),
-                       ld_src, rows, cols, static_cast<uint32_t*>(dst), ld_dst, vs, vd);
+  auto go = [&](auto e) {
+    using E = decltype(e);
+    hipLaunchKernelGGL(transpose_kernel<E>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream,
+                       static_cast<const E*>(src), ld_src, rows, cols, static_cast<E*>(dst), ld_dst);
+  };
+  if (elem_bytes == 1) go(uint8_t{});
+  else if (elem_bytes == 2) go(uint16_t{});
+  else go(uint32_t{});
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return void_internal_fail(VOID_ERR_HIP, hipGetErrorString(e));
   return VOID_OK;

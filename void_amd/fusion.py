@@ -15,6 +15,10 @@ from typing import Optional, Union
 
 import torch
 
+from . import _runtime
+from .format import VOIDTensor
+from .ops import float_spmm
+
 
 class ActivationType(Enum):
     """fusion.py:24-31."""
@@ -78,12 +82,10 @@ def _spmm_activation(a, b: torch.Tensor, bias: Optional[torch.Tensor], out: Opti
     if isinstance(a, FP8VOIDTensor):
         return void_spmm_fp8(a, b, output_dtype=out_dtype, b_scale=b_scale, activation=activation,
                              bias=bias, out=out)
-    from .format import VOIDTensor
     if isinstance(a, VOIDTensor):
         # Float tiles: the reference's own case (fusion.py:444-511), fp32 MFMA
         # kernel; output in B's dtype.  An all-empty A keeps the reference's
         # torch activation of the bias (fusion.py:466-476).
-        from .ops import float_spmm
         if a.n_blocks == 0:
             res = torch.zeros(a.shape[0], b.shape[1], dtype=b.dtype, device=b.device) if out is None else out.zero_()
             if bias is not None:
@@ -131,12 +133,9 @@ def _void_spmm_activation_row_bias(a, b: torch.Tensor, bias: Optional[torch.Tens
     """activation(A @ B + bias[:, None]) with a per-row bias [M] for float A
     (fusion.py:307-377): the fp32 kernel with bias_per_row, output in B's dtype;
     B is made row-major as the reference does."""
-    from . import _runtime
-    from .format import VOIDTensor
-    from .ops import float_spmm
     if not isinstance(a, VOIDTensor):
         raise TypeError("the row-bias activation SpMM takes a float VOIDTensor")
-    b = _runtime.row_major(b)
+    b = _runtime.row_major(b, a.n_blocks)
     if a.n_blocks == 0:
         res = torch.zeros(a.shape[0], b.shape[1], dtype=b.dtype, device=b.device) if out is None else out.zero_()
         if bias is not None:
@@ -193,7 +192,6 @@ class FusedSparseLinear(torch.nn.Module):
 
     def get_void_tensor(self):
         """The weight as a VOIDTensor over the module's buffers (fusion.py:793-806)."""
-        from .format import VOIDTensor
         vt = self._vt
         if vt is None or vt.values is not self.values:
             vt = VOIDTensor(values=self.values, block_rows=self.block_rows, block_cols=self.block_cols,
@@ -203,9 +201,8 @@ class FusedSparseLinear(torch.nn.Module):
         return vt
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from . import _runtime
         x_flat = x.reshape(-1, self.in_features)
-        b = _runtime.row_major(x_flat.t())  # [in, batch], as the reference passes it
+        b = _runtime.row_major(x_flat.t(), self.n_blocks)  # [in, batch], as the reference passes it
         bias = self.bias.detach() if self.bias is not None else None
         vt = self.get_void_tensor()
         if vt.n_blocks == 0:

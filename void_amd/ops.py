@@ -67,14 +67,14 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
     entry = "void_spmm_f32"
     bk = None
     if a.values.dtype == b.dtype and b.dtype in _K16:
-        bk = _runtime.row_major(b)
+        bk = _runtime.row_major(b, a.n_blocks)
         if not _fits16(a, bk, target):
             bk = None
     if bk is not None:
         entry = _K16[b.dtype]
         dbsr = a.device_bsr(b.dtype)
     else:
-        bk = _runtime.row_major(b.to(torch.float32))
+        bk = _runtime.row_major(b.to(torch.float32), a.n_blocks)
         dbsr = a.device_bsr()
     flags = _lib.DENSE_PADDED_B if _runtime.aligned_rows(bk) else 0
     if plan is None:

@@ -89,14 +89,19 @@ def narrow(N: int, n_split_tiles: int) -> bool:
 # row-major copy of B (one pass over it) pays for itself: on the FFN config
 # the SpMM with GELU took 183 us with B column-major against 91 us
 # row-major.  VOID_AMD_BT=0 / 1 forces the copy off / on.
+
+
+# Columns that are not 16-byte aligned (or K not a multiple of 32) leave only
+# single-byte loads (``bytewise``): there the copy always pays (4615 x 646,
+# 554 tiles, N = 1248: 150 -> 19 us).
 COL_MAJOR_COPY_RATIO = 32
 
 
-def copy_col_major_b(n_blocks: int, K: int) -> bool:
+def copy_col_major_b(n_blocks: int, K: int, bytewise: bool = False) -> bool:
     env = os.environ.get("VOID_AMD_BT")
     if env in ("0", "1"):
         return env == "1"
-    return 32 * n_blocks >= COL_MAJOR_COPY_RATIO * max(K, 1)
+    return bytewise or 32 * n_blocks >= COL_MAJOR_COPY_RATIO * max(K, 1)
 
 
 # An 8-bit row-major B whose rows are not 16-byte aligned (N or the row pitch
