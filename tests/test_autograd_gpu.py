@@ -257,7 +257,7 @@ def test_layout_plans_shared_and_streams(gpu):
     torch.cuda.current_stream().wait_stream(side)
     for other in (got, step()):
         assert all(torch.equal(p, q) for p, q in zip(ref, other))
-    assert lay.plans[64] is plan and len(plan.workspaces) == 2
+    assert lay.plans[64] is plan and len(plan.workspaces) == 2 and not plan.capture_spares
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
     with pytest.raises(RuntimeError, match="captured"):
@@ -366,3 +366,41 @@ def test_sddmm_non_finite_follow_fp32(gpu, monkeypatch, bad, grouped):
     assert torch.equal(torch.isnan(a), torch.isnan(r)) and torch.equal(torch.isinf(a), torch.isinf(r))
     ok = torch.isfinite(r).all(dim=2).all(dim=1)
     assert bool(ok.any()) and bool(((a - r)[ok].abs() <= 1e-5 * r[ok].abs().max()).all())
+
+
+def test_layout_cache_eviction(gpu):
+    """More structures than the cache holds, used on two streams in turn."""
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for i in range(70):
+        case = cases.uniform_blocks(64, 96, 40, 1 + i % 5, seed=i)
+        vt = cases.make_void_tensor(case, "cpu").to(gpu)
+        lin = void_amd.SparseLinear(96, 64, vt).to(gpu)
+        x = torch.ones(40, 96, device=gpu)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side if i % 2 else torch.cuda.current_stream()):
+            y = lin(x)
+        torch.cuda.current_stream().wait_stream(side)
+        ref = vt.values.double().sum(2).new_zeros(64)
+        for t, r in enumerate(case.block_rows):
+            ref[32 * r:32 * r + 32] += vt.values[t].double().sum(1)
+        assert bool(((y.double() - ref).abs() <= 1e-4).all()), i
+
+
+def test_linear_output_in_place_and_shapes(gpu):
+    """The output takes in-place operations and 3-D and empty inputs as before."""
+    case = cases.uniform_blocks(64, 96, 40, 4, seed=9)
+    lin = void_amd.SparseLinear(96, 64, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu)
+    x = torch.randn(2, 5, 96, device=gpu, requires_grad=True)
+    y = lin(x)
+    assert y.shape == (2, 5, 64)
+    z = lin(x).relu_()
+    z.sum().backward()
+    got = x.grad.clone()
+    x.grad = None
+    torch.relu(lin(x)).sum().backward()
+    assert torch.equal(z.detach(), torch.relu(y).detach()) and torch.equal(got, x.grad)
+    e = torch.randn(0, 96, device=gpu, requires_grad=True)
+    out = lin(e)
+    out.sum().backward()
+    assert out.shape == (0, 64) and e.grad.shape == (0, 96)

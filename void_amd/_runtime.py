@@ -75,6 +75,7 @@ class DevicePlan:
     capture_spares: Dict[int, torch.Tensor] = field(default_factory=dict)  # nbytes -> zeroed, for the next capture
     capture_by_id: Dict[Tuple[int, int, int], torch.Tensor] = field(default_factory=dict)  # (capture, stream, nbytes)
     ws_sizes: Dict[int, int] = field(default_factory=dict)  # N -> void_workspace_bytes
+    captures: bool = True        # whether a capture may come: keep a zeroed spare workspace for it
     _cplan: Optional["_lib.Plan"] = None
     _cplan_ref: object = None
 
@@ -149,7 +150,7 @@ class DevicePlan:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
             _zero_on_stream(ws[:self.counter_bytes(N)], int(stream), device)
             self.workspaces[key] = ws
-            if nbytes <= MAX_SPARE_WORKSPACE and nbytes not in self.capture_spares:
+            if self.captures and nbytes <= MAX_SPARE_WORKSPACE and nbytes not in self.capture_spares:
                 spare = torch.empty(nbytes, dtype=torch.uint8, device=device)
                 spare[:self.counter_bytes(N)].zero_()
                 # Zeroed before any graph can use it, whatever stream replays it.
@@ -159,8 +160,11 @@ class DevicePlan:
                 # The oldest stream's workspace is freed; the caching allocator
                 # keeps its memory until the work queued on that stream is done.
                 self.workspaces.popitem(last=False)
-        else:
-            self.workspaces.move_to_end(key)
+        elif next(reversed(self.workspaces)) != key:
+            try:
+                self.workspaces.move_to_end(key)
+            except KeyError:  # another thread has just evicted it; ws itself stays alive here
+                pass
         return ws, nbytes
 
 
@@ -285,6 +289,7 @@ class DeviceBsr:
     _desc_ref: object = None
     order: Optional[torch.Tensor] = None  # BSR position -> index of the source tile
     src_key: tuple = ()                   # source_key of the tensors the arrays were gathered from
+    captures: bool = True                 # False where calls are never captured (the differentiable SpMM)
 
     def refresh(self, values: torch.Tensor, scales: torch.Tensor) -> None:
         """Gather the tile values and scales again from their sources into the
@@ -317,7 +322,7 @@ class DeviceBsr:
         if p is None:
             items, n_tiles, n_slots = plan_rows(self.row_ptr_host, chunk, self.col_idx_host)
             dev_items = torch.from_numpy(items).to(self.row_ptr.device)
-            p = DevicePlan(dev_items, items.shape[0], n_tiles, n_slots, chunk, items)
+            p = DevicePlan(dev_items, items.shape[0], n_tiles, n_slots, chunk, items, captures=self.captures)
             self.plans[chunk] = p
         return p
 
@@ -361,7 +366,8 @@ def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torc
                     block_cols: torch.Tensor, shape: Tuple[int, int], tile_size: Tuple[int, int],
                     device: torch.device, per_tensor: bool, layout=None, transpose: bool = False) -> DeviceBsr:
     """Gather the tiles into block-row-major order.  ``layout`` (a BsrLayout
-    of the same block structure) skips the host-side ordering; ``transpose``
+    of the same block structure, as the differentiable SpMM caches) skips the
+    host-side ordering and shares its plans; ``transpose``
     takes every (float) tile transposed, the indices being the result's."""
     if tuple(tile_size) != (32, 32):
         raise NotImplementedError(f"the gfx950 kernels take 32x32 tiles, got {tile_size}")
@@ -385,7 +391,7 @@ def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torc
                      row_ptr_host=lay.row_ptr_host,
                      col_idx_host=lay.col_idx_host if lay.col_idx_host is not None else lay.col_idx.cpu().numpy(),
                      per_tensor=per_tensor, M=M, K=K,
-                     n_blocks=int(values.shape[0]), n_block_rows=n_br, order=lay.order, plans=lay.plans)
+                     n_blocks=int(values.shape[0]), n_block_rows=n_br, order=lay.order, plans=lay.plans, captures=layout is None)
 
 
 def source_key(*tensors: torch.Tensor) -> tuple:

@@ -33,24 +33,15 @@ def _layout(block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int
     key = (_runtime.source_key(block_rows, block_cols), int(block_rows.numel()), tuple(shape),
            str(block_rows.device))
     hit = _LAYOUTS.get(key)
-    stream = _runtime.raw_stream(block_rows.device) if block_rows.is_cuda else 0
     if hit is None:
         n_br, n_bc = (shape[0] + 31) // 32, (shape[1] + 31) // 32
         lay = build_bsr_layout(block_rows, block_cols, n_br, n_bc, block_rows.device)
         if len(_LAYOUTS) > 64:
+            # Any stream's launches may still read the entries' arrays and plans.
+            for dev in {v[1].device for v in _LAYOUTS.values() if v[1].is_cuda}:
+                torch.cuda.synchronize(dev)
             _LAYOUTS.clear()
-        hit = _LAYOUTS[key] = (lay, block_rows, block_cols, stream)
-    elif stream != hit[3]:
-        # The entry's arrays came from another stream's pool and may be
-        # dropped from the cache while this stream's launches still read them.
-        lay = hit[0]
-        cur = torch.cuda.current_stream(block_rows.device)
-        arrays = [lay.order, lay.row_ptr, lay.col_idx] + [p.items for p in lay.plans.values()
-                                                          if isinstance(p, _runtime.DevicePlan)]
-        if lay.sddmm_groups is not None:
-            arrays.append(lay.sddmm_groups)
-        for t in arrays:
-            t.record_stream(cur)
+        hit = _LAYOUTS[key] = (lay, block_rows, block_cols)
     return hit[0]
 
 
