@@ -117,6 +117,9 @@ typedef struct void_plan {
  * on C of the float SpMMs below; b stays 16-byte aligned with ldb a multiple
  * of 16 bytes. */
 #define VOID_DENSE_PADDED_B 2
+/* The product is rounded to out_dtype before the bias is added (and the result
+ * rounded again): the bits of a bias added to a stored C.  Float SpMM only. */
+#define VOID_DENSE_ROUND_BEFORE_BIAS 4
 
 /* The dense operand and the output of one SpMM call. */
 typedef struct void_dense_args {

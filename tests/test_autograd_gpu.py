@@ -283,8 +283,8 @@ def test_gather_tiles_transposed(gpu, dtype, n):
 def test_linear_bias_fused_step(gpu, monkeypatch, dtype, tokens, token_major_grad):
     """SparseLinear on token-major input: output, gradients of input, tiles and
     bias against float64, with either layout of the incoming gradient; a
-    forward hook on the weight module takes the unfused path to the same
-    values within one more rounding."""
+    forward hook on the weight module takes the unfused path to the same bits
+    (the bias's gradient, summed in another order, within its bound)."""
     monkeypatch.setattr(_runtime, "TRANSPOSE_MIN_NUMEL", 1)
     case = cases.uniform_blocks(130, 200, tokens, 20, seed=tokens)
     vt = cases.make_void_tensor(case, "cpu").to(gpu).to_dtype(dtype)
@@ -325,10 +325,70 @@ def test_linear_bias_fused_step(gpu, monkeypatch, dtype, tokens, token_major_gra
             gp[:, :130].abs().sum(0)]
     rnd = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dtype]
     for k, (out, alt, ref, mag) in enumerate(zip(fused, plain, refs, mags)):
-        tol = 300 * U * mag + rnd * ref.abs() + 1e-30
+        # The output rounds twice: the product, at most mag, and the sum.
+        tol = 300 * U * mag + rnd * ref.abs() + (rnd * mag if k == 0 else 0) + 1e-30
         assert bool(((out.double() - ref).abs() <= tol).all()), k
-        # The unfused sum rounds twice.
-        assert bool(((alt.double() - ref).abs() <= tol + rnd * mag).all()), k
+        assert bool(((alt.double() - ref).abs() <= tol).all()), k
+        if k < 3:
+            assert torch.equal(out, alt), k
+
+
+def _linear(gpu, dtype, tokens, seed=3):
+    case = cases.uniform_blocks(130, 200, tokens, 20, seed=seed)
+    lin = void_amd.SparseLinear(200, 130, cases.make_void_tensor(case, "cpu").to(gpu).to_dtype(dtype)).to(gpu)
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    with torch.no_grad():
+        lin.bias.copy_(torch.randn(130, generator=g, device=gpu))
+    return lin, torch.randn(tokens, 200, generator=g, device=gpu).to(dtype)
+
+
+@pytest.mark.parametrize("kernel", ["", "cgd", "f32"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens", [1, 37, 64])
+def test_linear_bias_is_an_addition(gpu, monkeypatch, dtype, tokens, kernel):
+    """y = w(x) + b to the bit: the product is rounded to x's type, then the sum."""
+    if kernel:
+        monkeypatch.setenv("VOID_AMD_KERNEL", kernel)
+    lin, x = _linear(gpu, dtype, tokens)
+    with torch.no_grad():
+        assert lin._bias_in_epilogue(x)
+        assert torch.equal(lin(x), lin.sparse_weight(x.T).T + lin.bias)
+
+
+def test_linear_bias_keeps_autograd(gpu, monkeypatch):
+    """The bias alone: batched gradients, no SpMM in its backward, forward-mode
+    tangents; and a frozen bias or weight."""
+    import torch.autograd.forward_ad as fwd
+    from void_amd import autograd
+    lin, x = _linear(gpu, torch.float32, 12)
+    gy = torch.randn(4, 12, 130, device=gpu)
+    y = lin(x)
+    calls = []
+    monkeypatch.setattr(autograd, "float_spmm", lambda *a, **k: calls.append(a))
+    monkeypatch.setattr(_runtime, "sddmm_tiles", lambda *a, **k: calls.append(a))
+    (one,) = torch.autograd.grad(y, lin.bias, gy[0], retain_graph=True)
+    (many,) = torch.autograd.grad(y, lin.bias, gy, is_grads_batched=True)
+    monkeypatch.undo()
+    assert not calls
+    for got, ref in ((one, gy[0].double().sum(0)), (many, gy.double().sum(1))):
+        assert got.shape == ref.shape and bool(((got.double() - ref).abs() <= 12 * U * gy.abs().sum(1).max()).all())
+    with fwd.dual_level():
+        bias = lin.bias
+        del lin.bias
+        tangent = torch.randn(130, device=gpu)
+        lin.bias = fwd.make_dual(bias.detach(), tangent)
+        with torch.no_grad():
+            lin.sparse_weight.values.requires_grad_(False)
+        assert torch.equal(fwd.unpack_dual(lin(x)).tangent, tangent.expand(12, 130))
+    lin.bias = bias
+    out = lin(x)  # only the bias trains
+    out.backward(gy[0])
+    assert torch.equal(lin.bias.grad, one) and lin.sparse_weight.values.grad is None
+    lin.bias.requires_grad_(False)
+    lin.bias.grad = None
+    lin.sparse_weight.values.requires_grad_(True)
+    lin(x).backward(gy[0])
+    assert lin.bias.grad is None and lin.sparse_weight.values.grad is not None
 
 
 def test_linear_create_graph_bias(gpu):

@@ -19,7 +19,7 @@ NOALLOC_COUNTER_BYTES = 1 << 20
 NOALLOC_PARTIAL_BYTES = 31 << 20
 
 # void_dense_args.flags
-DENSE_ONE_B_SCALE, DENSE_PADDED_B = 1, 2
+DENSE_ONE_B_SCALE, DENSE_PADDED_B, DENSE_ROUND_BEFORE_BIAS = 1, 2, 4
 
 # enum void_epilogue
 EPI_RAW_I32 = 0

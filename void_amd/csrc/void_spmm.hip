@@ -99,6 +99,7 @@ struct Params {
   int32_t item_piles;   // XCDs among which one panel group's items are dealt (see wg_map)
   int32_t xcd_exact;    // grid laid out per XCD (see wg_map)
   int32_t bias_per_row;  // float kernel: bias indexed by output row
+  int32_t round_before_bias;  // float kernel: C rounded to its type before the bias too
   int32_t out_dtype;     // narrow kernel (the others take it as a template argument)
   int32_t pair_snake;    // exact layout: second half of an XCD's share reversed (see wg_map)
 };
@@ -512,6 +513,14 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float x) {
   uint16_t u;
   __builtin_memcpy(&u, &h, 2);
   return u;
+}
+
+// x rounded to the output type, as a float.
+template <int OUT>
+__device__ __forceinline__ float round_out(float x) {
+  if constexpr (OUT == VOID_DT_BF16) return (float)(__bf16)x;
+  else if constexpr (OUT == VOID_DT_F16) return (float)(_Float16)x;
+  else return x;
 }
 
 template <int OUT, bool VEC>
@@ -1918,6 +1927,7 @@ __global__ __launch_bounds__(kThreads * KS) __attribute__((amdgpu_waves_per_eu(
         float x;
         if constexpr (EPI == VOID_EPI_ROW_MEAN || EPI == VOID_EPI_PER_BLOCK) x = __fmul_rn((float)acc[r], mul);
         else x = 0.f;
+        if constexpr (kFloat) x = p.round_before_bias ? round_out<OUT>(x) : x;
         if (p.bias) x = __fadd_rn(x, p.bias_per_row ? row_bias(rr) : bias);
         xv[r] = x;
       }
@@ -1956,6 +1966,7 @@ __global__ __launch_bounds__(kThreads * KS) __attribute__((amdgpu_waves_per_eu(
     if constexpr (EPI == VOID_EPI_ROW_MEAN) x = __fmul_rn((float)acc[r], mul);
     else if constexpr (EPI == VOID_EPI_PER_BLOCK) x = __fmul_rn((float)acc[r], mul);
     else x = 0.f;
+    if constexpr (kFloat) x = p.round_before_bias ? round_out<OUT>(x) : x;
     if (p.bias) x = __fadd_rn(x, p.bias_per_row ? row_bias(rr + 4 * g) : bias);
     x = activate(x, p.activation);
     if (full || (row0 + rr + 4 * g < p.M && col < p.N)) {
@@ -2458,7 +2469,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const float rbias = (p.bias && p.bias_per_row) ? p.bias[min(grow, p.M - 1)] : 0.f;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      float x = sum[i][c];
+      float x = p.round_before_bias ? round_out<OUT>(sum[i][c]) : sum[i][c];
       if (p.bias) x = __fadd_rn(x, p.bias_per_row ? rbias : bias[c]);
       v[c] = activate(x, p.activation);
       vi[c] = 0;
@@ -2558,6 +2569,9 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   if (b_f32 && d->b_col_major) return fail(VOID_ERR_UNSUPPORTED, "an fp32 B must be row-major");
   if (d->bias_per_row && !unscaled)
     return fail(VOID_ERR_UNSUPPORTED, "a per-row bias is supported by the float SpMM only");
+  const bool round_before_bias = (d->flags & VOID_DENSE_ROUND_BEFORE_BIAS) != 0;
+  if (round_before_bias && !unscaled)
+    return fail(VOID_ERR_UNSUPPORTED, "C is rounded before the bias by the float SpMM only");
   if (b_f32 && plan->chunk_tiles > 64)
     return fail(VOID_ERR_ARG, "an fp32 B takes work items of at most 64 tiles (chunk_tiles %d)", plan->chunk_tiles);
   if (d->activation < VOID_ACT_NONE || d->activation > VOID_ACT_SILU)
@@ -2621,6 +2635,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     }
   }
   p.bias_per_row = d->bias_per_row;
+  p.round_before_bias = round_before_bias;
   p.out_dtype = d->out_dtype;
   p.items = items;
   p.trace = g_trace;

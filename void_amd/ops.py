@@ -29,11 +29,12 @@ def _fits16(a, b: torch.Tensor, c: torch.Tensor) -> bool:
 
 
 def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
-               activation: int = _lib.ACT_NONE, bias_per_row: bool = False,
+               activation: int = _lib.ACT_NONE, bias_per_row: bool = False, round_before_bias: bool = False,
                plan: Optional["_runtime.DevicePlan"] = None) -> torch.Tensor:
     """activation(A @ B + bias) for a float VOIDTensor A; the output has B's
     dtype (f32, bf16 or f16), as the reference's kernels write.  bias is [N]
-    (per column), or [M] with bias_per_row (fusion.py:202-304).  ``plan``
+    (per column), or [M] with bias_per_row (fusion.py:202-304);
+    round_before_bias gives the bits of a bias added to the stored product.  ``plan``
     (work items of at most 64 tiles) replaces the default partition."""
     if b.dim() != 2:
         raise ValueError("B must be 2-D")
@@ -77,6 +78,8 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
         bk = _runtime.row_major(b.to(torch.float32), a.n_blocks)
         dbsr = a.device_bsr()
     flags = _lib.DENSE_PADDED_B if _runtime.aligned_rows(bk) else 0
+    if round_before_bias:
+        flags |= _lib.DENSE_ROUND_BEFORE_BIAS
     if plan is None:
         plan = dbsr.plan(F32_CHUNK)
     elif plan.chunk > F32_CHUNK:
