@@ -464,3 +464,32 @@ def test_linear_output_in_place_and_shapes(gpu):
     out = lin(e)
     out.sum().backward()
     assert out.shape == (0, 64) and e.grad.shape == (0, 96)
+
+
+@pytest.mark.parametrize("grouped", ["tiles", "grouped", "rows"])
+@pytest.mark.parametrize("terms", [1, 2, 64])
+@pytest.mark.parametrize("kind", ["normal", "constant", "tiny", "tinier"])
+def test_sddmm_precision(gpu, monkeypatch, kind, terms, grouped):
+    """fp32 products keep all 24 bits: one rounding for one term, n for n, also
+    for operands far below one (still normal numbers) and for equal operands,
+    whose errors would all have one sign."""
+    from void_amd.format import build_bsr_layout
+    monkeypatch.setenv("VOID_AMD_SDDMM", grouped)
+    rng = np.random.default_rng(terms)
+    N = max(terms, 4)
+    case = cases.uniform_blocks(128, 192, N, 16, seed=4)
+    G, B = rng.standard_normal((128, N)), rng.standard_normal((192, N))
+    if kind == "constant":
+        G[:], B[:] = (1 + 2.0 ** -7 - 2.0 ** -16,) * 2
+    elif kind != "normal":
+        G *= 2.0 ** (-118 if kind == "tiny" else -122)
+        B *= 2.0 ** 100
+    G, B = G.astype(np.float32), B.astype(np.float32)
+    G[:, terms:] = 0
+    rows, cols = torch.from_numpy(case.block_rows).to(gpu), torch.from_numpy(case.block_cols).to(gpu)
+    lay = build_bsr_layout(rows, cols, 4, 6, gpu)
+    got = _runtime.sddmm_tiles(torch.from_numpy(G).to(gpu), torch.from_numpy(B).to(gpu), rows, cols, (128, 192),
+                               torch.float32, layout=lay).double().cpu().numpy()
+    for t, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+        x, y = G[32 * r:32 * r + 32].astype(np.float64), B[32 * c:32 * c + 32].astype(np.float64)
+        assert np.all(np.abs(got[t] - x @ y.T) <= terms * U * (np.abs(x) @ np.abs(y).T)), t

@@ -25,7 +25,6 @@
 
 #include "void_amd.h"
 #include "lds_dma.h"
-#include "split_bf16.h"
 
 extern "C" __attribute__((visibility("hidden"))) int void_internal_fail(int code, const char* msg);
 
@@ -398,7 +397,7 @@ __global__ __launch_bounds__(64 * kRW) void sddmm_ring_kernel(
   int rd[kHalf];
 #pragma unroll
   for (int q = 0; q < kHalf; ++q) rd[q] = i * (kCW4 * 4) + (((kHalf * g + q) ^ Geo::swz(i)) << 4);
-  v16f acc = {}, acc_small = {};  // fp32: acc_small holds the corrections of split_bf16.h
+  v16f acc = {};
 #pragma unroll
   for (int k = 0; k < kRing - 1; ++k)
     if (k < n_chunks) issue(k);
@@ -417,15 +416,10 @@ __global__ __launch_bounds__(64 * kRW) void sddmm_ring_kernel(
         y[q] = *reinterpret_cast<const v4f*>(st + yoff + rd[q]);
       }
       if constexpr (IN == VOID_DT_F32) {
-        float xf[4 * kHalf], yf[4 * kHalf];
 #pragma unroll
         for (int q = 0; q < kHalf; ++q)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            xf[4 * q + e] = x[q][e];
-            yf[4 * q + e] = y[q][e];
-          }
-        mfma_split3(split3<kHalf / 2>(xf), split3<kHalf / 2>(yf), acc, acc_small);
+          for (int s2 = 0; s2 < 4; ++s2) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[q][s2], y[q][s2], acc, 0, 0, 0);
       } else if constexpr (IN == VOID_DT_BF16) {
 #pragma unroll
         for (int q = 0; q < kHalf; ++q)
@@ -440,26 +434,6 @@ __global__ __launch_bounds__(64 * kRW) void sddmm_ring_kernel(
     }
   }
   if (!has) return;
-  if constexpr (IN == VOID_DT_F32) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] += acc_small[r];
-    if (any_nonfinite(acc)) {
-      // Infinities, NaN or overflow: this tile again on the fp32 MFMA, straight
-      // from memory, in the order of the loop above.  Rows past M or K count
-      // as zero, as do columns past N (N is a multiple of 4 here).
-      acc = v16f{};
-      const int gr = br * kT + i, br2 = bc * kT + i;
-      const float* xr = static_cast<const float*>(dC) + (int64_t)min(gr, M - 1) * ldg;
-      const float* yr = static_cast<const float*>(B) + (int64_t)min(br2, K - 1) * ldb;
-      for (int n0 = 0; n0 < N; n0 += kCW)
-#pragma unroll
-        for (int s2 = 0; s2 < kCW / 2; ++s2) {
-          const int n = n0 + kCW / 2 * g + s2;
-          const float xv = xr[min(n, N - 1)], yv = yr[min(n, N - 1)];
-          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(n < N && gr < M ? xv : 0.f, n < N && br2 < K ? yv : 0.f, acc, 0, 0, 0);
-        }
-    }
-  }
   // Lane (j, g), register r: tile row 8 (r / 4) + 4 g + r % 4, column j.
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
