@@ -87,3 +87,35 @@ def test_fp8_float_b_beyond_2gib(gpu):
         ref[32 * br[t]:32 * br[t] + 32] += sc[t] * (codes[t][:, :k1 - k0] @ bt)
         bound[32 * br[t]:32 * br[t] + 32] += abs(sc[t]) * (np.abs(codes[t][:, :k1 - k0]) @ np.abs(bt))
     assert np.all(np.abs(out.cpu().numpy() - ref) <= 2.0 ** -13 * bound + 1e-6)
+
+
+@pytest.mark.parametrize("case", ["near_limit", "view_of_b", "view_of_out"])
+def test_fp8_float_b_at_the_offset_limit(gpu, case):
+    """E4M3 x fp32 B with N % 4 != 0 at the edge of the ring's 31-bit offsets:
+    a B just under 2 GiB, a narrow view of a 2 GiB B, a narrow view of a 2 GiB
+    output.  Products of two bf16 parts: within 2^-13 of sum |a b|."""
+    rng = np.random.default_rng(7)
+    M, K = (8192, 128) if case == "view_of_out" else (64, 8192)
+    N = 65510 if case == "near_limit" else 37
+    br, bc = np.array([0, 0, 1, 1]), np.array([0, 3, 1, K // 32 - 1])
+    tiles = rng.standard_normal((4, 32, 32)).astype(np.float32)
+    vt = void_amd.VOIDTensor(
+        values=torch.from_numpy(tiles), block_rows=torch.from_numpy(br.astype(np.int32)),
+        block_cols=torch.from_numpy(bc.astype(np.int32)), morton_codes=torch.zeros(4, dtype=torch.int64),
+        shape=(M, K), tile_size=(32, 32), nnz_original=4096, n_blocks=4, density=0.0)
+    a = void_amd.void_tensor_to_fp8(vt.to(gpu))
+    g = torch.Generator(device=gpu).manual_seed(3)
+    wide = torch.randn(K, 65536 if case == "view_of_b" else N, device=gpu, generator=g)
+    b = wide[:, :N]
+    out = torch.empty(M, 65536, device=gpu)[:, :N] if case == "view_of_out" else None
+    got = void_amd.void_spmm_fp8(a, b, torch.float32, out=out)
+    assert out is None or got is out
+    scale = a.scaling_info.scale.double()
+    ref = torch.zeros(M, N, dtype=torch.float64, device=gpu)
+    mag = torch.zeros_like(ref)
+    for t in range(4):
+        q = a.values_fp8[t].float().double() * scale[t]
+        bt = b[32 * bc[t]:32 * bc[t] + 32].double()
+        ref[32 * br[t]:32 * br[t] + 32] += q @ bt
+        mag[32 * br[t]:32 * br[t] + 32] += q.abs() @ bt.abs()
+    assert bool(((got.double() - ref).abs() <= 2.0 ** -13 * mag + 1e-30).all())

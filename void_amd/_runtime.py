@@ -468,21 +468,48 @@ def aligned_rows(t: torch.Tensor) -> bool:
     return s1 == 1 and s0 >= t.shape[1] and s0 * t.element_size() % 16 == 0 and t.data_ptr() % 16 == 0
 
 
-def padded_rows(t: torch.Tensor, zero_tail: bool = False) -> torch.Tensor:
+RING_LIMIT = 1 << 31  # the ring kernels' byte offsets are 31-bit
+
+
+def padded_layout(R: int, C: int, s0: int, s1: int, ptr: int, esz: int, zero_tail: bool = False,
+                  limit: Optional[int] = None) -> Optional[Tuple[bool, int]]:
+    """How padded_rows gives an R x C operand of esz-byte elements at ptr with
+    strides s0, s1 its rows: (in place?, row pitch in elements), or None where
+    R rounded up to whole tiles at that pitch reaches ``limit`` bytes.  The
+    pitch of a copy is whole 128-byte lines (16-byte chunks up to one line, or
+    where only those stay below the limit)."""
+    per = 16 // esz
+    fits = lambda ld: limit is None or -(-R // 32) * 32 * ld * esz < limit
+    if (s1 == 1 and s0 >= C and s0 % per == 0 and ptr % 16 == 0 and not (zero_tail and C % per) and fits(s0)):
+        return True, s0
+    chunks = -(-C // per) * per
+    lines = -(-C // (8 * per)) * 8 * per if C > 8 * per else chunks
+    for pitch in (lines, chunks):
+        if fits(pitch):
+            return False, pitch
+    return None
+
+
+def padded_rows(t: torch.Tensor, zero_tail: bool = False, limit: Optional[int] = None) -> torch.Tensor:
     """A 2-D 16- or 32-bit GPU tensor as aligned_rows: t itself where it is,
-    else a copy whose pitch is a multiple of 16 bytes (of a 128-byte line from
-    there on) and whose rows are zero from their end to the next multiple of
-    16 bytes.  With zero_tail, t itself only if its rows end on one."""
+    else a copy whose rows are zero from their end to the next multiple of 16
+    bytes, as padded_layout says (which finds a layout under ``limit``, or the
+    caller has asked it before).  With zero_tail, t itself only if its rows end
+    on a multiple of 16 bytes."""
     R, C = t.shape
-    per = 16 // t.element_size()
-    s0, s1 = t.stride()
-    if not t.numel() or (aligned_rows(t) and not (zero_tail and C % per)):
+    if not t.numel():
         return t
-    line = 8 * per
-    pitch = -(-C // line) * line if C > line else -(-C // per) * per
+    esz = t.element_size()
+    per = 16 // esz
+    s0, s1 = t.stride()
+    lay = padded_layout(R, C, s0, s1, t.data_ptr(), esz, zero_tail, limit)
+    if lay is None:
+        raise ValueError(f"{R} padded rows of {C} {t.dtype} values reach {limit} bytes")
+    in_place, pitch = lay
+    if in_place:
+        return t
     if s1 == 1 and s0 >= C and R * -(-C // per) < 1 << 31:
         out = torch.empty(R, pitch, dtype=t.dtype, device=t.device)[:, :C]
-        esz = t.element_size()
         st = _lib.lib().void_copy_rows_b8(t.data_ptr(), s0 * esz, R, C * esz, out.data_ptr(), pitch * esz,
                                           raw_stream(t.device))
         _lib.check(st, "void_copy_rows_b8")
@@ -492,8 +519,7 @@ def padded_rows(t: torch.Tensor, zero_tail: bool = False) -> torch.Tensor:
         buf[:, C:-(-C // per) * per].zero_()
     out = buf[:, :C]
     if s0 == 1 and s1 >= R and t.numel() >= TRANSPOSE_MIN_NUMEL and max(R, C) <= 64 * 65535:
-        st = _lib.lib().void_transpose(t.data_ptr(), s1, C, R, out.data_ptr(), pitch, t.element_size(),
-                                       raw_stream(t.device))
+        st = _lib.lib().void_transpose(t.data_ptr(), s1, C, R, out.data_ptr(), pitch, esz, raw_stream(t.device))
         _lib.check(st, "void_transpose")
     else:
         out.copy_(t)

@@ -312,27 +312,28 @@ def void_spmm_fp8(a: FP8VOIDTensor, b: torch.Tensor, output_dtype: torch.dtype =
     for n0 in range(0, N, width):
         n1 = min(N, n0 + width)
         whole = n0 == 0 and n1 == N
-        _launch_f32b(dbsr, b if whole else b[:, n0:n1], out if whole else None, output_dtype, scalar_scale,
+        _launch_f32b(dbsr, b if whole else b[:, n0:n1], out[:, n0:n1], scalar_scale,
                      None if scale_vec is None else scale_vec[n0:n1], act, None if bias is None else bias[n0:n1],
-                     chunk, dst=out[:, n0:n1])
+                     chunk)
     return out
 
 
-def _launch_f32b(dbsr, b: torch.Tensor, out: Optional[torch.Tensor], output_dtype: torch.dtype, scalar_scale: float,
-                 scale_vec: Optional[torch.Tensor], act: int, bias: Optional[torch.Tensor], chunk: int,
-                 dst: torch.Tensor) -> None:
-    """One E4M3 x fp32-B launch over B's columns, written to dst.  out, when
-    given, is dst itself and takes the result directly."""
-    M, N = dst.shape[0], b.shape[1]
+def _launch_f32b(dbsr, b: torch.Tensor, out: torch.Tensor, scalar_scale: float, scale_vec: Optional[torch.Tensor],
+                 act: int, bias: Optional[torch.Tensor], chunk: int) -> None:
+    """One E4M3 x fp32-B launch over columns that fit the kernel's 31-bit
+    offsets as a compact B and C: a wider B is copied to a pitch that fits, a
+    wider out written by way of a compact one."""
+    M, N = out.shape
     b32 = b.to(torch.float32)
-    b32 = _runtime.contiguous_2d(b32) if N % 4 == 0 else _runtime.padded_rows(b32)
+    b32 = _runtime.contiguous_2d(b32) if N % 4 == 0 else _runtime.padded_rows(b32, limit=_runtime.RING_LIMIT)
     if b32.data_ptr() % 16:
         b32 = b32.clone()
-    tgt = out if out is not None else torch.empty(M, N, dtype=output_dtype, device=b.device)
+    direct = out.stride(1) == 1 and M * out.stride(0) * out.element_size() < _runtime.RING_LIMIT
+    tgt = out if direct else torch.empty(M, N, dtype=out.dtype, device=b.device)
     _runtime.launch("fp8_f32b", dbsr, b32, b_scale=scalar_scale, b_scale_vec=scale_vec, flags=_lib.DENSE_PADDED_B,
                     out=tgt, epilogue=_lib.EPI_PER_BLOCK, activation=act, bias=bias, chunk=chunk)
-    if out is None:
-        dst.copy_(tgt)
+    if tgt is not out:
+        out.copy_(tgt)
 
 
 def void_tensor_to_fp8(void_tensor, format: str = "e4m3", scale_mode: str = "per_block") -> FP8VOIDTensor:
