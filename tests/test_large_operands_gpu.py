@@ -119,3 +119,28 @@ def test_fp8_float_b_at_the_offset_limit(gpu, case):
         ref[32 * br[t]:32 * br[t] + 32] += q @ bt
         mag[32 * br[t]:32 * br[t] + 32] += q.abs() @ bt.abs()
     assert bool(((got.double() - ref).abs() <= 2.0 ** -13 * mag + 1e-30).all())
+
+
+def test_float_b_beyond_2gib_is_not_padded(gpu):
+    """A bf16 B that no ring can address (16384 x 65537, 2.1 GB): widened for
+    the fp32 kernel, and copied no further.  Within fp32 summation and one
+    rounding to bf16."""
+    K, N = 16384, 65537
+    g = torch.Generator(device=gpu).manual_seed(4)
+    br, bc = [0, 0, 1, 1], [0, 300, 5, K // 32 - 1]
+    tiles = torch.randn(4, 32, 32, device=gpu, generator=g).bfloat16()
+    a = void_amd.VOIDTensor(
+        values=tiles, block_rows=torch.tensor(br, dtype=torch.int32, device=gpu),
+        block_cols=torch.tensor(bc, dtype=torch.int32, device=gpu), morton_codes=torch.zeros(4, dtype=torch.int64),
+        shape=(64, K), tile_size=(32, 32), nnz_original=4096, n_blocks=4, density=0.0, dtype=torch.bfloat16)
+    b = torch.empty(K, N, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    out = void_amd.void_spmm(a, b)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - base < 2.2 * b.numel() * 2
+    for r in range(2):
+        ref = sum(tiles[t].double() @ b[32 * bc[t]:32 * bc[t] + 32].double() for t in range(4) if br[t] == r)
+        mag = sum(tiles[t].double().abs() @ b[32 * bc[t]:32 * bc[t] + 32].double().abs() for t in range(4) if br[t] == r)
+        err = (out[32 * r:32 * r + 32].double() - ref).abs()
+        assert bool((err <= 64 * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs()).all())

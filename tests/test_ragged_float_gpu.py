@@ -20,6 +20,7 @@ ABS = {torch.float32: 0.0, torch.bfloat16: 0.0, torch.float16: 2.0 ** -25}
 @pytest.fixture(autouse=True)
 def always_pad(monkeypatch):
     monkeypatch.setattr(_runtime, "PAD_FLOAT_MIN_WORK", 1)
+    monkeypatch.setenv("VOID_AMD_PAD", "1")
 
 
 def _views(b):
@@ -129,3 +130,43 @@ def test_small_widths_keep_one_launch(gpu, monkeypatch):
     assert _runtime.row_major(b, 60) is b
     out = _runtime.row_major(b, 600)
     assert _runtime.aligned_rows(out) and torch.equal(out, b)
+
+
+@pytest.mark.parametrize("kind", ["int8", "int8_col", "float"])
+def test_tall_b_is_read_in_place(gpu, monkeypatch, kind):
+    """Few tiles over a tall B: nothing of B's size is allocated, and the
+    result is right (int32 exact, fp32 within its summation bound)."""
+    monkeypatch.undo()
+    K, N, n = 1 << 20, 101, 40
+    rng = np.random.default_rng(1)
+    br, bc = np.arange(n) % 16, rng.choice(K // 32, n, replace=False)
+    vt = void_amd.VOIDTensor(
+        values=torch.from_numpy(rng.standard_normal((n, 32, 32)).astype(np.float32)).to(gpu),
+        block_rows=torch.from_numpy(br.astype(np.int32)).to(gpu), block_cols=torch.from_numpy(bc.astype(np.int32)).to(gpu),
+        morton_codes=torch.zeros(n, dtype=torch.int64, device=gpu), shape=(512, K), tile_size=(32, 32),
+        nnz_original=n * 1024, n_blocks=n, density=0.0)
+    if kind == "float":
+        a, b = vt, torch.randn(K, N, device=gpu)
+        run = lambda: void_amd.void_spmm(a, b)
+        tiles = vt.values.double()
+    else:
+        a = void_amd.quantize_void_tensor(vt)
+        b = torch.randint(-128, 128, (K, N), dtype=torch.int8, device=gpu)
+        if kind == "int8_col":
+            b = torch.cat([b.t().contiguous(), b.t()[:, :1].contiguous()], 1)[:, :K].t()  # columns of K + 1 bytes
+        run = lambda: void_amd.void_spmm_int8(a, b, epilogue="raw_i32")
+        tiles = a.values.double()
+    run()
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    out = run()
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - base < b.numel() * b.element_size() // 8
+    ref = torch.zeros(512, N, dtype=torch.float64, device=gpu)
+    mag = torch.zeros_like(ref)
+    for t in range(n):
+        bt = b[32 * bc[t]:32 * bc[t] + 32].double()
+        ref[32 * br[t]:32 * br[t] + 32] += tiles[t] @ bt
+        mag[32 * br[t]:32 * br[t] + 32] += tiles[t].abs() @ bt.abs()
+    assert bool(((out.double() - ref).abs() <= (96 * U * mag if kind == "float" else 0)).all())

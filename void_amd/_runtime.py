@@ -526,31 +526,46 @@ def padded_rows(t: torch.Tensor, zero_tail: bool = False, limit: Optional[int] =
     return out
 
 
-# A float B (or gradient) whose rows are not 16-byte aligned is copied to
-# padded rows for the LDS-DMA rings where the tiles times the width reach this
-# (eager calls: 1638 tiles, N = 15 bf16 23.0 -> 19.2 us; 200 tiles, N = 257 bf16
-# 29.7 -> 19.8; 1638 tiles, N = 730 bf16 87 -> 19, fp32 80 -> 39; bf16 training
-# step of 4096 x 4096, 1001 tokens 802 -> 334).  Below, the element-wise fp32
-# kernels' single launch takes no longer (60 tiles, N = 130: bf16 18.3 against
-# 20.0 us with the copy, fp32 15.1 against 18.5).
-PAD_FLOAT_MIN_WORK = 1 << 14
+PAD_FLOAT_MIN_WORK = tuning.PAD_FLOAT_MIN_WORK
 
 
-def pad_float(n_blocks: int, N: int) -> bool:
-    return n_blocks * N >= PAD_FLOAT_MIN_WORK
+def _pad_forced(n_blocks: int, N: int) -> Optional[bool]:
+    """What VOID_AMD_PAD or a small call decides about padded rows, else None."""
+    forced = tuning._forced("VOID_AMD_PAD")
+    if forced is None and n_blocks * N < PAD_FLOAT_MIN_WORK:
+        return False
+    return forced
 
 
-def row_major(t: torch.Tensor, n_blocks: int) -> torch.Tensor:
-    """t (2-D) row-major for the float kernels on n_blocks tiles: in place with
-    aligned rows, a padded copy where pad_float says so, else contiguous."""
+def ring_rows(t: torch.Tensor, n_blocks: int, a=None, zero_tail: bool = False) -> Optional[torch.Tensor]:
+    """t (2-D) with aligned rows that the float rings address, in place or
+    copied, or None where a copy does not pay (for the VOIDTensor a) or every
+    pitch reaches the rings' limit."""
     esz = t.element_size()
-    if t.is_cuda and esz in (2, 4):
-        if aligned_rows(t):
-            return t
-        N = t.shape[1]
-        if N * esz % 16 and pad_float(n_blocks, N):
-            return padded_rows(t)
-    return contiguous_2d(t)
+    if not t.is_cuda or esz not in (2, 4) or not t.numel():
+        return None
+    K, N = t.shape
+    s0, s1 = t.stride()
+    lay = padded_layout(K, N, s0, s1, t.data_ptr(), esz, zero_tail, RING_LIMIT)
+    if lay is None:
+        return None
+    in_place, pitch = lay
+    if in_place:
+        return t
+    if N * esz % 16 == 0:
+        t = contiguous_2d(t)
+        return t if aligned_rows(t) else None
+    pad = _pad_forced(n_blocks, N)
+    if pad is None:
+        pad = a is None or tuning.pad_float_b(n_blocks, a.longest_row(), K, N, pitch, esz, t.is_contiguous())
+    return padded_rows(t, zero_tail, RING_LIMIT) if pad else None
+
+
+def row_major(t: torch.Tensor, n_blocks: int, a=None) -> torch.Tensor:
+    """t (2-D) row-major for the float kernels on n_blocks tiles: as ring_rows
+    gives it, else contiguous."""
+    r = ring_rows(t, n_blocks, a)
+    return contiguous_2d(t) if r is None else r
 
 
 def aligned_copy_b8(b: torch.Tensor, ld: int) -> torch.Tensor:
@@ -576,19 +591,25 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
     plan = dbsr.plan(chunk)
     short = chunk <= tuning.FP32_B_MAX_CHUNK  # items the narrow and column-group kernels take
     panels8 = kind in ("int8", "fp8") and not (short and tuning.narrow(N, plan.n_split_tiles))
-    if col_major and panels8 and N and tuning.copy_col_major_b(
-            dbsr.n_blocks, dbsr.K, bytewise=short and bool(ldb % 16 or dbsr.K % 32 or b_t.data_ptr() % 16)):
-        b_t, col_major = row_major_copy_b8(b_t, ldb), False  # for the LDS-DMA ring
-        ldb = max(b_t.stride(0), N)
     target = out
     so0, so1 = out.stride()
     if so1 != 1 or so0 < N:
         target = torch.empty(out.shape, dtype=out.dtype, device=out.device)
-    if panels8 and short and N and not col_major and (ldb % 16 or b_t.data_ptr() % 16):
-        dword = ((N | ldb | b_t.data_ptr() | target.stride(0)) % 4 == 0) and target.data_ptr() % 16 == 0
-        if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword):
-            b_t = aligned_copy_b8(b_t, ldb)
-            ldb = b_t.stride(0)
+    if panels8 and N and (col_major or ldb % 16 or b_t.data_ptr() % 16):
+        # Copies for the LDS-DMA ring, where its offsets reach every operand.
+        ring = (short and dbsr.n_blocks << 10 < RING_LIMIT
+                and out.shape[0] * target.stride(0) * target.element_size() < RING_LIMIT
+                and -(-dbsr.K // 32) * 32 * tuning.aligned_pitch(N) < RING_LIMIT)
+        if col_major:
+            bytewise = ring and bool(ldb % 16 or dbsr.K % 32 or b_t.data_ptr() % 16)
+            if tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K, bytewise, N, min(dbsr.max_row, chunk)):
+                b_t, col_major = row_major_copy_b8(b_t, ldb), False
+                ldb = max(b_t.stride(0), N)
+        if ring and not col_major and (ldb % 16 or b_t.data_ptr() % 16):
+            dword = ((N | ldb | b_t.data_ptr() | target.stride(0)) % 4 == 0) and target.data_ptr() % 16 == 0
+            if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword, min(dbsr.max_row, chunk)):
+                b_t = aligned_copy_b8(b_t, ldb)
+                ldb = b_t.stride(0)
     stream = raw_stream(out.device)
     ws, ws_bytes = plan.workspace(N, out.device, stream)
     # Fields in the struct's order.
@@ -703,9 +724,22 @@ def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor,
     if N == 0:
         return out.zero_()
     stream = raw_stream(grad_c.device)
-    pad = pad_float(n, N)
     entry16 = {torch.bfloat16: "void_sddmm_rows_bf16", torch.float16: "void_sddmm_rows_f16"}.get(grad_c.dtype)
-    if layout is not None and entry16 is not None and b.dtype == grad_c.dtype and (N % 8 == 0 or pad):
+
+
+    def pad(g, bb):
+        """Whether g (unless it is grad_padded's) and bb get padded rows."""
+        forced = _pad_forced(n, N)
+        if forced is not None:
+            return forced
+        copied = []
+        for t in (bb,) if grad_padded and g is grad_c else (g, bb):
+            lay = padded_layout(*t.shape, *t.stride(), t.data_ptr(), t.element_size(), zero_tail=True)
+            copied.append((t.shape[0], lay[1], t.is_contiguous()))
+        return tuning.pad_float_sddmm(n, N, g.element_size(), copied)
+
+    if (layout is not None and entry16 is not None and b.dtype == grad_c.dtype
+            and (N % 8 == 0 or pad(grad_c, b))):
         # 16-bit operands of one dtype on the 16-bit MFMA (16-byte rows).
         if N % 8 == 0:
             g16 = grad_c if grad_c.stride(1) == 1 else contiguous_2d(grad_c)
@@ -723,7 +757,7 @@ def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor,
             _lib.check(st, entry16)
             return out
     g, bb = grad_c.to(torch.float32), b.to(torch.float32)
-    if N % 4 and pad:
+    if N % 4 and pad(g, bb):
         g = g if grad_padded and g is grad_c else padded_rows(g, zero_tail=True)
         bb = padded_rows(bb, zero_tail=True)
         N = -(-N // 4) * 4

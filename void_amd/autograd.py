@@ -96,13 +96,16 @@ class VOIDSpMMFunction(Function):
         M, K = ctx.a_shape
         grad_a = grad_b = None
         # One row-major copy of a token-major gradient serves both products
-        # (rows of whole 16-byte chunks where the kernels would copy it to such).
-        N, per = grad_output.shape[1], 16 // max(grad_output.element_size(), 1)
-        padded = (N % per != 0 and _runtime.pad_float(ctx.a_n_blocks, N) and grad_output.is_cuda
-                  and grad_output.element_size() in (2, 4))
-        grad = _runtime.padded_rows(grad_output, zero_tail=True) if padded else _runtime.contiguous_2d(grad_output)
+        # (rows of whole 16-byte chunks where the SpMM would copy it to such).
+        grad, padded, at = grad_output, False, None
         if ctx.needs_input_grad[6]:
             at = _vt(a_values.detach(), cols, rows, (K, M), ctx.a_tile_size[::-1], ctx.a_n_blocks, cls=_TransposedTiles)
+            if grad_output.shape[1] * grad_output.element_size() % 16 and ctx.a_n_blocks:
+                grad = _runtime.ring_rows(grad_output, ctx.a_n_blocks, at, zero_tail=True)
+                padded = grad is not None
+        if not padded:
+            grad = _runtime.contiguous_2d(grad_output)
+        if at is not None:
             grad_b = float_spmm(at, grad).to(b.dtype)
             if b.stride(0) == 1 and b.stride(1) >= K > 1:
                 # A column-major B (X.t() of token-major activations) gets a

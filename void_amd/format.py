@@ -69,6 +69,14 @@ class BsrLayout:
     # device copy of tiles with this layout shares them.
     plans: dict = field(default_factory=dict)
     sddmm_groups: Optional[torch.Tensor] = None  # int32 [n_groups, 3], built on first use
+    _max_row: Optional[int] = None
+
+    @property
+    def max_row(self) -> int:
+        """Tiles in the longest block-row (the structure is fixed: computed once)."""
+        if self._max_row is None:
+            self._max_row = int(np.diff(self.row_ptr_host).max(initial=0))
+        return self._max_row
 
     def row_groups(self) -> torch.Tensor:
         """(block row, first BSR position, count <= 8) per group of a row's tiles,
@@ -153,6 +161,14 @@ class VOIDTensor:
             d.refresh(self.values.detach().to(dtype).contiguous(), d.scales)
             d.src_key = src
         return d
+
+    def longest_row(self) -> int:
+        """Tiles in the longest block-row."""
+        for d in self._device_bsr.values():
+            return d.max_row
+        if self._bsr_layout is not None:
+            return self._bsr_layout.max_row
+        return int(np.bincount(self.block_rows.detach().cpu().numpy()).max(initial=0))
 
     @property
     def padded_shape(self) -> Tuple[int, int]:

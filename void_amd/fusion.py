@@ -131,11 +131,9 @@ def void_spmm_silu(a, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
 def _void_spmm_activation_row_bias(a, b: torch.Tensor, bias: Optional[torch.Tensor], out: Optional[torch.Tensor],
                                    activation: str) -> torch.Tensor:
     """activation(A @ B + bias[:, None]) with a per-row bias [M] for float A
-    (fusion.py:307-377): the fp32 kernel with bias_per_row, output in B's dtype;
-    B is made row-major as the reference does."""
+    (fusion.py:307-377): the fp32 kernel with bias_per_row, output in B's dtype."""
     if not isinstance(a, VOIDTensor):
         raise TypeError("the row-bias activation SpMM takes a float VOIDTensor")
-    b = _runtime.row_major(b, a.n_blocks)
     if a.n_blocks == 0:
         res = torch.zeros(a.shape[0], b.shape[1], dtype=b.dtype, device=b.device) if out is None else out.zero_()
         if bias is not None:
@@ -202,7 +200,7 @@ class FusedSparseLinear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x_flat = x.reshape(-1, self.in_features)
-        b = _runtime.row_major(x_flat.t(), self.n_blocks)  # [in, batch], as the reference passes it
+        b = x_flat.t()  # [in, batch]
         bias = self.bias.detach() if self.bias is not None else None
         vt = self.get_void_tensor()
         if vt.n_blocks == 0:

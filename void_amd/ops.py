@@ -19,13 +19,10 @@ F32_CHUNK = 64
 _K16 = {torch.bfloat16: "void_spmm_bf16", torch.float16: "void_spmm_f16"}
 
 
-def _fits16(a, b: torch.Tensor, c: torch.Tensor) -> bool:
-    """What void_spmm_bf16 / void_spmm_f16 take: row-major B with 16-byte
-    aligned rows, and operands within 31-bit offsets."""
-    M, K = a.shape
-    lim = 1 << 31
-    return (_runtime.aligned_rows(b) and a.n_blocks * 2048 < lim and ((K + 31) // 32) * 32 * b.stride(0) * 2 < lim and
-            M * c.stride(0) * c.element_size() < lim)
+def _rings_reach(a, c: torch.Tensor, tile_bytes: int) -> bool:
+    """Whether the rings' 31-bit offsets reach A's tiles and all of C."""
+    return (a.n_blocks * tile_bytes < _runtime.RING_LIMIT
+            and a.shape[0] * c.stride(0) * c.element_size() < _runtime.RING_LIMIT)
 
 
 def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
@@ -67,15 +64,16 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
     # kernel, whose products of widened 16-bit values are the same numbers.
     entry = "void_spmm_f32"
     bk = None
-    if a.values.dtype == b.dtype and b.dtype in _K16:
-        bk = _runtime.row_major(b, a.n_blocks)
-        if not _fits16(a, bk, target):
-            bk = None
+    if a.values.dtype == b.dtype and b.dtype in _K16 and _rings_reach(a, target, 2048):
+        bk = _runtime.ring_rows(b, a.n_blocks, a)
     if bk is not None:
         entry = _K16[b.dtype]
         dbsr = a.device_bsr(b.dtype)
     else:
-        bk = _runtime.row_major(b.to(torch.float32), a.n_blocks)
+        wide = b.to(torch.float32)
+        bk = _runtime.ring_rows(wide, a.n_blocks, a) if _rings_reach(a, target, 4096) else None
+        if bk is None:
+            bk = _runtime.contiguous_2d(wide)
         dbsr = a.device_bsr()
     flags = _lib.DENSE_PADDED_B if _runtime.aligned_rows(bk) else 0
     if round_before_bias:
