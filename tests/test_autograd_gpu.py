@@ -493,3 +493,46 @@ def test_sddmm_precision(gpu, monkeypatch, kind, terms, grouped):
     for t, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
         x, y = G[32 * r:32 * r + 32].astype(np.float64), B[32 * c:32 * c + 32].astype(np.float64)
         assert np.all(np.abs(got[t] - x @ y.T) <= terms * U * (np.abs(x) @ np.abs(y).T)), t
+
+
+def test_layout_cache_threads_and_streams(gpu):
+    """Two threads on streams of their own, each with more structures than the
+    cache holds: dropped layouts' memory is recorded on both streams, and every
+    result is right.  Outputs are checked at the end, without waits between."""
+    import threading
+    from void_amd import autograd
+    done, errors = [], []
+
+    def work(k):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for i in range(90):
+                    case = cases.uniform_blocks(96, 160, 24, 3 + (i + k) % 9, seed=1000 * k + i)
+                    vt = cases.make_void_tensor(case, "cpu").to(gpu)
+                    lin = void_amd.SparseLinear(160, 96, vt).to(gpu)
+                    x = torch.randn(24, 160, device=gpu, requires_grad=True)
+                    gy = torch.randn(24, 96, device=gpu)
+                    y = lin(x)
+                    y.backward(gy)
+                    done.append((case, vt, x, gy, y.detach(), x.grad))
+                    assert stream.cuda_stream in autograd._layout(
+                        lin.sparse_weight.block_rows, lin.sparse_weight.block_cols, lin.sparse_weight.shape).streams
+            stream.synchronize()
+        except Exception as e:  # reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    torch.cuda.synchronize()
+    assert len(done) == 180
+    for case, vt, x, gy, y, gx in done:
+        W = torch.zeros(96, 160, dtype=torch.float64, device=gpu)
+        for t, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+            W[32 * r:32 * r + 32, 32 * c:32 * c + 32] = vt.values[t].double()
+        for got, l, m in ((y, x.detach().double(), W.t()), (gx, gy.double(), W)):
+            assert bool(((got.double() - l @ m).abs() <= 160 * U * (l.abs() @ m.abs()) + 1e-30).all())

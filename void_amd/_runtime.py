@@ -44,6 +44,19 @@ def raw_stream(device: torch.device) -> int:
                                               else torch.cuda.current_device())
 
 
+def record_once(seen: set, device: torch.device, *arrays: torch.Tensor) -> None:
+    """Record GPU arrays on the current stream, once for each stream (seen: the
+    raw streams so far).  The allocator then gives their memory out again only
+    when what was queued on these streams before they were freed is done; a
+    caller between this and its launch still holds them, so its launch is
+    queued before.  (record_stream lasts until the array is freed.)"""
+    raw = raw_stream(device)
+    if raw not in seen:
+        for t in arrays:
+            t.record_stream(torch.cuda.current_stream(device))
+        seen.add(raw)
+
+
 _DEVICE_KEYS: Dict[torch.device, str] = {}
 
 
@@ -76,6 +89,8 @@ class DevicePlan:
     capture_by_id: Dict[Tuple[int, int, int], torch.Tensor] = field(default_factory=dict)  # (capture, stream, nbytes)
     ws_sizes: Dict[int, int] = field(default_factory=dict)  # N -> void_workspace_bytes
     captures: bool = True        # whether a capture may come: keep a zeroed spare workspace for it
+    streams: set = field(default_factory=set)  # raw streams that items is recorded on (shared plans)
+    _last_key: Optional[tuple] = None  # the workspace used last (most recent in workspaces)
     _cplan: Optional["_lib.Plan"] = None
     _cplan_ref: object = None
 
@@ -160,11 +175,12 @@ class DevicePlan:
                 # The oldest stream's workspace is freed; the caching allocator
                 # keeps its memory until the work queued on that stream is done.
                 self.workspaces.popitem(last=False)
-        elif next(reversed(self.workspaces)) != key:
+        elif self._last_key != key:
             try:
                 self.workspaces.move_to_end(key)
             except KeyError:  # another thread has just evicted it; ws itself stays alive here
                 pass
+        self._last_key = key
         return ws, nbytes
 
 
@@ -324,6 +340,8 @@ class DeviceBsr:
             dev_items = torch.from_numpy(items).to(self.row_ptr.device)
             p = DevicePlan(dev_items, items.shape[0], n_tiles, n_slots, chunk, items, captures=self.captures)
             self.plans[chunk] = p
+        if not self.captures:  # shared through a cached layout, which may drop it
+            record_once(p.streams, self.row_ptr.device, p.items)
         return p
 
     def desc(self) -> _lib.BsrDesc:
@@ -375,6 +393,8 @@ def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torc
     n_br = (M + 31) // 32
     n_bc = (K + 31) // 32
     lay = layout if layout is not None else build_bsr_layout(block_rows, block_cols, n_br, n_bc, device)
+    if layout is not None and device.type == "cuda":
+        layout.on_stream()
     v = values.to(device)
     if transpose and v.shape[0]:
         tiles = gather_tiles_t(v, lay.order)
@@ -391,7 +411,8 @@ def make_device_bsr(values: torch.Tensor, scales: torch.Tensor, block_rows: torc
                      row_ptr_host=lay.row_ptr_host,
                      col_idx_host=lay.col_idx_host if lay.col_idx_host is not None else lay.col_idx.cpu().numpy(),
                      per_tensor=per_tensor, M=M, K=K,
-                     n_blocks=int(values.shape[0]), n_block_rows=n_br, order=lay.order, plans=lay.plans, captures=layout is None)
+                     n_blocks=int(values.shape[0]), n_block_rows=n_br, order=lay.order, plans=lay.plans,
+                     captures=layout is None)
 
 
 def source_key(*tensors: torch.Tensor) -> tuple:
@@ -724,6 +745,8 @@ def sddmm_tiles(grad_c: torch.Tensor, b: torch.Tensor, block_rows: torch.Tensor,
     if N == 0:
         return out.zero_()
     stream = raw_stream(grad_c.device)
+    if layout is not None:
+        layout.on_stream()
     entry16 = {torch.bfloat16: "void_sddmm_rows_bf16", torch.float16: "void_sddmm_rows_f16"}.get(grad_c.dtype)
 
 

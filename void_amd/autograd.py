@@ -14,6 +14,7 @@ plans nor waits for the device (4096 x 4096, 3277 tiles, fp32, 1024 tokens:
 
 from __future__ import annotations
 
+import threading
 from typing import Any, Optional, Tuple
 
 import torch
@@ -24,31 +25,32 @@ from .format import VOIDTensor, build_bsr_layout
 from .ops import float_spmm
 
 _LAYOUTS: dict = {}
+_LOCK = threading.RLock()
 
 
 def _layout(block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int, int]):
     # Keyed on the structure tensors' identity and in-place version; each
     # entry holds the tensors themselves, so their memory cannot be handed
     # to other structure tensors (same address, version 0) while cached.
+    # A dropped entry's device arrays go back to the allocator, which waits for
+    # the streams that they were recorded on (BsrLayout.on_stream).
     key = (_runtime.source_key(block_rows, block_cols), int(block_rows.numel()), tuple(shape),
            str(block_rows.device))
-    hit = _LAYOUTS.get(key)
-    if hit is None:
-        n_br, n_bc = (shape[0] + 31) // 32, (shape[1] + 31) // 32
-        lay = build_bsr_layout(block_rows, block_cols, n_br, n_bc, block_rows.device)
-        if len(_LAYOUTS) > 64:
-            # Any stream's launches may still read the entries' arrays and plans.
-            for dev in {v[1].device for v in _LAYOUTS.values() if v[1].is_cuda}:
-                torch.cuda.synchronize(dev)
-            _LAYOUTS.clear()
-        hit = _LAYOUTS[key] = (lay, block_rows, block_cols)
+    with _LOCK:
+        hit = _LAYOUTS.get(key)
+        if hit is None:
+            n_br, n_bc = (shape[0] + 31) // 32, (shape[1] + 31) // 32
+            lay = build_bsr_layout(block_rows, block_cols, n_br, n_bc, block_rows.device)
+            if len(_LAYOUTS) > 64:
+                _LAYOUTS.clear()
+            hit = _LAYOUTS[key] = (lay, block_rows, block_cols)
     return hit[0]
 
 
 def _vt(values, block_rows, block_cols, shape, tile_size, n_blocks, cls=VOIDTensor) -> VOIDTensor:
     vt = cls(values=values, block_rows=block_rows, block_cols=block_cols,
-                    morton_codes=torch.empty(0, dtype=torch.int64, device=values.device), shape=tuple(shape),
-                    tile_size=tuple(tile_size), nnz_original=0, n_blocks=n_blocks, density=0.0, dtype=values.dtype)
+             morton_codes=torch.empty(0, dtype=torch.int64, device=values.device), shape=tuple(shape),
+             tile_size=tuple(tile_size), nnz_original=0, n_blocks=n_blocks, density=0.0, dtype=values.dtype)
     if n_blocks and values.is_cuda:
         if torch.cuda.is_current_stream_capturing():
             # The cached layout and its plans may be dropped while the graph lives.

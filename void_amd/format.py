@@ -70,6 +70,14 @@ class BsrLayout:
     plans: dict = field(default_factory=dict)
     sddmm_groups: Optional[torch.Tensor] = None  # int32 [n_groups, 3], built on first use
     _max_row: Optional[int] = None
+    streams: set = field(default_factory=set)        # raw streams that the arrays are recorded on
+    group_streams: set = field(default_factory=set)  # the same for sddmm_groups
+
+    def on_stream(self) -> None:
+        """The arrays are about to be used on the current stream: where a cache
+        drops this layout, their memory is not handed out before that work is done."""
+        from . import _runtime
+        _runtime.record_once(self.streams, self.row_ptr.device, self.order, self.row_ptr, self.col_idx)
 
     @property
     def max_row(self) -> int:
@@ -91,6 +99,9 @@ class BsrLayout:
             cnt = np.minimum(8, rp[rows + 1] - start)
             arr = np.stack([rows, start, cnt], axis=1).astype(np.int32).reshape(-1, 3)
             self.sddmm_groups = torch.from_numpy(arr).to(self.row_ptr.device)
+        if self.row_ptr.is_cuda:
+            from . import _runtime
+            _runtime.record_once(self.group_streams, self.row_ptr.device, self.sddmm_groups)
         return self.sddmm_groups
 
 
