@@ -536,3 +536,28 @@ def test_layout_cache_threads_and_streams(gpu):
             W[32 * r:32 * r + 32, 32 * c:32 * c + 32] = vt.values[t].double()
         for got, l, m in ((y, x.detach().double(), W.t()), (gx, gy.double(), W)):
             assert bool(((got.double() - l @ m).abs() <= 160 * U * (l.abs() @ m.abs()) + 1e-30).all())
+
+
+def test_many_layers_plan_once(gpu, monkeypatch):
+    """Two steps of more layers than the list of recent structures is long: the
+    second orders, plans and uploads nothing."""
+    from void_amd import autograd
+    layers = []
+    for i in range(autograd.MAX_RECENT + 16):
+        case = cases.uniform_blocks(96, 96, 8, 4, seed=i)
+        layers.append(void_amd.SparseLinear(96, 96, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu))
+    x = torch.randn(8, 96, device=gpu, requires_grad=True)
+    calls = []
+
+    def step():
+        y = x
+        for lin in layers:
+            y = lin(y) + y
+        y.sum().backward()
+
+    step()
+    for mod, name in ((autograd, "build_bsr_layout"), (_runtime, "build_bsr_layout"), (_runtime, "plan_rows")):
+        fn = getattr(mod, name)
+        monkeypatch.setattr(mod, name, lambda *a, fn=fn, name=name, **k: calls.append(name) or fn(*a, **k))
+    step()
+    assert not calls

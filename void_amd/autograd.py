@@ -6,7 +6,7 @@ Forward: C = A @ B on the fp32 kernel (void_spmm_f32).  Backward:
   dL/dA_values = dL/dC @ B^T on the nonzero tiles only, the SDDMM kernel
                  void_sddmm_f32 (autograd.py:191-215).
 The block structure's device ordering is computed once per structure and
-reused across steps, together with its Stream-K plans; only the tile values
+kept with the module, together with its Stream-K plans; only the tile values
 are regathered, since an optimiser updates them in place.  A step neither
 plans nor waits for the device (4096 x 4096, 3277 tiles, fp32, 1024 tokens:
 545 us a step when each built its plans anew, 335 us since).
@@ -15,6 +15,8 @@ plans nor waits for the device (4096 x 4096, 3277 tiles, fp32, 1024 tokens:
 from __future__ import annotations
 
 import threading
+import weakref
+from collections import OrderedDict
 from typing import Any, Optional, Tuple
 
 import torch
@@ -24,41 +26,80 @@ from . import _runtime
 from .format import VOIDTensor, build_bsr_layout
 from .ops import float_spmm
 
-_LAYOUTS: dict = {}
+class _Structure:
+    """The block-row order of a tile set (forward, SDDMM) and of its transpose
+    (gradient of B), with the plans that live in them."""
+
+    def __init__(self, key: tuple, block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int, int]):
+        self.key, self.rows, self.cols, self.shape = key, block_rows, block_cols, tuple(shape)
+        self.layout = self._build(block_rows, block_cols, *self.shape)
+        self._transposed = None
+
+    @staticmethod
+    def _build(rows, cols, M, K):
+        return build_bsr_layout(rows, cols, (M + 31) // 32, (K + 31) // 32, rows.device)
+
+    @property
+    def transposed(self):
+        if self._transposed is None:
+            with _LOCK:
+                if self._transposed is None:
+                    self._transposed = self._build(self.cols, self.rows, *self.shape[::-1])
+        return self._transposed
+
+
+# A structure lives as long as the module that used it last (_OWNED), a forward
+# whose backward is still to come (ctx), or among the last MAX_RECENT used
+# (VOIDSpMMFunction called on bare tensors); _ALIVE finds it.  Its key is the
+# structure tensors' identity and in-place version; it holds the tensors
+# themselves, so their memory cannot be handed to other structure tensors
+# (same address, version 0) while it lives.  Its device arrays go back to the
+# allocator, which waits for the streams they were recorded on
+# (BsrLayout.on_stream).
+MAX_RECENT = 64
+_ALIVE: "weakref.WeakValueDictionary[tuple, _Structure]" = weakref.WeakValueDictionary()
+_OWNED: "weakref.WeakKeyDictionary[torch.nn.Module, _Structure]" = weakref.WeakKeyDictionary()
+_RECENT: "OrderedDict[tuple, _Structure]" = OrderedDict()
 _LOCK = threading.RLock()
 
 
-def _layout(block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int, int]):
-    # Keyed on the structure tensors' identity and in-place version; each
-    # entry holds the tensors themselves, so their memory cannot be handed
-    # to other structure tensors (same address, version 0) while cached.
-    # A dropped entry's device arrays go back to the allocator, which waits for
-    # the streams that they were recorded on (BsrLayout.on_stream).
-    key = (_runtime.source_key(block_rows, block_cols), int(block_rows.numel()), tuple(shape),
-           str(block_rows.device))
+def _structure(block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int, int],
+               owner: Optional[torch.nn.Module] = None) -> _Structure:
+    key = (_runtime.source_key(block_rows, block_cols), block_rows.numel(), block_rows.stride(), block_cols.stride(),
+           block_rows.dtype, block_cols.dtype, tuple(shape), block_rows.device)
+    if owner is not None:
+        s = _OWNED.get(owner)
+        if s is not None and s.key == key:
+            return s
     with _LOCK:
-        hit = _LAYOUTS.get(key)
-        if hit is None:
-            n_br, n_bc = (shape[0] + 31) // 32, (shape[1] + 31) // 32
-            lay = build_bsr_layout(block_rows, block_cols, n_br, n_bc, block_rows.device)
-            if len(_LAYOUTS) > 64:
-                _LAYOUTS.clear()
-            hit = _LAYOUTS[key] = (lay, block_rows, block_cols)
-    return hit[0]
+        s = _ALIVE.get(key)
+        if s is None:
+            s = _ALIVE[key] = _Structure(key, block_rows, block_cols, shape)
+        if owner is not None:
+            _OWNED[owner] = s
+        else:
+            _RECENT[key] = s
+            _RECENT.move_to_end(key)
+            while len(_RECENT) > MAX_RECENT:
+                _RECENT.popitem(last=False)
+    return s
 
 
-def _vt(values, block_rows, block_cols, shape, tile_size, n_blocks, cls=VOIDTensor) -> VOIDTensor:
-    vt = cls(values=values, block_rows=block_rows, block_cols=block_cols,
-             morton_codes=torch.empty(0, dtype=torch.int64, device=values.device), shape=tuple(shape),
-             tile_size=tuple(tile_size), nnz_original=0, n_blocks=n_blocks, density=0.0, dtype=values.dtype)
-    if n_blocks and values.is_cuda:
-        if torch.cuda.is_current_stream_capturing():
-            # The cached layout and its plans may be dropped while the graph lives.
-            raise RuntimeError("the differentiable SpMM cannot be captured in a HIP graph; capture void_spmm instead")
-        # The device copy (fp32 or 16-bit, as the SpMM needs) is built on
-        # first use from this cached block-row order.
-        vt._bsr_layout = _layout(block_rows, block_cols, vt.shape)
-    return vt
+def _layout(block_rows: torch.Tensor, block_cols: torch.Tensor, shape: Tuple[int, int]):
+    """The block-row order of a tile set, with its plans."""
+    return _structure(block_rows, block_cols, shape).layout
+
+
+def _vt(values, block_rows, block_cols, shape, tile_size, n_blocks, layout=None, cls=VOIDTensor) -> VOIDTensor:
+    """The tiles as a VOIDTensor whose device copy (fp32 or 16-bit, as the SpMM
+    needs) is built on first use in a layout's order."""
+    if layout is not None and torch.cuda.is_current_stream_capturing():
+        # The layout and its plans may be dropped while the graph lives.
+        raise RuntimeError("the differentiable SpMM cannot be captured in a HIP graph; capture void_spmm instead")
+    return cls(values=values, block_rows=block_rows, block_cols=block_cols,
+               morton_codes=torch.empty(0, dtype=torch.int64, device=values.device), shape=tuple(shape),
+               tile_size=tuple(tile_size), nnz_original=0, n_blocks=n_blocks, density=0.0, dtype=values.dtype,
+               _bsr_layout=layout)
 
 
 class _TransposedTiles(VOIDTensor):
@@ -83,11 +124,16 @@ class VOIDSpMMFunction(Function):
     """C = A @ B with gradients for the tile values and for B (autograd.py:99-216)."""
 
     @staticmethod
-    def forward(ctx: Any, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b, row_bias=None):
+    def forward(ctx: Any, a_values, a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks, b, row_bias=None,
+                owner=None):
         # row_bias [M]: added to C's rows as a constant (SparseLinear gives it
-        # its gradient with _RowBias).
-        c = float_spmm(_vt(a_values.detach(), a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks), b,
-                       bias=row_bias, bias_per_row=row_bias is not None, round_before_bias=row_bias is not None)
+        # its gradient with _RowBias); owner: the module that keeps the structure.
+        ctx.structure = None
+        if a_n_blocks and a_values.is_cuda:
+            ctx.structure = _structure(a_block_rows, a_block_cols, a_shape, owner)
+        vt = _vt(a_values.detach(), a_block_rows, a_block_cols, a_shape, a_tile_size, a_n_blocks,
+                 ctx.structure and ctx.structure.layout)
+        c = float_spmm(vt, b, bias=row_bias, bias_per_row=row_bias is not None, round_before_bias=row_bias is not None)
         ctx.save_for_backward(a_values, a_block_rows, a_block_cols, b)
         ctx.a_shape, ctx.a_tile_size, ctx.a_n_blocks = tuple(a_shape), tuple(a_tile_size), a_n_blocks
         return c
@@ -101,7 +147,8 @@ class VOIDSpMMFunction(Function):
         # (rows of whole 16-byte chunks where the SpMM would copy it to such).
         grad, padded, at = grad_output, False, None
         if ctx.needs_input_grad[6]:
-            at = _vt(a_values.detach(), cols, rows, (K, M), ctx.a_tile_size[::-1], ctx.a_n_blocks, cls=_TransposedTiles)
+            at = _vt(a_values.detach(), cols, rows, (K, M), ctx.a_tile_size[::-1], ctx.a_n_blocks,
+                     ctx.structure and ctx.structure.transposed, cls=_TransposedTiles)
             if grad_output.shape[1] * grad_output.element_size() % 16 and ctx.a_n_blocks:
                 grad = _runtime.ring_rows(grad_output, ctx.a_n_blocks, at, zero_tail=True)
                 padded = grad is not None
@@ -115,9 +162,8 @@ class VOIDSpMMFunction(Function):
                 grad_b = _runtime.contiguous_2d(grad_b.t()).t()
         if ctx.needs_input_grad[0]:
             grad_a = _runtime.sddmm_tiles(grad, b, rows, cols, (M, K), a_values.dtype,
-                                          layout=_layout(rows, cols, (M, K)) if rows.is_cuda else None,
-                                          grad_padded=padded)
-        return grad_a, None, None, None, None, None, grad_b, None
+                                          layout=ctx.structure and ctx.structure.layout, grad_padded=padded)
+        return grad_a, None, None, None, None, None, grad_b, None, None
 
 
 class _RowBias(Function):
@@ -159,7 +205,7 @@ class VOIDSpMM(torch.nn.Module):
         if squeeze:
             x = x.unsqueeze(1)
         y = VOIDSpMMFunction.apply(self.values, self.block_rows, self.block_cols, self.shape, self.tile_size,
-                                   self.n_blocks, x)
+                                   self.n_blocks, x, None, self)
         return y.squeeze(1) if squeeze else y
 
     def get_void_tensor(self) -> VOIDTensor:
@@ -207,7 +253,7 @@ class SparseLinear(torch.nn.Module):
         w, bias = self.sparse_weight, self.bias
         if bias is not None and self._bias_in_epilogue(x):
             y = VOIDSpMMFunction.apply(w.values, w.block_rows, w.block_cols, w.shape, w.tile_size, w.n_blocks,
-                                       x_flat.T, bias.detach())
+                                       x_flat.T, bias.detach(), w)
             if bias.requires_grad and torch.is_grad_enabled():
                 y = _RowBias.apply(y, bias)
             y = y.T
