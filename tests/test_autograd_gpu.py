@@ -561,3 +561,40 @@ def test_many_layers_plan_once(gpu, monkeypatch):
         monkeypatch.setattr(mod, name, lambda *a, fn=fn, name=name, **k: calls.append(name) or fn(*a, **k))
     step()
     assert not calls
+
+
+def test_split_layers_share_one_workspace(gpu):
+    """Layers whose plans split rows, of several sizes and widths in turn on one
+    stream: one buffer in all, and every step repeats the first one's bits."""
+    rng = np.random.default_rng(0)
+    layers = []
+    for i, (M, K) in enumerate([(96, 4096), (4096, 64), (160, 6000), (64, 8192)]):
+        case = cases.uniform_blocks(M, K, 8, (M // 32) * (K // 32) * 3 // 4, seed=i)
+        layers.append(void_amd.SparseLinear(K, M, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu))
+    ins = [(lin, torch.from_numpy(rng.standard_normal((n, lin.in_features)).astype(np.float32)).to(gpu))
+           for n in (40, 300, 7) for lin in layers]
+
+    def step():
+        out = []
+        for lin, x in ins:
+            x = x.clone().requires_grad_()
+            y = lin(x)
+            y.backward(torch.ones_like(y))
+            out += [y.detach(), x.grad]
+        return out
+
+    _runtime.STEP_WORKSPACES.buffers.clear()
+    ref = step()
+    held = _runtime.STEP_WORKSPACES.buffers
+    assert len(held) == 1
+    for _ in range(3):
+        assert all(torch.equal(p, q) for p, q in zip(ref, step()))
+    assert len(held) == 1 and sum(b.numel() for b, _ in held.values()) <= _runtime.MAX_SPARE_WORKSPACE
+    for (lin, x), y in zip(ins, ref[::2]):
+        w = lin.sparse_weight
+        W = torch.zeros(-(-lin.out_features // 32) * 32, -(-lin.in_features // 32) * 32, dtype=torch.float64, device=gpu)
+        for t, (r, c) in enumerate(zip(w.block_rows.tolist(), w.block_cols.tolist())):
+            W[32 * r:32 * r + 32, 32 * c:32 * c + 32] = w.values[t].detach().double()
+        W = W[:lin.out_features, :lin.in_features]
+        mag = x.double().abs() @ W.abs().t()
+        assert bool(((y.double() - x.double() @ W.t()).abs() <= lin.in_features * U * mag + 1e-30).all())

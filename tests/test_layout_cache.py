@@ -126,3 +126,23 @@ def test_modules_copy_and_pickle():
     for other in (copy.deepcopy(lin), torch.load(buf, weights_only=False)):
         assert torch.equal(other.sparse_weight.values, lin.sparse_weight.values)
         assert other.sparse_weight not in autograd._OWNED
+
+
+def test_stream_workspaces(monkeypatch):
+    """Plans of one stream share a buffer: counters are zero on entry whatever
+    the plan before wrote as partials; large ones are not kept; streams are bounded."""
+    monkeypatch.setattr(_runtime, "_zero_on_stream", lambda t, s, d: t.zero_())
+    monkeypatch.setattr(_runtime, "MAX_SPARE_WORKSPACE", 1 << 16)
+    pool, dev = _runtime.StreamWorkspaces(), torch.device("cpu")
+    g = torch.Generator().manual_seed(0)
+    for _ in range(200):
+        counters = 256 * int(torch.randint(1, 9, (1,), generator=g))
+        nbytes = counters + 256 * int(torch.randint(1, 300, (1,), generator=g))
+        ws = pool.take(counters, nbytes, dev, int(torch.randint(0, 3, (1,), generator=g)))
+        assert ws.numel() >= nbytes and not ws[:counters].any()
+        ws[counters:nbytes] = 1  # a launch writes its partials and leaves the counters at zero
+        assert all(b.numel() <= 1 << 16 for b, _ in pool.buffers.values())
+    assert len(pool.buffers) == 3
+    for stream in range(20):
+        pool.take(256, 1024, dev, stream)
+    assert list(pool.buffers) == [(dev, s) for s in range(12, 20)]

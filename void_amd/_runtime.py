@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from dataclasses import dataclass, field
 from collections import OrderedDict
 from typing import Dict, List, Optional, Tuple
@@ -75,6 +76,47 @@ def vector_f32(t: torch.Tensor, device: torch.device) -> torch.Tensor:
     return t.reshape(-1).to(device=device, dtype=torch.float32).contiguous()
 
 
+class StreamWorkspaces:
+    """One split-row workspace for each HIP stream, for all plans of the
+    differentiable SpMM: their launches on one stream run in order, so they can
+    share it however many layers there are.
+
+    A buffer holds a region of arrival counters, zero between launches, then
+    the partial blocks.  A call takes the region's last counter bytes, so that
+    every plan's partials start behind every plan's counters.  Buffers of more
+    than MAX_SPARE_WORKSPACE are made for one call; the last
+    MAX_STREAM_WORKSPACES streams' are kept."""
+
+    def __init__(self) -> None:
+        self.buffers: "OrderedDict[tuple, Tuple[torch.Tensor, int]]" = OrderedDict()  # -> (buffer, region bytes)
+        self._lock = threading.Lock()
+
+    def take(self, counters: int, nbytes: int, device: torch.device, stream: int) -> torch.Tensor:
+        """A workspace of nbytes, its first ``counters`` bytes zero, for a launch on the stream."""
+        partials = nbytes - counters
+        key = (device, stream)
+        with self._lock:
+            buf, region = self.buffers.get(key, (None, 0))
+            if buf is None or region < counters or buf.numel() - region < partials:
+                old = 0 if buf is None else buf.numel() - region
+                region, size = max(region, counters), max(old, partials)
+                if region + size > MAX_SPARE_WORKSPACE:
+                    region, size = counters, partials
+                # A smaller buffer's memory goes back in stream order.
+                buf = torch.empty(region + size, dtype=torch.uint8, device=device)
+                _zero_on_stream(buf[:region], stream, device)
+                if region + size <= MAX_SPARE_WORKSPACE:
+                    self.buffers[key] = buf, region
+            if key in self.buffers:
+                self.buffers.move_to_end(key)
+            while len(self.buffers) > MAX_STREAM_WORKSPACES:
+                self.buffers.popitem(last=False)
+        return buf[region - counters:]
+
+
+STEP_WORKSPACES = StreamWorkspaces()
+
+
 @dataclass
 class DevicePlan:
     items: torch.Tensor          # int32 [n_items, 32] on device (void_work_item)
@@ -88,7 +130,7 @@ class DevicePlan:
     capture_spares: Dict[int, torch.Tensor] = field(default_factory=dict)  # nbytes -> zeroed, for the next capture
     capture_by_id: Dict[Tuple[int, int, int], torch.Tensor] = field(default_factory=dict)  # (capture, stream, nbytes)
     ws_sizes: Dict[int, int] = field(default_factory=dict)  # N -> void_workspace_bytes
-    captures: bool = True        # whether a capture may come: keep a zeroed spare workspace for it
+    captures: bool = True        # False for the differentiable SpMM's (never captured): workspaces are STEP_WORKSPACES'
     streams: set = field(default_factory=set)  # raw streams that items is recorded on (shared plans)
     _last_key: Optional[tuple] = None  # the workspace used last (most recent in workspaces)
     _cplan: Optional["_lib.Plan"] = None
@@ -157,6 +199,8 @@ class DevicePlan:
             return ws, nbytes
         if stream is None:
             stream = torch.cuda.current_stream(device).cuda_stream
+        if not self.captures:
+            return STEP_WORKSPACES.take(self.counter_bytes(N), nbytes, device, int(stream)), nbytes
         key = (nbytes, int(stream))
         ws = self.workspaces.get(key)
         if ws is None:
@@ -165,7 +209,7 @@ class DevicePlan:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
             _zero_on_stream(ws[:self.counter_bytes(N)], int(stream), device)
             self.workspaces[key] = ws
-            if self.captures and nbytes <= MAX_SPARE_WORKSPACE and nbytes not in self.capture_spares:
+            if nbytes <= MAX_SPARE_WORKSPACE and nbytes not in self.capture_spares:
                 spare = torch.empty(nbytes, dtype=torch.uint8, device=device)
                 spare[:self.counter_bytes(N)].zero_()
                 # Zeroed before any graph can use it, whatever stream replays it.
@@ -339,6 +383,8 @@ class DeviceBsr:
             items, n_tiles, n_slots = plan_rows(self.row_ptr_host, chunk, self.col_idx_host)
             dev_items = torch.from_numpy(items).to(self.row_ptr.device)
             p = DevicePlan(dev_items, items.shape[0], n_tiles, n_slots, chunk, items, captures=self.captures)
+            if not self.captures:
+                p.workspaces = STEP_WORKSPACES.buffers
             self.plans[chunk] = p
         if not self.captures:  # shared through a cached layout, which may drop it
             record_once(p.streams, self.row_ptr.device, p.items)
