@@ -11,7 +11,7 @@ import torch
 import cases
 import oracle
 import void_amd
-from void_amd import _runtime
+from void_amd import _runtime, autograd
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
@@ -233,7 +233,6 @@ def test_inference_mode(gpu):
 def test_layout_plans_shared_and_streams(gpu):
     """One structure's plans serve every step, also from a second stream, with
     bit-identical results; capture is refused as before."""
-    from void_amd import autograd
     case = cases.uniform_blocks(256, 4096, 96, 700, seed=5)  # rows beyond 64 tiles: split plans
     vt = cases.make_void_tensor(case, "cpu").to(gpu)
     mod = void_amd.VOIDSpMM(vt)
@@ -286,6 +285,7 @@ def test_linear_bias_fused_step(gpu, monkeypatch, dtype, tokens, token_major_gra
     forward hook on the weight module takes the unfused path to the same bits
     (the bias's gradient, summed in another order, within its bound)."""
     monkeypatch.setattr(_runtime, "TRANSPOSE_MIN_NUMEL", 1)
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
     case = cases.uniform_blocks(130, 200, tokens, 20, seed=tokens)
     vt = cases.make_void_tensor(case, "cpu").to(gpu).to_dtype(dtype)
     lin = void_amd.SparseLinear(200, 130, vt).to(gpu)
@@ -347,6 +347,7 @@ def _linear(gpu, dtype, tokens, seed=3):
 @pytest.mark.parametrize("tokens", [1, 37, 64])
 def test_linear_bias_is_an_addition(gpu, monkeypatch, dtype, tokens, kernel):
     """y = w(x) + b to the bit: the product is rounded to x's type, then the sum."""
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
     if kernel:
         monkeypatch.setenv("VOID_AMD_KERNEL", kernel)
     lin, x = _linear(gpu, dtype, tokens)
@@ -359,16 +360,16 @@ def test_linear_bias_keeps_autograd(gpu, monkeypatch):
     """The bias alone: batched gradients, no SpMM in its backward, forward-mode
     tangents; and a frozen bias or weight."""
     import torch.autograd.forward_ad as fwd
-    from void_amd import autograd
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
     lin, x = _linear(gpu, torch.float32, 12)
     gy = torch.randn(4, 12, 130, device=gpu)
     y = lin(x)
     calls = []
-    monkeypatch.setattr(autograd, "float_spmm", lambda *a, **k: calls.append(a))
-    monkeypatch.setattr(_runtime, "sddmm_tiles", lambda *a, **k: calls.append(a))
-    (one,) = torch.autograd.grad(y, lin.bias, gy[0], retain_graph=True)
-    (many,) = torch.autograd.grad(y, lin.bias, gy, is_grads_batched=True)
-    monkeypatch.undo()
+    with monkeypatch.context() as m:
+        m.setattr(autograd, "float_spmm", lambda *a, **k: calls.append(a))
+        m.setattr(_runtime, "sddmm_tiles", lambda *a, **k: calls.append(a))
+        (one,) = torch.autograd.grad(y, lin.bias, gy[0], retain_graph=True)
+        (many,) = torch.autograd.grad(y, lin.bias, gy, is_grads_batched=True)
     assert not calls
     for got, ref in ((one, gy[0].double().sum(0)), (many, gy.double().sum(1))):
         assert got.shape == ref.shape and bool(((got.double() - ref).abs() <= 12 * U * gy.abs().sum(1).max()).all())
@@ -391,8 +392,9 @@ def test_linear_bias_keeps_autograd(gpu, monkeypatch):
     assert lin.bias.grad is None and lin.sparse_weight.values.grad is not None
 
 
-def test_linear_create_graph_bias(gpu):
+def test_linear_create_graph_bias(gpu, monkeypatch):
     """With create_graph the bias gradient stays differentiable in the output gradient."""
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
     case = cases.uniform_blocks(64, 64, 5, 3, seed=2)
     lin = void_amd.SparseLinear(64, 64, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu)
     x = torch.randn(5, 64, device=gpu)
@@ -447,8 +449,11 @@ def test_layout_cache_eviction(gpu):
         assert bool(((y.double() - ref).abs() <= 1e-4).all()), i
 
 
-def test_linear_output_in_place_and_shapes(gpu):
-    """The output takes in-place operations and 3-D and empty inputs as before."""
+@pytest.mark.parametrize("least", [0, 1 << 60])
+def test_linear_output_in_place_and_shapes(gpu, monkeypatch, least):
+    """The output takes in-place operations and 3-D and empty inputs as before,
+    with the bias in the epilogue and as an addition."""
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", least)
     case = cases.uniform_blocks(64, 96, 40, 4, seed=9)
     lin = void_amd.SparseLinear(96, 64, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu)
     x = torch.randn(2, 5, 96, device=gpu, requires_grad=True)
@@ -500,7 +505,6 @@ def test_layout_cache_threads_and_streams(gpu):
     cache holds: dropped layouts' memory is recorded on both streams, and every
     result is right.  Outputs are checked at the end, without waits between."""
     import threading
-    from void_amd import autograd
     done, errors = [], []
 
     def work(k):
@@ -541,7 +545,6 @@ def test_layout_cache_threads_and_streams(gpu):
 def test_many_layers_plan_once(gpu, monkeypatch):
     """Two steps of more layers than the list of recent structures is long: the
     second orders, plans and uploads nothing."""
-    from void_amd import autograd
     layers = []
     for i in range(autograd.MAX_RECENT + 16):
         case = cases.uniform_blocks(96, 96, 8, 4, seed=i)

@@ -664,17 +664,20 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
         target = torch.empty(out.shape, dtype=out.dtype, device=out.device)
     if panels8 and N and (col_major or ldb % 16 or b_t.data_ptr() % 16):
         # Copies for the LDS-DMA ring, where its offsets reach every operand.
-        ring = (short and dbsr.n_blocks << 10 < RING_LIMIT
-                and out.shape[0] * target.stride(0) * target.element_size() < RING_LIMIT
-                and -(-dbsr.K // 32) * 32 * tuning.aligned_pitch(N) < RING_LIMIT)
+        def ring() -> bool:
+            return (short and dbsr.n_blocks << 10 < RING_LIMIT
+                    and out.shape[0] * target.stride(0) * target.element_size() < RING_LIMIT
+                    and -(-dbsr.K // 32) * 32 * tuning.aligned_pitch(N) < RING_LIMIT)
+
+        longest = min(dbsr.max_row, chunk)
         if col_major:
-            bytewise = ring and bool(ldb % 16 or dbsr.K % 32 or b_t.data_ptr() % 16)
-            if tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K, bytewise, N, min(dbsr.max_row, chunk)):
+            bytewise = bool(ldb % 16 or dbsr.K % 32 or b_t.data_ptr() % 16) and ring()
+            if tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K, bytewise, N, longest):
                 b_t, col_major = row_major_copy_b8(b_t, ldb), False
                 ldb = max(b_t.stride(0), N)
-        if ring and not col_major and (ldb % 16 or b_t.data_ptr() % 16):
+        if not col_major and (ldb % 16 or b_t.data_ptr() % 16):
             dword = ((N | ldb | b_t.data_ptr() | target.stride(0)) % 4 == 0) and target.data_ptr() % 16 == 0
-            if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword, min(dbsr.max_row, chunk)):
+            if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword, longest) and ring():
                 b_t = aligned_copy_b8(b_t, ldb)
                 ldb = b_t.stride(0)
     stream = raw_stream(out.device)

@@ -220,6 +220,13 @@ def _observed(m: torch.nn.Module) -> bool:
                 or "forward" in m.__dict__ or torch.nn.modules.module._has_any_global_hook())
 
 
+# C from this size on takes the bias in the SpMM's epilogue; below, an addition
+# of its own, whose autograd nodes cost the host less (steps with the epilogue
+# and with the addition, us: bf16 4096 x 2048 321 and 306, 14336 x 1024 329 and 338,
+# 14336 x 2048 466 and 603; fp32 4096 x 1024 312 and 307, 4096 x 2048 434 and 450).
+BIAS_EPILOGUE_BYTES = 1 << 25
+
+
 class SparseLinear(torch.nn.Module):
     """nn.Linear with a VOID weight: y = x W^T + b (autograd.py:288-352)."""
 
@@ -242,7 +249,8 @@ class SparseLinear(torch.nn.Module):
         rounded before the bias).  Everything else, forward-mode tangents of the
         bias among it, takes the addition of its own."""
         w, bias = self.sparse_weight, self.bias
-        return (type(bias) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda
+        return (x.numel() // self.in_features * self.out_features * x.element_size() >= BIAS_EPILOGUE_BYTES
+                and type(bias) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda
                 and x.dtype in (torch.float32, torch.bfloat16, torch.float16)
                 and bias.dtype == x.dtype and bias.device == x.device and bias.shape == (self.out_features,)
                 and type(w) is VOIDSpMM and w.n_blocks > 0 and not _observed(w)
