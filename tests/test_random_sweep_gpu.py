@@ -120,3 +120,22 @@ def test_random_fp8_float_b(gpu, seed, monkeypatch):
     bound = oracle.fp8_spmm_float_b(Aabs, np.abs(bf))
     err = np.abs(out.cpu().numpy().astype(np.float64) - ref)
     assert np.all(err <= FP8_TOL * bound + 1e-30), (case.M, case.K, case.N)
+
+
+@pytest.mark.parametrize("M,K,N", [(3200, 16384, 3072), (3200, 16384, 2176), (2048, 16384, 4000), (512, 16384, 3072),
+                                   (512, 33000, 2100)])
+@pytest.mark.parametrize("split", [False, True])
+def test_panel_groups_past_the_l2(gpu, monkeypatch, M, K, N, split):
+    """16 and more panels whose columns exceed an XCD's L2, in grids of several
+    rounds (limited groups, some of a width that does not divide the panels, a
+    last panel cut off) and short ones (full groups): int32 bit-exact."""
+    monkeypatch.delenv("VOID_AMD_KERNEL", raising=False)
+    case = cases.uniform_blocks(M, K, 8, M // 32 * 5, seed=N)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu")).to(gpu)
+    b = torch.randint(-128, 128, (K, N), dtype=torch.int8, device=gpu)
+    got = void_amd.void_spmm_int8(q, b, epilogue="raw_i32", chunk_tiles=3 if split else None)
+    ref = torch.zeros(M, N, dtype=torch.float64, device=gpu)
+    for t, (r, c) in enumerate(zip(case.block_rows, case.block_cols)):
+        bt = b[32 * c:32 * c + 32].double()
+        ref[32 * r:32 * r + 32] += q.values[t][:, :bt.shape[0]].double() @ bt
+    assert torch.equal(got.double(), ref)

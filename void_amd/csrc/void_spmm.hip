@@ -2601,15 +2601,22 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   p.n_panels = n_panels;
   p.activation = d->activation;
   p.n_items = n_items;
-  // Panels per XCD share, as long as the B columns of a group fit the XCD's
-  // 4 MB L2: past it, each panel's columns come from the Infinity Cache again
-  // (4096 x 14336, 14336 bf16 tiles, N = 2048, 3.7 MB a panel: 180 us in groups of
-  // two, 135 us one by one; at 2 MB a panel both take the same time).
+  // Panels per XCD share: the panels over the 8 XCDs, in grids of several
+  // rounds only as many as fit the XCD's 4 MB L2 with their B columns. Past
+  // it, each panel's columns come from the Infinity Cache again (16384 x 16384,
+  // 24576 tiles, bf16, N = 2048: 302 us in groups of two, 218 one by one; int8,
+  // N = 4096: 346 -> 295). In shorter grids, where few workgroups share a
+  // panel, the balance that the full groups' dealt layout gives weighs more
+  // (1024 x 8192, Zipf rows, fp32, N = 4096: 65 us, 94 limited; 512 x 8192: 47 and
+  // 73; int8 1024 x 16384, N = 3072: 18.6 and 22.0), with a 4-byte B up to some 2500
+  // workgroups (2048 x 8192, Zipf rows, N = 4096: 126 and 156), with a smaller
+  // one up to 1900 (bf16 2048 x 8192, 1536 workgroups: 40 and 47; 2048: 56 and 48).
   {
     const int b_esz = (elt == kEltF32 || elt == kEltFp8F32) ? 4 : (elt == kEltI8 || elt == kEltFp8) ? 1 : 2;
     const int64_t panel_bytes = (int64_t)a->K * kPanel * b_esz;
     const int fit = (int)std::max<int64_t>(1, ((int64_t)4 << 20) / std::max<int64_t>(panel_bytes, 1));
-    p.panel_group = n_panels >= 16 ? std::min(n_panels / 8, fit) : 1;
+    p.panel_group = n_panels >= 16 ? n_panels / 8 : 1;
+    if (grid64 > (b_esz == 4 ? 2560 : 1920)) p.panel_group = std::min(p.panel_group, fit);
   }
   // With split rows (a long-tailed distribution) every XCD that shares a
   // panel group gets a dealt share of the longest-first list; otherwise the
