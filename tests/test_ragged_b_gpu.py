@@ -208,3 +208,19 @@ def test_column_major_any_alignment(gpu, K, N):
         if b.stride(0) == 1 and K > 1:
             copy = _runtime.row_major_copy_b8(b, b.stride(1))
             assert copy.stride(0) % 16 == 0 and torch.equal(copy, b)
+
+
+@pytest.mark.parametrize("M,N", [(512, 512), (4096, 2048)])
+def test_narrow_named_on_a_wide_call(gpu, monkeypatch, M, N):
+    """VOID_AMD_KERNEL=narrow on a call that is too wide for it: the default
+    kernel, bit for bit (per-block sums in fp32 differ between ring shapes)."""
+    case = cases.uniform_blocks(M, 1024, N, M // 32 * 16, seed=N)
+    q = void_amd.quantize_void_tensor(cases.make_void_tensor(case, "cpu")).to(gpu)
+    bq, bs = oracle.quantize_i8_columns(case.b)
+    out = {}
+    for kernel in (None, "narrow"):
+        if kernel:
+            monkeypatch.setenv("VOID_AMD_KERNEL", kernel)
+        out[kernel] = void_amd.void_spmm_int8(q, torch.from_numpy(bq).to(gpu), b_scale=torch.from_numpy(bs).to(gpu),
+                                              epilogue="per_block")
+    assert torch.equal(out[None], out["narrow"])

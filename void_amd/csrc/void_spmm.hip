@@ -2792,6 +2792,7 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   const int64_t b_span = d->b_col_major ? (int64_t)d->N * d->ldb
                                         : (int64_t)((a->K + kTile - 1) / kTile) * kTile * d->ldb;
   const char* force = getenv("VOID_AMD_KERNEL");
+  if (force && strcmp(force, "narrow") == 0) force = nullptr;  // the default where it applies
   const bool force_bsr = force && strcmp(force, "bsr") == 0;
   const bool force_cg = force && strcmp(force, "cg") == 0;
   const bool force_deep = force && strcmp(force, "cgd3") == 0;
@@ -2799,9 +2800,9 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   const bool offsets_ok = (int64_t)a->n_blocks * kTile * kTile < kLim && b_span < kLim &&
                           (int64_t)a->M * d->ldc * esz < kLim;
 
-  // Few columns: the narrow kernel, for every B layout (VOID_AMD_KERNEL=narrow
-  // names it, any other value keeps the panel kernels).
-  if (d->N <= (n_split_tiles > 0 ? kTile : kNarrowN) && plan->chunk_tiles <= kCgMaxTiles && offsets_ok && (!force || strcmp(force, "narrow") == 0)) {
+  // Few columns: the narrow kernel, for every B layout (forcing a panel kernel
+  // keeps that one).
+  if (d->N <= (n_split_tiles > 0 ? kTile : kNarrowN) && plan->chunk_tiles <= kCgMaxTiles && offsets_ok && !force) {
     if (d->out_dtype < VOID_DT_F32 || d->out_dtype > VOID_DT_I32)
       return fail(VOID_ERR_UNSUPPORTED, "out_dtype %d not supported with this epilogue", d->out_dtype);
     const int bmode = d->b_col_major ? (b16 ? kNbCol16 : kNbColAny) : (b16 ? kNbRow16 : kNbRowAny);
