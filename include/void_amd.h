@@ -301,7 +301,8 @@ int void_transpose_b8(const void* src, int64_t ld_src, int32_t rows, int32_t col
 
 /* dst[c * ld_dst + r] = src[r * ld_src + c] for a rows x cols matrix of 1-, 2-
  * or 4-byte elements (elem_bytes), any sizes, leading dimensions in elements:
- * a column-major B or gradient (token-major activations) made row-major.  rows at most 64 * 65535.  No counterpart in the reference. */
+ * a column-major B or gradient (token-major activations) made row-major.
+ * rows at most 64 * 65535.  No counterpart in the reference. */
 int void_transpose(const void* src, int64_t ld_src, int32_t rows, int32_t cols, void* dst, int64_t ld_dst,
                    int32_t elem_bytes, hipStream_t stream);
 

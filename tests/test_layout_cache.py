@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import void_amd
-from void_amd import _runtime, autograd
+from void_amd import _runtime, _streams, autograd
 
 
 def test_record_once(monkeypatch):
@@ -24,13 +24,13 @@ def test_record_once(monkeypatch):
         def record_stream(self, s):
             log.append((self.name, s))
 
-    monkeypatch.setattr(_runtime, "raw_stream", lambda d: now[0])
+    monkeypatch.setattr(_streams, "raw_stream", lambda d: now[0])
     monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: now[0])
     seen = set()
     arrays = Array("a"), Array("b")
     for s in (7, 9, 7, 9):
         now[0] = s
-        _runtime.record_once(seen, torch.device("cpu"), *arrays)
+        _streams.record_once(seen, torch.device("cpu"), *arrays)
     assert log == [("a", 7), ("b", 7), ("a", 9), ("b", 9)]
 
 

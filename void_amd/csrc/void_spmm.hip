@@ -2687,12 +2687,15 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
   const int grid = p.xcd_exact ? (int)grid_exact : (int)grid64;
 
   if (elt == kEltFp8F32) {
-    // E4M3 tiles times fp32 B: the LDS-DMA ring only (16-byte aligned rows,
-    // N % 4 == 0, 31-bit byte offsets); the Python wrapper pads other shapes.
+    // E4M3 tiles times fp32 B: the LDS-DMA ring only (b 16-byte aligned with ldb
+    // a multiple of 16 bytes, 31-bit byte offsets; without VOID_DENSE_PADDED_B
+    // also N % 4 == 0 and 16-byte aligned C rows).  The Python wrapper copies
+    // other operands to such rows.
     const int64_t lim = (int64_t)1 << 31;
     const int esz = (d->out_dtype == VOID_DT_BF16 || d->out_dtype == VOID_DT_F16) ? 2 : 4;
     if (!((c_ok || padded) && (bu % 16 == 0) && (d->ldb % 4 == 0)))
-      return fail(VOID_ERR_UNSUPPORTED, "E4M3 x fp32 SpMM needs 16-byte aligned B and C rows and N %% 4 == 0");
+      return fail(VOID_ERR_UNSUPPORTED, "E4M3 x fp32 SpMM needs 16-byte aligned B rows, and 16-byte aligned C rows and "
+                                       "N %% 4 == 0 without VOID_DENSE_PADDED_B");
     if (!((int64_t)a->n_blocks * kTile * kTile < lim && (int64_t)((a->K + kTile - 1) / kTile) * kTile * d->ldb * 4 < lim &&
           (int64_t)a->M * d->ldc * esz < lim))
       return fail(VOID_ERR_UNSUPPORTED, "E4M3 x fp32 SpMM operands must stay below 2 GiB");
@@ -2711,15 +2714,17 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     }
   }
   if (elt == kEltBf16 || elt == kEltF16 || elt == kEltFp8Bf16 || elt == kEltFp8F16) {
-    // A 16-bit B (with 16-bit or E4M3 tiles): the LDS-DMA ring only
-    // (row-major B and C with 16-byte aligned rows, N % 8 == 0, items of at
-    // most 64 tiles, 31-bit byte offsets).  The Python wrappers take the
-    // fp32 B kernels otherwise.
+    // A 16-bit B (with 16-bit or E4M3 tiles): the LDS-DMA ring only (row-major
+    // b, 16-byte aligned with ldb a multiple of 16 bytes, items of at most 64
+    // tiles, 31-bit byte offsets; without VOID_DENSE_PADDED_B also N % 8 == 0
+    // and 16-byte aligned C rows).  The Python wrappers copy other operands to
+    // such rows or take the fp32 B kernels.
     const int64_t lim = (int64_t)1 << 31;
     const int64_t a_tile_bytes = (elt == kEltBf16 || elt == kEltF16) ? 2048 : 1024;
     const int esz = (d->out_dtype == VOID_DT_BF16 || d->out_dtype == VOID_DT_F16) ? 2 : 4;
     if (d->b_col_major || !((bu % 16 == 0) && (d->ldb % 8 == 0) && (padded || (c_ok && d->N % 8 == 0))))
-      return fail(VOID_ERR_UNSUPPORTED, "16-bit SpMM needs a row-major B, 16-byte aligned B and C rows and N %% 8 == 0");
+      return fail(VOID_ERR_UNSUPPORTED, "16-bit SpMM needs a row-major B with 16-byte aligned rows, and 16-byte aligned C "
+                                       "rows and N %% 8 == 0 without VOID_DENSE_PADDED_B");
     if (plan->chunk_tiles > kCgMaxTiles)
       return fail(VOID_ERR_ARG, "16-bit SpMM takes work items of at most %d tiles (chunk_tiles %d)", kCgMaxTiles,
                   plan->chunk_tiles);
@@ -2755,7 +2760,8 @@ int run(int elt, const void_bsr_desc* a, const void_dense_args* d, int32_t epilo
     // keeps the fp32 kernel of its own (the fallback for everything else).
     const char* fk = getenv("VOID_AMD_KERNEL");
     const int64_t lim = (int64_t)1 << 31;
-    const bool ring_ok = (vec || (padded && (bu % 16 == 0) && (d->ldb % 4 == 0))) && !d->b_col_major && plan->chunk_tiles <= kCgMaxTiles &&
+    const bool ring_ok = (vec || (padded && (bu % 16 == 0) && (d->ldb % 4 == 0))) && !d->b_col_major &&
+                         plan->chunk_tiles <= kCgMaxTiles &&
                          (int64_t)a->n_blocks * kTile * kTile * 4 < lim &&
                          (int64_t)((a->K + kTile - 1) / kTile) * kTile * d->ldb * 4 < lim &&
                          (int64_t)a->M * d->ldc * 4 < lim && !(fk && strcmp(fk, "f32") == 0);

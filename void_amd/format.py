@@ -18,6 +18,8 @@ import numpy as np
 import torch
 from scipy import sparse
 
+from ._streams import record_once
+
 # format.py:12 — tile sizes below 16 were rejected by the reference's tensor-core path.
 MIN_TENSOR_CORE_TILE = 16
 
@@ -76,8 +78,7 @@ class BsrLayout:
     def on_stream(self) -> None:
         """The arrays are about to be used on the current stream: where a cache
         drops this layout, their memory is not handed out before that work is done."""
-        from . import _runtime
-        _runtime.record_once(self.streams, self.row_ptr.device, self.order, self.row_ptr, self.col_idx)
+        record_once(self.streams, self.row_ptr.device, self.order, self.row_ptr, self.col_idx)
 
     @property
     def max_row(self) -> int:
@@ -100,8 +101,7 @@ class BsrLayout:
             arr = np.stack([rows, start, cnt], axis=1).astype(np.int32).reshape(-1, 3)
             self.sddmm_groups = torch.from_numpy(arr).to(self.row_ptr.device)
         if self.row_ptr.is_cuda:
-            from . import _runtime
-            _runtime.record_once(self.group_streams, self.row_ptr.device, self.sddmm_groups)
+            record_once(self.group_streams, self.row_ptr.device, self.sddmm_groups)
         return self.sddmm_groups
 
 
