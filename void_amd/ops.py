@@ -70,7 +70,10 @@ def float_spmm(a, b: torch.Tensor, *, out: Optional[torch.Tensor] = None, bias: 
         entry = _K16[b.dtype]
         dbsr = a.device_bsr(b.dtype)
     else:
-        wide = b.to(torch.float32)
+        # A 16-bit column-major B is transposed before it is widened (half the bytes).
+        wide = b
+        if b.dtype is not torch.float32:
+            wide = (b if b.stride(1) == 1 else _runtime.contiguous_2d(b)).to(torch.float32)
         bk = _runtime.ring_rows(wide, a.n_blocks, a) if _rings_reach(a, target, 4096) else None
         if bk is None:
             bk = _runtime.contiguous_2d(wide)
