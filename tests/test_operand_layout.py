@@ -61,9 +61,12 @@ def test_copy_rules_weigh_the_pass_over_b(n, max_row, K, N, row8, col8, f32):
 
 def test_copy_rules_forced(monkeypatch):
     monkeypatch.setenv("VOID_AMD_PAD", "1")
-    assert tuning.copy_unaligned_b(1, 1 << 20, 101, False, 1) and _runtime._pad_forced(1, 1)
+    assert tuning.copy_unaligned_b(1, 1 << 20, 101, False, 1)
     monkeypatch.setenv("VOID_AMD_PAD", "0")
-    assert not tuning.copy_unaligned_b(14336, 4096, 2004, True, 64) and _runtime._pad_forced(14336, 2004) is False
+    assert not tuning.copy_unaligned_b(14336, 4096, 2004, True, 64)
+    for forced in (True, False):
+        monkeypatch.setattr(tuning, "PAD_FLOAT", forced)
+        assert _runtime._pad_forced(1, 1) is forced and _runtime._pad_forced(14336, 2004) is forced
 
 
 def test_sddmm_copies_weigh_the_passes():

@@ -9,7 +9,7 @@ import torch
 import cases
 import oracle
 import void_amd
-from void_amd import _runtime
+from void_amd import _runtime, tuning
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
@@ -20,7 +20,7 @@ ABS = {torch.float32: 0.0, torch.bfloat16: 0.0, torch.float16: 2.0 ** -25}
 @pytest.fixture(autouse=True)
 def always_pad(monkeypatch):
     monkeypatch.setattr(_runtime, "PAD_FLOAT_MIN_WORK", 1)
-    monkeypatch.setenv("VOID_AMD_PAD", "1")
+    monkeypatch.setattr(tuning, "PAD_FLOAT", True)
 
 
 def _views(b):

@@ -527,35 +527,27 @@ def padded_layout(R: int, C: int, s0: int, s1: int, ptr: int, esz: int, zero_tai
     pitch of a copy is whole 128-byte lines (16-byte chunks up to one line, or
     where only those stay below the limit)."""
     per = 16 // esz
-    fits = lambda ld: limit is None or -(-R // 32) * 32 * ld * esz < limit
-    if (s1 == 1 and s0 >= C and s0 % per == 0 and ptr % 16 == 0 and not (zero_tail and C % per) and fits(s0)):
+    rows = (R + 31) // 32 * 32 * esz
+    if (s1 == 1 and s0 >= C and s0 % per == 0 and ptr % 16 == 0 and not (zero_tail and C % per)
+            and (limit is None or rows * s0 < limit)):
         return True, s0
-    chunks = -(-C // per) * per
-    lines = -(-C // (8 * per)) * 8 * per if C > 8 * per else chunks
-    for pitch in (lines, chunks):
-        if fits(pitch):
-            return False, pitch
-    return None
+    chunks = (C + per - 1) // per * per
+    pitch = (C + 8 * per - 1) // (8 * per) * 8 * per if C > 8 * per else chunks
+    if limit is not None and rows * pitch >= limit:
+        pitch = chunks
+        if rows * pitch >= limit:
+            return None
+    return False, pitch
 
 
-def padded_rows(t: torch.Tensor, zero_tail: bool = False, limit: Optional[int] = None) -> torch.Tensor:
-    """A 2-D 16- or 32-bit GPU tensor as aligned_rows: t itself where it is,
-    else a copy whose rows are zero from their end to the next multiple of 16
-    bytes, as padded_layout says (which finds a layout under ``limit``, or the
-    caller has asked it before).  With zero_tail, t itself only if its rows end
-    on a multiple of 16 bytes."""
+def padded_copy(t: torch.Tensor, pitch: int) -> torch.Tensor:
+    """Row-major copy of a 2-D 16- or 32-bit GPU tensor with aligned rows (of a
+    pitch that padded_layout gave), zero from their end to the next multiple of
+    16 bytes."""
     R, C = t.shape
-    if not t.numel():
-        return t
     esz = t.element_size()
     per = 16 // esz
     s0, s1 = t.stride()
-    lay = padded_layout(R, C, s0, s1, t.data_ptr(), esz, zero_tail, limit)
-    if lay is None:
-        raise ValueError(f"{R} padded rows of {C} {t.dtype} values reach {limit} bytes")
-    in_place, pitch = lay
-    if in_place:
-        return t
     if s1 == 1 and s0 >= C and R * -(-C // per) < 1 << 31:
         out = torch.empty(R, pitch, dtype=t.dtype, device=t.device)[:, :C]
         st = _lib.lib().void_copy_rows_b8(t.data_ptr(), s0 * esz, R, C * esz, out.data_ptr(), pitch * esz,
@@ -574,15 +566,28 @@ def padded_rows(t: torch.Tensor, zero_tail: bool = False, limit: Optional[int] =
     return out
 
 
+def padded_rows(t: torch.Tensor, zero_tail: bool = False, limit: Optional[int] = None) -> torch.Tensor:
+    """A 2-D 16- or 32-bit GPU tensor as aligned_rows: t itself where it is,
+    else a padded_copy, as padded_layout says (which finds a layout under
+    ``limit``, or the caller has asked it before).  With zero_tail, t itself
+    only if its rows end on a multiple of 16 bytes."""
+    if not t.numel():
+        return t
+    R, C = t.shape
+    lay = padded_layout(R, C, *t.stride(), t.data_ptr(), t.element_size(), zero_tail, limit)
+    if lay is None:
+        raise ValueError(f"{R} padded rows of {C} {t.dtype} values reach {limit} bytes")
+    return t if lay[0] else padded_copy(t, lay[1])
+
+
 PAD_FLOAT_MIN_WORK = tuning.PAD_FLOAT_MIN_WORK
 
 
 def _pad_forced(n_blocks: int, N: int) -> Optional[bool]:
-    """What VOID_AMD_PAD or a small call decides about padded rows, else None."""
-    forced = tuning._forced("VOID_AMD_PAD")
-    if forced is None and n_blocks * N < PAD_FLOAT_MIN_WORK:
+    """What tuning.PAD_FLOAT or a small call decides about padded rows, else None."""
+    if tuning.PAD_FLOAT is None and n_blocks * N < PAD_FLOAT_MIN_WORK:
         return False
-    return forced
+    return tuning.PAD_FLOAT
 
 
 def ring_rows(t: torch.Tensor, n_blocks: int, a=None, zero_tail: bool = False) -> Optional[torch.Tensor]:
@@ -606,7 +611,7 @@ def ring_rows(t: torch.Tensor, n_blocks: int, a=None, zero_tail: bool = False) -
     pad = _pad_forced(n_blocks, N)
     if pad is None:
         pad = a is None or tuning.pad_float_b(n_blocks, a.longest_row(), K, N, pitch, esz, t.is_contiguous())
-    return padded_rows(t, zero_tail, RING_LIMIT) if pad else None
+    return padded_copy(t, pitch) if pad else None
 
 
 def row_major(t: torch.Tensor, n_blocks: int, a=None) -> torch.Tensor:
@@ -645,20 +650,17 @@ def launch(kind: str, dbsr: DeviceBsr, b: torch.Tensor, *, b_scale: float = 1.0,
         target = torch.empty(out.shape, dtype=out.dtype, device=out.device)
     if panels8 and N and (col_major or ldb % 16 or b_t.data_ptr() % 16):
         # Copies for the LDS-DMA ring, where its offsets reach every operand.
-        def ring() -> bool:
-            return (short and dbsr.n_blocks << 10 < RING_LIMIT
-                    and out.shape[0] * target.stride(0) * target.element_size() < RING_LIMIT
-                    and -(-dbsr.K // 32) * 32 * tuning.aligned_pitch(N) < RING_LIMIT)
-
-        longest = min(dbsr.max_row, chunk)
+        n, K = dbsr.n_blocks, dbsr.K
+        ring = (short and n << 10 < RING_LIMIT and (K + 31) * tuning.aligned_pitch(N) < RING_LIMIT
+                and dbsr.M * target.stride(0) * target.element_size() < RING_LIMIT)
         if col_major:
-            bytewise = bool(ldb % 16 or dbsr.K % 32 or b_t.data_ptr() % 16) and ring()
-            if tuning.copy_col_major_b(dbsr.n_blocks, dbsr.K, bytewise, N, longest):
+            bytewise = ring and bool(ldb % 16 or K % 32 or b_t.data_ptr() % 16)
+            if tuning.copy_col_major_b(n, K, bytewise, N, dbsr.max_row):
                 b_t, col_major = row_major_copy_b8(b_t, ldb), False
                 ldb = max(b_t.stride(0), N)
-        if not col_major and (ldb % 16 or b_t.data_ptr() % 16):
+        if ring and not col_major and (ldb % 16 or b_t.data_ptr() % 16):
             dword = ((N | ldb | b_t.data_ptr() | target.stride(0)) % 4 == 0) and target.data_ptr() % 16 == 0
-            if tuning.copy_unaligned_b(dbsr.n_blocks, dbsr.K, N, dword, longest) and ring():
+            if tuning.copy_unaligned_b(n, K, N, dword, dbsr.max_row):
                 b_t = aligned_copy_b8(b_t, ldb)
                 ldb = b_t.stride(0)
     stream = raw_stream(out.device)

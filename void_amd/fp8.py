@@ -286,9 +286,10 @@ def void_spmm_fp8(a: FP8VOIDTensor, b: torch.Tensor, output_dtype: torch.dtype =
         # to its type), in rows that are (or are copied to be) 16-byte aligned
         # (512 x 37 bf16, 60 tiles: 18.5 us with the copy, 24.2 widened to fp32),
         # where the ring's offsets reach every operand.
-        if (a.n_blocks * 1024 < _runtime.RING_LIMIT and M * N * out.element_size() < _runtime.RING_LIMIT
-                and _runtime.padded_layout(K, N, *b.stride(), b.data_ptr(), 2, limit=_runtime.RING_LIMIT)):
-            b16 = _runtime.padded_rows(b, limit=_runtime.RING_LIMIT)
+        lay = _runtime.padded_layout(K, N, *b.stride(), b.data_ptr(), 2, limit=_runtime.RING_LIMIT)
+        if (lay is not None and a.n_blocks * 1024 < _runtime.RING_LIMIT
+                and M * N * out.element_size() < _runtime.RING_LIMIT):
+            b16 = b if lay[0] or not N else _runtime.padded_copy(b, lay[1])
             kind = "fp8_bf16b" if b.dtype == torch.bfloat16 else "fp8_f16b"
             direct = out.stride(1) == 1 and M * out.stride(0) * out.element_size() < (1 << 31)
             tgt = out if direct else torch.empty(M, N, dtype=output_dtype, device=b.device)

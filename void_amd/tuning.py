@@ -95,8 +95,8 @@ def aligned_pitch(N: int) -> int:
 # the tiles: the chain of the longest block-row and the values gathered
 # (tiles x 32 x N).  Both sides below in us, fitted to eager calls with 50, 400
 # and 3200 tiles (about 3 to 20 a row), N = 101 and 730, K from 4099 to
-# 1048579.  VOID_AMD_BT=0 / 1 forces the column-major copy off / on,
-# VOID_AMD_PAD=0 / 1 the others.
+# 1048579.  VOID_AMD_BT=0 / 1 forces the copy of a column-major 8-bit B off / on,
+# VOID_AMD_PAD=0 / 1 that of a row-major one.
 
 
 def _forced(name: str):
@@ -130,7 +130,7 @@ def copy_col_major_b(n_blocks: int, K: int, bytewise: bool = False, N: int = 0, 
         return forced
     if 32 * n_blocks >= COL_MAJOR_COPY_RATIO * max(K, 1):
         return True
-    saved = 8 + 1.5 * max_row + 1.9e-6 * 32 * n_blocks * N
+    saved = 8 + 1.5 * min(max_row, 64) + 1.9e-6 * 32 * n_blocks * N  # (an item's chain: 64 tiles at most)
     return bytewise and saved > _pass_us(K, N, aligned_pitch(N), 2.6e6)
 
 
@@ -151,7 +151,7 @@ def copy_unaligned_b(n_blocks: int, K: int, N: int, dword: bool, max_row: int = 
         return forced
     if dword:
         return N > PANEL_COLUMNS and 32 * n_blocks >= COL_MAJOR_COPY_RATIO * max(K, 1)
-    saved = 10 + 1.1 * max_row + 1.2e-6 * 32 * n_blocks * N
+    saved = 10 + 1.1 * min(max_row, 64) + 1.2e-6 * 32 * n_blocks * N
     return saved > _pass_us(K, N, aligned_pitch(N), 4.2e6)
 
 
@@ -160,6 +160,7 @@ def copy_unaligned_b(n_blocks: int, K: int, N: int, dword: bool, max_row: int = 
 # read an fp32 B in place and a 16-bit one widened (a pass of its own).  Below
 # this many tiles times columns the element-wise kernels take no longer.
 PAD_FLOAT_MIN_WORK = 1 << 14
+PAD_FLOAT = None  # True / False forces these copies on / off (comparisons and tests)
 
 
 def pad_float_b(n_blocks: int, max_row: int, K: int, N: int, pitch: int, esz: int, in_place: bool) -> bool:
@@ -172,8 +173,8 @@ def pad_float_b(n_blocks: int, max_row: int, K: int, N: int, pitch: int, esz: in
     gathered = 32e-6 * n_blocks * N
     if esz == 2:
         widened = _pass_us(K, 2 * N, 4 * N, 5.2e6)
-        return 1.0 * max_row - 8 + 1.1 * gathered + widened > _pass_us(K, 2 * N, 2 * pitch, 4.2e6)
-    saved = 1.0 * max_row - 4.5 + 0.5 * gathered
+        return 1.0 * min(max_row, 64) - 8 + 1.1 * gathered + widened > _pass_us(K, 2 * N, 2 * pitch, 4.2e6)
+    saved = 1.0 * min(max_row, 64) - 4.5 + 0.5 * gathered
     return saved > (6.5 + _pass_us(K, 4 * N, 4 * pitch, 4.4e6) if in_place else 0)
 
 
