@@ -285,7 +285,7 @@ def test_linear_bias_fused_step(gpu, monkeypatch, dtype, tokens, token_major_gra
     forward hook on the weight module takes the unfused path to the same bits
     (the bias's gradient, summed in another order, within its bound)."""
     monkeypatch.setattr(_runtime, "TRANSPOSE_MIN_NUMEL", 1)
-    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", {2: 0, 4: 0})
     case = cases.uniform_blocks(130, 200, tokens, 20, seed=tokens)
     vt = cases.make_void_tensor(case, "cpu").to(gpu).to_dtype(dtype)
     lin = void_amd.SparseLinear(200, 130, vt).to(gpu)
@@ -347,7 +347,7 @@ def _linear(gpu, dtype, tokens, seed=3):
 @pytest.mark.parametrize("tokens", [1, 37, 64])
 def test_linear_bias_is_an_addition(gpu, monkeypatch, dtype, tokens, kernel):
     """y = w(x) + b to the bit: the product is rounded to x's type, then the sum."""
-    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", {2: 0, 4: 0})
     if kernel:
         monkeypatch.setenv("VOID_AMD_KERNEL", kernel)
     lin, x = _linear(gpu, dtype, tokens)
@@ -360,7 +360,7 @@ def test_linear_bias_keeps_autograd(gpu, monkeypatch):
     """The bias alone: batched gradients, no SpMM in its backward, forward-mode
     tangents; and a frozen bias or weight."""
     import torch.autograd.forward_ad as fwd
-    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", {2: 0, 4: 0})
     lin, x = _linear(gpu, torch.float32, 12)
     gy = torch.randn(4, 12, 130, device=gpu)
     y = lin(x)
@@ -394,7 +394,7 @@ def test_linear_bias_keeps_autograd(gpu, monkeypatch):
 
 def test_linear_create_graph_bias(gpu, monkeypatch):
     """With create_graph the bias gradient stays differentiable in the output gradient."""
-    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", 0)
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", {2: 0, 4: 0})
     case = cases.uniform_blocks(64, 64, 5, 3, seed=2)
     lin = void_amd.SparseLinear(64, 64, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu)
     x = torch.randn(5, 64, device=gpu)
@@ -453,7 +453,7 @@ def test_layout_cache_eviction(gpu):
 def test_linear_output_in_place_and_shapes(gpu, monkeypatch, least):
     """The output takes in-place operations and 3-D and empty inputs as before,
     with the bias in the epilogue and as an addition."""
-    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", least)
+    monkeypatch.setattr(autograd, "BIAS_EPILOGUE_BYTES", {4: least})
     case = cases.uniform_blocks(64, 96, 40, 4, seed=9)
     lin = void_amd.SparseLinear(96, 64, cases.make_void_tensor(case, "cpu").to(gpu)).to(gpu)
     x = torch.randn(2, 5, 96, device=gpu, requires_grad=True)

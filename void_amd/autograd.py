@@ -220,11 +220,13 @@ def _observed(m: torch.nn.Module) -> bool:
                 or "forward" in m.__dict__ or torch.nn.modules.module._has_any_global_hook())
 
 
-# C from this size on takes the bias in the SpMM's epilogue; below, an addition
-# of its own, whose autograd nodes cost the host less (steps with the epilogue
-# and with the addition, us: bf16 4096 x 2048 321 and 306, 14336 x 1024 329 and 338,
-# 14336 x 2048 466 and 603; fp32 4096 x 1024 312 and 307, 4096 x 2048 434 and 450).
-BIAS_EPILOGUE_BYTES = 1 << 25
+# C of this many bytes (by element size) takes the bias in the SpMM's epilogue.
+# Below, an addition of its own, whose autograd nodes cost the host less (a
+# 16-bit bias is also widened for the epilogue).  Steps with the epilogue and
+# with the addition, us: fp32 4096 x 1024 236 and 276 (307 and 303 where the
+# host, in its slower mode, bounds both), 2048 x 2048 206 and 220; bf16
+# 4096 x 2048 199 and 189, 8192 x 2048 246 and 260, 14336 x 2048 466 and 603.
+BIAS_EPILOGUE_BYTES = {4: 1 << 24, 2: 1 << 25}
 
 
 class SparseLinear(torch.nn.Module):
@@ -249,9 +251,10 @@ class SparseLinear(torch.nn.Module):
         rounded before the bias).  Everything else, forward-mode tangents of the
         bias among it, takes the addition of its own."""
         w, bias = self.sparse_weight, self.bias
-        return (x.numel() // self.in_features * self.out_features * x.element_size() >= BIAS_EPILOGUE_BYTES
+        esz = x.element_size()
+        return (x.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                and x.numel() // self.in_features * self.out_features * esz >= BIAS_EPILOGUE_BYTES[esz]
                 and type(bias) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda
-                and x.dtype in (torch.float32, torch.bfloat16, torch.float16)
                 and bias.dtype == x.dtype and bias.device == x.device and bias.shape == (self.out_features,)
                 and type(w) is VOIDSpMM and w.n_blocks > 0 and not _observed(w)
                 and forward_ad.unpack_dual(bias).tangent is None)
