@@ -190,4 +190,4 @@ def pad_float_sddmm(n_blocks: int, N: int, esz: int, operands) -> bool:
             saved += _pass_us(rows, 2 * N, 4 * N, 5.2e6) - _pass_us(rows, 2 * N, 2 * pitch, 4.2e6)
         elif in_place:
             saved -= 6.5 + _pass_us(rows, 4 * N, 4 * pitch, 4.4e6)
-    return saved + (0.02 * N - 7 if esz == 2 else -1) > 0
+    return saved + (0.02 * N - 3.5 * len(operands) if esz == 2 else -1) > 0
