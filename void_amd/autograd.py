@@ -27,6 +27,7 @@ from . import _runtime
 from .format import VOIDTensor, build_bsr_layout
 from .ops import float_spmm
 
+
 class _Structure:
     """The block-row order of a tile set (forward, SDDMM) and of its transpose
     (gradient of B), with the plans that live in them."""

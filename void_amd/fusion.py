@@ -15,7 +15,6 @@ from typing import Optional, Union
 
 import torch
 
-from . import _runtime
 from .format import VOIDTensor
 from .ops import float_spmm
 
